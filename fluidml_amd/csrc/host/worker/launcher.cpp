@@ -170,6 +170,14 @@ void LaunchPlan::Materialize() {
     for (auto &kv : *slots) Check(fluidml_hip_arena_create(kv.second.bytes, &kv.second.device), "allocating a device buffer");
   }
   for (Step &s : steps_) s.kernel->Prepare();
+  std::vector<Transfer::Slot> in, out;
+  for (const Argument &a : arguments_) {
+    Transfer::Slot slot;
+    slot.device = interfaces_.at(a.name).device;
+    slot.bytes = a.meta.GetSize();
+    (a.type == Argument::Type::Input ? in : out).push_back(slot);
+  }
+  transfer_ = std::make_unique<Transfer>(std::move(in), std::move(out));
   Check(fluidml_hip_arena_create(arena_bytes_, &arena_), "allocating the arena");
   TuneContractions();
 }
@@ -928,33 +936,31 @@ size_t LaunchPlan::Run(const std::unordered_map<std::string, void *> &args, size
   // the literal LayerNorm mode reads its scratch before writing it: give every
   // call the zero-filled arena the reference allocates per Invoke (runner.cpp:87-88)
   if (flags_ & FL_REF_LN_STALE_SCRATCH) Check(fluidml_hip_arena_zero(arena_, arena_bytes_, stream_), "zeroing the arena");
+  std::vector<const void *> in;
+  std::vector<void *> out;
   for (const Argument &a : arguments_) {
     void *host = args.at(a.name);
     if (a.type == Argument::Type::Input) {
-      Check(fluidml_hip_memcpy_h2d(interfaces_.at(a.name).device, host, a.meta.GetSize(), stream_), "copying an input to HBM");
+      in.push_back(host);
+    } else {
+      out.push_back(host);
     }
   }
-  Check(fluidml_hip_stream_synchronize(stream_), "waiting for input copies");
-  DecideBranches();
   kernel::LaunchContext ctx;
   ctx.stream = stream_;
   ctx.flags = flags_;
   ctx.bf16 = bf16_;
-  if (use_graph_ && graph_ == nullptr) {  // record outside the timed region
-    Replay(ctx);
+  if (!branches_decided_ || (use_graph_ && graph_ == nullptr)) {  // decide and record outside the timed region
+    transfer_->In(in, stream_);
+    DecideBranches();
+    if (use_graph_ && graph_ == nullptr) Replay(ctx);
     Check(fluidml_hip_stream_synchronize(stream_), "waiting for the first replay");
   }
-  const auto t0 = std::chrono::high_resolution_clock::now();
+  // Nothing waits in between: the replays queue up behind the copies of the inputs, the copies of the outputs behind
+  // the replays, and the device's own clock tells how long the replays took.
+  transfer_->In(in, stream_);
   for (size_t e = 0; e < epoch; ++e) Replay(ctx);
-  Check(fluidml_hip_stream_synchronize(stream_), "waiting for the replays");
-  const auto t1 = std::chrono::high_resolution_clock::now();
-  for (const Argument &a : arguments_) {
-    if (a.type == Argument::Type::Output) {
-      Check(fluidml_hip_memcpy_d2h(args.at(a.name), interfaces_.at(a.name).device, a.meta.GetSize(), stream_), "copying an output to the host");
-    }
-  }
-  Check(fluidml_hip_stream_synchronize(stream_), "waiting for output copies");
-  return static_cast<size_t>(std::chrono::duration_cast<std::chrono::nanoseconds>(t1 - t0).count()) / epoch;
+  return static_cast<size_t>(transfer_->Out(out, stream_)) / epoch;
 }
 
 // Which kernels gain from running beside each other is not something the estimate above can tell (GPT-NeoX: its MLP

@@ -16,6 +16,7 @@
 #include "structure/flow/flow.h"
 #include "structure/kernel/kernel.h"
 #include "structure/kernel/tuner.h"
+#include "worker/transfer.h"
 
 namespace fluidml {
 namespace worker {
@@ -215,9 +216,10 @@ class LaunchPlan {
   // Materialize(), then everything the first run would decide by timing (the side branches), so that the plan
   // replays the same schedule from its first Invoke on and the decisions can be written down at Compile.
   void Settle();
-  // H2D inputs, `epoch` replays of all steps, D2H outputs; returns mean wall
-  // nanoseconds per replay of the launch-and-wait loop alone (reference
-  // runner.cpp:101-119). `args` maps every argument name to a host buffer of
+  // H2D inputs, `epoch` replays of all steps, D2H outputs; returns the mean
+  // nanoseconds of a replay, without the copies (reference runner.cpp:101-119;
+  // here on the device's clock, from the end of the last input copy to the
+  // start of the output copy). `args` maps every argument name to a host buffer of
   // exactly Meta::GetSize() bytes; a missing name throws std::out_of_range
   // (reference runner.cpp:70).
   size_t Run(const std::unordered_map<std::string, void *> &args, size_t epoch);
@@ -325,6 +327,7 @@ class LaunchPlan {
   void *arena_ = nullptr;
   void *stream_ = nullptr;
   void *graph_ = nullptr;
+  std::unique_ptr<Transfer> transfer_;
 };
 
 }  // namespace worker
