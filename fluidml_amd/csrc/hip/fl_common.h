@@ -110,6 +110,65 @@ __host__ __device__ __forceinline__ void StaticFor(F &&body) {
   StaticForImpl<N>(static_cast<F &&>(body), std::make_integer_sequence<int, N>{});
 }
 
+// ---- fp32 products on the bf16 matrix instructions ----------------------------------------------------------------
+// An fp32 value is the sum of three bf16 values, a = h + m + l: h = a rounded to bf16 (nearest even), m the remainder
+// rounded, l what is left.  Each step is exact: the remainder a - h has at most 16 significant bits, l at most 8.  (So
+// far as the parts stay normal numbers: below 2^-110 a value loses at most 2^-126.)  Of the nine products of two such
+// sums the kernels add six: l h', h l', m m', m h', h m' in one accumulator and h h' in another; the three left out are
+// together below 2^-24 of the product, which is the rounding of ONE fp32 product.  All sums are fp32, and the large ones
+// round once per sixteen values of k instead of once per value.  Against float64 (sums of 64 .. 25088 normal, positive
+// and worst-case mantissas) the result is closer than that of v_mfma_f32_32x32x2_f32: relative error 4.9e-8 against
+// 1.44e-7 for 64 normal products, 4.2e-7 against 1.20e-6 for 4608, positive ones 3.8e-7 against 1.05e-6; operands spread
+// over twenty powers of ten the same to within the run of the draw.  The six
+// v_mfma_f32_32x32x16_bf16 take 192 cycles per 16 values of k, the eight fp32 instructions 512; measured with operands
+// in registers on the whole chip 287 against 130-136 TFLOP/s.
+// What the parts cannot carry (an infinity minus itself is no number; a result so small that parts of its operands
+// may have been denormal) shows in the sum: BadSum tells, and the kernels then multiply that wave's tile again with
+// the fp32 instruction.
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// PARTS = 3: the three parts of eight values; PARTS = 1: the values rounded to bf16 (the opt-in precision)
+template <int PARTS>
+__device__ __forceinline__ void SplitParts(const float (&x)[8], u32x4 (&parts)[PARTS]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float a = x[2 * i], b = x[2 * i + 1];
+#pragma unroll
+    for (int q = 0; q < PARTS; ++q) {
+      const uint32_t packed = __builtin_bit_cast(uint32_t, bf16x2{static_cast<__bf16>(a), static_cast<__bf16>(b)});
+      parts[q][i] = packed;
+      a -= __builtin_bit_cast(float, packed << 16);
+      b -= __builtin_bit_cast(float, packed & 0xffff0000u);
+    }
+  }
+}
+
+// acc + low += A(32 x 16) B(16 x 32), every operand as its PARTS parts: the products of the leading parts go to acc, all
+// others (a 256th of them at most) to low, so that acc sees one rounding per sixteen values of k
+template <int PARTS>
+__device__ __forceinline__ void MfmaParts(const u32x4 (&a)[PARTS], const u32x4 (&b)[PARTS], floatx16 &acc, floatx16 &low) {
+  auto mul = [&](int i, int j, floatx16 &to) {
+    to = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[i]), __builtin_bit_cast(bf16x8, b[j]), to, 0, 0, 0);
+  };
+  if constexpr (PARTS == 3) {
+    mul(2, 0, low);
+    mul(0, 2, low);
+    mul(1, 1, low);
+    mul(1, 0, low);
+    mul(0, 1, low);
+  }
+  mul(0, 0, acc);
+}
+
+// a sum that is not finite, or neither zero nor at least 2^-80
+__device__ __forceinline__ bool BadSum(float v) {
+  const uint32_t bits = __builtin_bit_cast(uint32_t, v) & 0x7fffffffu;
+  return bits != 0 && bits - 0x17800000u >= 0x7f800000u - 0x17800000u;
+}
+
 // Interpreter of fl_ew_program, shared by the elementwise-chain kernel and the contraction epilogues.
 // Each case is the expression the standalone kernel of that operation evaluates.
 __device__ __forceinline__ float RunChain(const fl_ew_program &g, float x) {

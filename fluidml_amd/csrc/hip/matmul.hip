@@ -39,11 +39,8 @@
 namespace fl {
 namespace {
 
-typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 // float -> bf16 bits, round to nearest even (NaN stays NaN): the hardware conversion (v_cvt_pk_bf16_f32, two values

@@ -44,6 +44,7 @@ LaunchPlan::~LaunchPlan() {
   for (auto &kv : constants_) fluidml_hip_free(kv.second.device);
   for (auto &kv : privates_) fluidml_hip_free(kv.second.device);
   for (auto &kv : interfaces_) fluidml_hip_free(kv.second.device);
+  for (auto &kv : packed_) fluidml_hip_free(kv.second.device);
   if (arena_) fluidml_hip_arena_destroy(arena_);
   if (stream_) fluidml_hip_stream_destroy(stream_);
 }
@@ -72,6 +73,7 @@ size_t LaunchPlan::GetPrivateBytes() const {
   GetSchedule();
   size_t n = 0;
   for (const auto &kv : privates_) n += kv.second.bytes;
+  for (const auto &kv : packed_) n += kv.second.bytes;
   return n;
 }
 
@@ -170,6 +172,7 @@ void LaunchPlan::Materialize() {
     for (auto &kv : *slots) Check(fluidml_hip_arena_create(kv.second.bytes, &kv.second.device), "allocating a device buffer");
   }
   for (Step &s : steps_) s.kernel->Prepare();
+  PackConvWeights();
   std::vector<Transfer::Slot> in, out;
   for (const Argument &a : arguments_) {
     Transfer::Slot slot;
@@ -280,6 +283,55 @@ void LaunchPlan::FoldNorms() {
       fold(l, l.norm_owner);
     }
   }
+}
+
+// Environment FLUIDML_CONV_PACKED=0 (read at every compile) leaves all weights as they stand.
+void LaunchPlan::PackConvWeights() {
+  const char *env = std::getenv("FLUIDML_CONV_PACKED");
+  if (env != nullptr && std::strtol(env, nullptr, 10) == 0) return;
+  std::vector<std::pair<kernel::TensorView, PackedSlot>> jobs;
+  if (flags_ != 0) return;  // (literal-reference semantics)
+  for (const Launch &l : GetSchedule()) {
+    const Step &step = steps_[l.kind == Launch::Kind::ConvChain ? l.owner : l.members.front()];
+    const flow::OpKind kind = step.node->GetKind();
+    if (kind != flow::OpKind::ConvWithPadding && kind != flow::OpKind::ConvWithoutPadding) continue;
+    if (l.kind == Launch::Kind::ConvChain ? l.has_gate || l.has_skip || l.has_out2 : l.kind != Launch::Kind::Step) continue;
+    const Operand &op = l.kind == Launch::Kind::ConvChain || l.rewired ? l.b : step.in1;
+    if (op.space != Operand::Space::Constant || op.viewed || packed_.count(op.name)) continue;
+    const flow::Attrs &at = step.node->GetAttrs();
+    const std::vector<int64_t> &shape = op.meta.GetShape();
+    const std::vector<int64_t> ones{1, 1};
+    // (fewer than sixteen channels would mostly multiply padding)
+    if (at.group != 1 || at.strides != ones || at.dilations != ones || shape.size() != 4 || shape[1] < 16) continue;
+    const kernel::TensorView w = ViewOf(Resolve(op), op);
+    PackedSlot slot;
+    // bf16 contractions need one part; channels that do not come in sixteens stay fp32 there
+    slot.parts = bf16_ && shape[1] % 16 == 0 ? 1 : 3;
+    const int rc = fluidml_hip_conv3x3_packed_bytes(&w.t, slot.parts, &slot.bytes);
+    if (rc == FL_ERR_UNSUPPORTED) continue;
+    Check(rc, "sizing packed convolution weights");
+    Check(fluidml_hip_arena_create(slot.bytes, &slot.device), "allocating packed convolution weights");
+    packed_[op.name] = slot;
+    jobs.emplace_back(w, slot);
+  }
+  // (the allocations are cleared on the null stream, which the plan's stream does not wait for)
+  Check(fluidml_hip_stream_synchronize(nullptr), "waiting for the cleared buffers");
+  for (const auto &job : jobs) {
+    Check(fluidml_hip_conv3x3_pack(&job.first.t, job.second.parts, job.second.device, stream_), "packing convolution weights");
+  }
+}
+
+int LaunchPlan::IssuePackedConv(const Step &step, const Operand &weights, const fl_tensor &in, const fl_tensor &out,
+                                const fl_ew_program *chain, void *stream) const {
+  const auto it = weights.space == Operand::Space::Constant ? packed_.find(weights.name) : packed_.end();
+  if (it == packed_.end()) return FL_ERR_UNSUPPORTED;
+  const kernel::TensorView w = ViewOf(Resolve(weights), weights);
+  const kernel::DeviceConstant *bias = step.kernel->GetConstant(0);
+  kernel::TensorView c;
+  if (bias != nullptr) c = bias->View();
+  const bool padded = step.node->GetKind() == flow::OpKind::ConvWithPadding;
+  return fluidml_hip_conv3x3_packed_chain(&in, &w.t, it->second.device, it->second.parts, bias ? &c.t : nullptr, &out,
+                                          padded ? step.node->GetAttrs().pads.data() : nullptr, chain, 0, stream);
 }
 
 namespace {
@@ -502,7 +554,9 @@ void LaunchPlan::IssueStep(kernel::LaunchContext &ctx, const Step &s, const Oper
   } else {
     const Operand &op1 = in1_view ? *in1_view : s.in1;
     const kernel::TensorView in1 = ViewOf(Resolve(op1), op1);
-    if (s.has_buffer) dynamic_cast<kernel::DoubleInputsWithBufferKernel &>(*k).Run(ctx, in0, in1, out, buffer);
+    const int rc = IssuePackedConv(s, op1, in0.t, out.t, nullptr, ctx.stream);
+    if (rc != FL_ERR_UNSUPPORTED) ctx.Note(rc, "conv3x3_packed_chain");
+    else if (s.has_buffer) dynamic_cast<kernel::DoubleInputsWithBufferKernel &>(*k).Run(ctx, in0, in1, out, buffer);
     else dynamic_cast<kernel::DoubleInputsWithoutBufferKernel &>(*k).Run(ctx, in0, in1, out);
   }
   if (rc_out != nullptr) {
@@ -691,6 +745,8 @@ void LaunchPlan::Issue(kernel::LaunchContext &ctx, const Launch &l, int *rc_out)
                                               contract_flags | (l.skip_is_factor ? FL_CONTRACT_ADDEND_IS_FACTOR : 0u), ctx.stream);
         break;
       }
+      rc = IssuePackedConv(steps_[l.owner], l.b, a.t, out.t, &l.chain, ctx.stream);
+      if (rc != FL_ERR_UNSUPPORTED) break;
       rc = fluidml_hip_conv_chain(&a.t, &b.t, bias ? &c.t : nullptr, &out.t, padded ? at.pads.data() : nullptr,
                                   at.strides.data(), at.dilations.data(), at.group, &l.chain, contract_flags, ctx.stream);
       break;

@@ -196,7 +196,8 @@ class LaunchPlan {
   size_t GetArenaBytes() const { return arena_bytes_; }
   size_t GetConstantBytes() const;   // constant regions + constants kernels own
   size_t GetInterfaceBytes() const;  // device staging of graph inputs and outputs
-  size_t GetPrivateBytes() const;    // tensors outside the arena: regions no Memory edge uses, outputs of side branches
+  size_t GetPrivateBytes() const;    // buffers outside the arena: regions no Memory edge uses, outputs of side branches,
+                                     // packed weights (once materialised)
   size_t GetPeakDeviceBytes() const { return arena_bytes_ + GetConstantBytes() + GetInterfaceBytes() + GetPrivateBytes(); }
   const std::vector<Step> &GetSteps() const { return steps_; }
   // the launches actually replayed (steps grouped into chains when fusion is on)
@@ -295,6 +296,12 @@ class LaunchPlan {
   // ... and, once per plan, the scale folded into the weights of the contractions that read them, with the two
   // per-column vectors their epilogue needs (new constants "norm_c1:<weights>" and "norm_c2:<weights>")
   void FoldNorms();
+  // Weights of 3x3 convolutions laid out for the matrix cores (fluidml_hip_conv3x3_pack), once per plan; issuing a
+  // convolution whose weights are not among them takes them as they stand.
+  void PackConvWeights();
+  // (FL_ERR_UNSUPPORTED, nothing launched, where they are not, or the operands do not fit)
+  int IssuePackedConv(const Step &step, const Operand &weights, const fl_tensor &in, const fl_tensor &out,
+                      const fl_ew_program *chain, void *stream) const;
   void LaunchAll(kernel::LaunchContext &ctx) const;
   void Replay(kernel::LaunchContext &ctx);
   void PlanBranches() const;
@@ -307,6 +314,10 @@ class LaunchPlan {
   std::map<std::string, ConstantSlot> constants_;
   mutable std::map<std::string, RawSlot> privates_;
   std::map<std::string, RawSlot> interfaces_;
+  struct PackedSlot : RawSlot {
+    int32_t parts = 0;
+  };
+  std::map<std::string, PackedSlot> packed_;  // by the name of the weight constant
   uint32_t flags_ = 0;
   bool use_graph_ = true;
   bool fuse_ = true;

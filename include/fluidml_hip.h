@@ -485,6 +485,16 @@ int fluidml_hip_gemm_chain(const fl_tensor *lhs, const fl_tensor *rhs, const fl_
 /* Conv{With,Without}PaddingKernel -> elementwise chain (reference conv.cpp:27-280);
  * `pads` may be NULL.  ONNX semantics only (no literal-reference flags); `flags` = fl_contract_flags. */
 int fluidml_hip_conv_chain(const fl_tensor *in, const fl_tensor *weights, const fl_tensor *bias, const fl_tensor *out, const int64_t *pads, const int64_t *strides, const int64_t *dilations, int64_t group, const fl_ew_program *chain, uint32_t flags, void *stream);
+/* The same for a 3x3 convolution with unit stride and dilation and group 1 whose weights (fp32, at least 32 filters)
+ * have been laid out for the matrix cores: `packed` holds them as `parts` bf16 values each, 3 (every fp32 value is the
+ * sum of its three parts: fp32 results) or 1 (rounded to bf16: the FL_CONTRACT_BF16 precision).
+ * ..._packed_bytes: size of `packed` for these weights (FL_ERR_UNSUPPORTED where there is no such layout); ..._pack
+ * fills it, once, on `stream`; ..._packed_chain runs the convolution, `weights` are the ones that were packed.  `flags`:
+ * 0, or FL_CONTRACT_TILE(1 | 2) (2 or 4 tiles of 2 x 16 pixels per wave) and FL_CONTRACT_SPLITS(n) instead of the
+ * library's rule. */
+int fluidml_hip_conv3x3_packed_bytes(const fl_tensor *weights, int32_t parts, size_t *bytes);
+int fluidml_hip_conv3x3_pack(const fl_tensor *weights, int32_t parts, void *packed, void *stream);
+int fluidml_hip_conv3x3_packed_chain(const fl_tensor *in, const fl_tensor *weights, const void *packed, int32_t parts, const fl_tensor *bias, const fl_tensor *out, const int64_t *pads, const fl_ew_program *chain, uint32_t flags, void *stream);
 /* [MulCommonKernel(x, scale per channel) ->] Conv{With,Without}PaddingKernel -> elementwise chain [-> AddCommonKernel
  * with a tensor of the output's shape] as ONE launch (reference mul.cpp, conv.cpp:27-280, add.cpp:75-137: the
  * projection of an inverted-residual block behind its squeeze-and-excitation gate, with the skip connection).

@@ -1,0 +1,109 @@
+"""3x3 convolutions against packed weights (fluidml_hip_conv3x3_packed_chain) on the GPU, at the edges of its tiles,
+channel chunks, filter groups and splits, against the oracle; and the values its bf16 parts cannot carry."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from oracle import kernels as ok
+from tests.util import DeviceView, assert_close, some_layouts
+
+pytestmark = pytest.mark.gpu
+RELU = [("EW_RELU", 0.0)]
+
+
+def _run(device, x, w, bias, pads, parts, tile=0, splits=0, chain=RELU, layouts=(None, None, None), times=1):
+    import torch
+
+    from fluidml_amd import cabi
+
+    N, _, H, W = x.shape
+    F = w.shape[0]
+    shape = (N, F, H + pads[0] + pads[2] - 2, W + pads[1] + pads[3] - 2)
+    dx, dw = DeviceView(ok.View(x, layouts[0]), device), DeviceView(ok.View(w, layouts[1]), device)
+    db = DeviceView(ok.View(bias), device) if bias is not None else None
+    do = DeviceView(ok.View.empty(shape, layout=layouts[2], fill=9), device)
+    size = ctypes.c_size_t()
+    cabi.call("conv3x3_packed_bytes", dw.ref(), parts, ctypes.byref(size))
+    packed = torch.zeros(size.value, dtype=torch.uint8, device=device)
+    cabi.call("conv3x3_pack", dw.ref(), parts, packed.data_ptr(), None)
+    program = cabi.make_chain([(getattr(cabi, op), c) for op, c in chain])
+    for _ in range(times):  # (again: the arrival counters of a split launch are back at zero)
+        cabi.call("conv3x3_packed_chain", dx.ref(), dw.ref(), packed.data_ptr(), parts, db.ref() if db else None, do.ref(),
+                  cabi.i64_array(pads), ctypes.byref(program), tile << 4 | splits << 8, None)
+    return do.logical()
+
+
+def _oracle(x, w, bias, pads, relu=True):
+    N, _, H, W = x.shape
+    out = ok.View.empty((N, w.shape[0], H + pads[0] + pads[2] - 2, W + pads[1] + pads[3] - 2))
+    ok.conv(ok.View(x), ok.View(w), ok.View(bias) if bias is not None else None, out, pads, [1, 1], [1, 1], 1)
+    return np.maximum(out.logical(), 0) if relu else out.logical()
+
+
+def _operands(seed, N, C, H, W, F):
+    rng = np.random.default_rng(seed)
+    return (rng.standard_normal((N, C, H, W), np.float32), (rng.standard_normal((F, C, 3, 3)) * (C * 9) ** -0.5).astype(np.float32),
+            rng.standard_normal(F).astype(np.float32))
+
+
+@pytest.mark.parametrize("N,C,H,W,F,pads", [
+    (1, 16, 8, 16, 128, [1, 1, 1, 1]),    # one workgroup of four filter tiles
+    (1, 16, 16, 16, 64, [1, 1, 1, 1]),    # two filter tiles, two rows of waves
+    (2, 32, 9, 17, 65, [1, 1, 1, 1]),     # one past every tile
+    (1, 48, 7, 15, 127, [1, 1, 1, 1]),    # one short of it
+    (1, 17, 10, 20, 32, [0, 0, 0, 0]),    # channels and pads that leave remainders
+    (1, 5, 3, 3, 33, [0, 0, 0, 0]),       # a single output pixel
+    (3, 31, 5, 33, 96, [2, 0, 1, 2]),
+    (1, 160, 6, 6, 160, [1, 1, 1, 1]),    # split by the library's rule
+])
+@pytest.mark.parametrize("tile,splits", [(0, 0), (1, 1), (2, 1), (1, 3), (2, 2)])
+def test_packed_conv(device, N, C, H, W, F, pads, tile, splits):
+    x, w, bias = _operands(7, N, C, H, W, F)
+    print("[case]", N, C, H, W, F, pads, tile, splits, flush=True)
+    got = _run(device, x, w, bias, pads, 3, tile, splits, times=3)
+    assert_close(got, _oracle(x, w, bias, pads), what="three parts")
+    def rounded(v):  # to bf16, nearest even
+        bits = v.view(np.uint32).astype(np.uint64)
+        return ((bits + 0x7FFF + ((bits >> 16) & 1)) & 0xFFFF0000).astype(np.uint32).view(np.float32)
+    got = _run(device, x, w, None, pads, 1, tile, splits, chain=[])
+    assert_close(got, _oracle(rounded(x), rounded(w), None, pads, relu=False), what="bf16")
+
+
+def test_packed_conv_layouts(device):
+    x, w, bias = _operands(8, 2, 24, 11, 18, 40)
+    want = _oracle(x, w, bias, [1, 1, 1, 1])
+    rng = np.random.default_rng(9)
+    for lx, lw, lo in zip(some_layouts(4, rng), some_layouts(4, rng)[::-1], some_layouts(4, rng)):
+        assert_close(_run(device, x, w, bias, [1, 1, 1, 1], 3, layouts=(lx, lw, lo)), want, what=f"{lx} {lw} {lo}")
+
+
+@pytest.mark.parametrize("splits", [1, 2])
+def test_packed_conv_outside_the_parts(device, splits):
+    """Infinities and NaN behave as in fp32, and operands whose parts would be denormal keep their precision."""
+    x, w, bias = _operands(10, 1, 32, 12, 18, 64)
+    x[0, 3, 4, 5], x[0, 30, 9, 0] = np.inf, np.nan
+    w[2, 1, 1, 1] = -np.inf
+    with np.errstate(invalid="ignore"):
+        want = _oracle(x, w, bias, [1, 1, 1, 1], relu=False)
+    got = _run(device, x, w, bias, [1, 1, 1, 1], 3, splits=splits, chain=[])
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    fine = np.isfinite(want)
+    assert_close(got[fine], want[fine], what="finite results beside infinities")
+    x, w, _ = _operands(11, 1, 32, 12, 18, 64)
+    x = np.abs(x) * np.float32(1e-36)
+    got = _run(device, x, np.abs(w), None, [1, 1, 1, 1], 3, splits=splits, chain=[])
+    want = _oracle(x, np.abs(w), None, [1, 1, 1, 1], relu=False)
+    np.testing.assert_allclose(got, want, rtol=1e-5)
+
+
+def test_packed_conv_is_as_exact_as_fp32(device):
+    x, w, _ = _operands(12, 1, 512, 14, 14, 64)
+    pads = [1, 1, 1, 1]
+    got = _run(device, x, w, None, pads, 3, chain=[]).astype(np.float64)
+    padded = np.pad(x.astype(np.float64), ((0, 0), (0, 0), (1, 1), (1, 1)))
+    want = np.zeros(got.shape)
+    for kh in range(3):
+        for kw in range(3):
+            want[0] += np.einsum("fc,chw->fhw", w[:, :, kh, kw].astype(np.float64), padded[0, :, kh:kh + 14, kw:kw + 14])
+    assert np.linalg.norm(got - want) / np.linalg.norm(want) < 3e-7  # (fp32 sums of 4608 products: 4e-7 .. 1.2e-6)
