@@ -1376,6 +1376,8 @@ int LaunchConfig(const MatmulArgs &p, uint32_t n_batch, float *C, const float *A
       // the caller's number or nothing: a tuner must not time one configuration under two names
       if (forced_splits > n_chunks ||
           (forced_splits > 1 && static_cast<int64_t>(forced_splits) * tiles * WM * WN > static_cast<int64_t>(kWorkspaceTiles)) ||
+          // (four arrival counters per tile where each of its four waves finishes a quarter)
+          (forced_splits > 1 && WM * WN == 1 && tiles * 4 > static_cast<int64_t>(kWorkspaceTiles)) ||
           (n_chunks + forced_splits - 1) / forced_splits * (forced_splits - 1) >= n_chunks) {
         return FL_ERR_UNSUPPORTED;
       }
