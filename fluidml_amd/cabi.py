@@ -160,6 +160,8 @@ SIGNATURES = {
     "fluidml_hip_max_pool_without_padding": [_T, _T, _i64p, _i64p, _i32, _vp],
     "fluidml_hip_average_pool_without_padding": [_T, _T, _i64p, _i64p, _i32, _vp],
     # contractions
+    "fluidml_hip_contract_pack": [_T, _i32, _i64, _i32, _vp, _P(_vp), _P(_sz)],
+    "fluidml_hip_contract_unpack": [_vp],
     "fluidml_hip_matmul": [_T, _T, _T, _vp],
     "fluidml_hip_matmul_no_alloc": [_T, _T, _T, _vp],
     "fluidml_hip_matmul_bf16": [_T, _T, _T, _vp],

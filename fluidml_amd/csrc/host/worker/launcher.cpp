@@ -41,6 +41,7 @@ LaunchPlan::~LaunchPlan() {
   if (graph_) fluidml_hip_graph_destroy(graph_);
   for (void *e : region_events_) fluidml_hip_event_destroy(e);
   if (side_stream_) fluidml_hip_stream_destroy(side_stream_);
+  for (auto &kv : contract_packed_) fluidml_hip_contract_unpack(kv.second.device);
   for (auto &kv : constants_) fluidml_hip_free(kv.second.device);
   for (auto &kv : privates_) fluidml_hip_free(kv.second.device);
   for (auto &kv : interfaces_) fluidml_hip_free(kv.second.device);
@@ -74,6 +75,7 @@ size_t LaunchPlan::GetPrivateBytes() const {
   size_t n = 0;
   for (const auto &kv : privates_) n += kv.second.bytes;
   for (const auto &kv : packed_) n += kv.second.bytes;
+  for (const auto &kv : contract_packed_) n += kv.second.bytes;
   return n;
 }
 
@@ -173,6 +175,7 @@ void LaunchPlan::Materialize() {
   }
   for (Step &s : steps_) s.kernel->Prepare();
   PackConvWeights();
+  PackContractionWeights();
   std::vector<Transfer::Slot> in, out;
   for (const Argument &a : arguments_) {
     Transfer::Slot slot;
@@ -318,6 +321,40 @@ void LaunchPlan::PackConvWeights() {
   Check(fluidml_hip_stream_synchronize(nullptr), "waiting for the cleared buffers");
   for (const auto &job : jobs) {
     Check(fluidml_hip_conv3x3_pack(&job.first.t, job.second.parts, job.second.device, stream_), "packing convolution weights");
+  }
+}
+
+// Environment FLUIDML_MATMUL_PACKED=0 (read at every compile) leaves all weights as they stand.
+void LaunchPlan::PackContractionWeights() {
+  const char *env = std::getenv("FLUIDML_MATMUL_PACKED");
+  if (flags_ != 0 || (env != nullptr && std::strtol(env, nullptr, 10) == 0)) return;
+  auto pack = [&](const Operand &lhs, const Operand &rhs, bool trans_a, bool trans_b) {
+    if (rhs.space != Operand::Space::Constant || rhs.viewed || contract_packed_.count(rhs.name)) return;
+    const std::vector<int64_t> &shape = lhs.meta.GetShape();
+    if (rhs.meta.GetShape().size() != 2 || shape.size() < 2 || trans_a) return;
+    int64_t rows = 1;
+    for (size_t d = 0; d + 1 < shape.size(); ++d) rows *= shape[d];
+    if (shape.back() % 8 != 0) return;
+    const kernel::TensorView w = ViewOf(Resolve(rhs), rhs);
+    RawSlot slot;
+    const int rc = fluidml_hip_contract_pack(&w.t, trans_b ? 1 : 0, rows, bf16_ ? 1 : 3, stream_, &slot.device, &slot.bytes);
+    if (rc == FL_ERR_UNSUPPORTED) return;
+    Check(rc, "packing contraction weights");
+    contract_packed_[rhs.name] = slot;
+  };
+  for (const Launch &l : GetSchedule()) {
+    if (l.kind == Launch::Kind::MatMulGroup) {
+      for (const Launch &m : l.group) pack(l.a, m.b, false, false);
+    } else if (l.kind == Launch::Kind::MatMulChain) {
+      pack(l.a, l.b, false, false);
+    } else if (l.kind == Launch::Kind::GemmChain || l.kind == Launch::Kind::Step) {
+      const Step &step = steps_[l.kind == Launch::Kind::Step ? l.members.front() : l.owner];
+      const flow::OpKind kind = step.node->GetKind();
+      if (kind != flow::OpKind::MatMul && kind != flow::OpKind::GemmConstantWeightsBias) continue;
+      const flow::Attrs &at = step.node->GetAttrs();
+      const bool gemm = kind == flow::OpKind::GemmConstantWeightsBias, own = l.kind != Launch::Kind::Step || l.rewired;
+      pack(own ? l.a : step.in0, own ? l.b : step.in1, gemm && at.trans_a, gemm && at.trans_b);
+    }
   }
 }
 

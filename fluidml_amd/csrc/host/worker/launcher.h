@@ -299,6 +299,8 @@ class LaunchPlan {
   // Weights of 3x3 convolutions laid out for the matrix cores (fluidml_hip_conv3x3_pack), once per plan; issuing a
   // convolution whose weights are not among them takes them as they stand.
   void PackConvWeights();
+  // The same for the weights of MatMul and Gemm (fluidml_hip_contract_pack); the library finds them by their address.
+  void PackContractionWeights();
   // (FL_ERR_UNSUPPORTED, nothing launched, where they are not, or the operands do not fit)
   int IssuePackedConv(const Step &step, const Operand &weights, const fl_tensor &in, const fl_tensor &out,
                       const fl_ew_program *chain, void *stream) const;
@@ -317,7 +319,8 @@ class LaunchPlan {
   struct PackedSlot : RawSlot {
     int32_t parts = 0;
   };
-  std::map<std::string, PackedSlot> packed_;  // by the name of the weight constant
+  std::map<std::string, PackedSlot> packed_;      // by the name of the weight constant
+  std::map<std::string, RawSlot> contract_packed_;
   uint32_t flags_ = 0;
   bool use_graph_ = true;
   bool fuse_ = true;

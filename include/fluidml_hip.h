@@ -133,7 +133,14 @@ enum fl_contract_tile {
   FL_TILE_64x64_K2 = 6,     /*   64x64 tile, 2x2 waves times two K slices (eight waves) */
   FL_TILE_128x64 = 7,       /*   128x64 tile, 4x2 waves */
   FL_TILE_128x128_STAGED = 8, /* bf16 operands only: 128x128 tile, 2x2 waves with 2x2 accumulators each, four K chunks in flight */
-  FL_TILE_COUNT = 9
+  FL_TILE_COUNT = 9,
+  /* against packed weights (fluidml_hip_contract_pack) only, operands as bf16 parts; no entries of a tuner's table: where
+   * such weights are worth having, FL_TILE_RULE takes one of these */
+  FL_TILE_PACKED_32x64 = 9,       /* two waves side by side times four K slices */
+  FL_TILE_PACKED_64x64 = 10,      /* two times two, two row tiles per wave */
+  FL_TILE_PACKED_64x128 = 11,     /* four waves side by side, two row tiles each */
+  FL_TILE_PACKED_64x128_K2 = 12,  /* the same times two K slices */
+  FL_TILE_PACKED_128x128_K2 = 13  /* four row tiles each */
 };
 #define FL_CONTRACT_TILE_SHIFT 4
 #define FL_CONTRACT_SPLIT_SHIFT 8
@@ -480,6 +487,15 @@ typedef struct fl_norm_fusion {
  * statistics, the epilogue's correction and the addends stay fp32.  The tile configuration bits of `flags` apply
  * (FL_TILE_128x128_STAGED: deferred rows of at most 512 elements). */
 int fluidml_hip_matmul_chain_group_norm(int32_t count, const fl_tensor *lhs, const fl_tensor *const *rhs, const fl_tensor *const *bias, const fl_tensor *const *col_sum, const fl_tensor *const *out, int64_t n_inner, const int64_t *stride_outer, const fl_ew_program *chain, const fl_tensor *addend, const fl_norm_fusion *norm, uint32_t flags, void *stream);
+/* Lays constant weights out for the matrix cores, once: `rhs` is the rank-2 right operand of a MatMul ([K, N]) or, with
+ * `trans_b`, of a Gemm ([N, K]) whose left operand has `rows` rows (FL_ERR_UNSUPPORTED where the other kernels are the
+ * faster ones at that size).  Every value is stored as `parts` bf16 values, 3 (it is the sum of the three: fp32
+ * results) or 1 (rounded to bf16, for calls with FL_CONTRACT_BF16).  From then on every contraction of this library
+ * whose right operand is `rhs` (address, extents and strides) may use the packed form, which therefore has to be current:
+ * the weights must not change before fluidml_hip_contract_unpack(*packed), which frees it.  The packing runs on `stream`;
+ * a contraction on another stream has to be ordered behind it by the caller.  `*bytes`: size of the packed form. */
+int fluidml_hip_contract_pack(const fl_tensor *rhs, int32_t trans_b, int64_t rows, int32_t parts, void *stream, void **packed, size_t *bytes);
+int fluidml_hip_contract_unpack(void *packed);
 /* GemmConstantWeightsBiasKernel -> elementwise chain (reference gemm.cpp:39-182); `flags` = fl_contract_flags. */
 int fluidml_hip_gemm_chain(const fl_tensor *lhs, const fl_tensor *rhs, const fl_tensor *bias, const fl_tensor *out, double alpha, double beta, int32_t trans_a, int32_t trans_b, const fl_ew_program *chain, uint32_t flags, void *stream);
 /* Conv{With,Without}PaddingKernel -> elementwise chain (reference conv.cpp:27-280);

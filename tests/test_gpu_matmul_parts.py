@@ -1,0 +1,208 @@
+"""Contractions against packed weights (fluidml_hip_contract_pack) on the GPU: every tile at its edges, with K split over
+workgroups, against a float64 product; every epilogue against the same call before the weights were packed; and the
+values its bf16 parts cannot carry."""
+import ctypes
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+TILES = {"32x64": 9, "64x64": 10, "64x128": 11, "64x128_K2": 12, "128x128_K2": 13}
+UNSUPPORTED = -8
+
+
+class Problem:
+    """x [M, K] against `count` weights [K, N] (or [N, K]), their packed forms held while the object lives."""
+
+    def __init__(self, device, M, K, N, count=1, trans_b=False, seed=0, scale=1.0):
+        import torch
+
+        from fluidml_amd import cabi
+
+        self.torch, self.cabi, self.M, self.K, self.N = torch, cabi, M, K, N
+        g = torch.Generator(device=device)
+        g.manual_seed(seed + M * 7 + K * 3 + N)
+        self.rand = lambda *s: torch.randn(*s, device=device, generator=g)
+        self.x = self.rand(M, K) * scale
+        self.w = [self.rand(*((N, K) if trans_b else (K, N))) * K ** -0.5 for _ in range(count)]
+        self.b = [self.rand(N) for _ in range(count)]
+        self.trans_b, self.packed = trans_b, []
+
+    def pack(self, parts=3):
+        for w in self.w:
+            p, n = ctypes.c_void_p(), ctypes.c_size_t()
+            # (a number of rows at which packing is always worth it: the small problems here test the edges)
+            self.cabi.call("contract_pack", self.ref(w), int(self.trans_b), 1 << 40, parts, None, ctypes.byref(p), ctypes.byref(n))
+            self.packed.append(p)
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *_):
+        self.torch.cuda.synchronize()
+        for p in self.packed:
+            self.cabi.call("contract_unpack", p)
+
+    def tensor(self, t, shape=None, strides=None):
+        return self.cabi.make_tensor(t.data_ptr(), self.cabi.FL_FLOAT32, shape or t.shape, strides or t.stride())
+
+    def ref(self, t, shape=None, strides=None):
+        return ctypes.byref(self.tensor(t, shape, strides))
+
+    def list(self, ts):
+        ptr = ctypes.POINTER(self.cabi.FlTensor)
+        return (ptr * len(ts))(*[ctypes.pointer(t if isinstance(t, self.cabi.FlTensor) else self.tensor(t)) for t in ts])
+
+    def out(self):
+        return self.torch.full((self.M, self.N), 9.0, device=self.x.device)
+
+    def chain(self, out, flags, steps=()):
+        return self.cabi.lib.fluidml_hip_matmul_chain(self.ref(self.x), self.ref(self.w[0]), self.ref(self.b[0]), self.ref(out),
+                                                      ctypes.byref(self.cabi.make_chain(steps)), flags, None)
+
+
+def flags_of(tile, splits=1):
+    return TILES[tile] << 4 | splits << 8
+
+
+def close(got, want, what):
+    got, want = got.double().cpu().numpy(), want.double().cpu().numpy()
+    assert np.isfinite(got).all(), what
+    err = np.abs(got - want)
+    assert (err <= 1e-5 + 1e-4 * np.abs(want)).all(), f"{what}: max err {err.max():.3e}"
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("M,K,N", [
+    (1, 8, 1), (32, 16, 32), (33, 24, 65), (63, 128, 127), (65, 136, 129), (127, 248, 33), (128, 256, 128), (129, 520, 257), (40, 768, 64),
+])
+def test_packed_tiles(device, tile, M, K, N):
+    print("[case]", tile, M, K, N, flush=True)
+    with Problem(device, M, K, N) as p:
+        want = p.x.double() @ p.w[0].double() + p.b[0].double()
+        p.pack()
+        ran = 0
+        for splits in (1, 2, 3, 8):
+            for _ in range(2):  # (again: the arrival counters are back at zero)
+                out = p.out()
+                rc = p.chain(out, flags_of(tile, splits))
+                if rc == UNSUPPORTED:
+                    assert splits > 1  # too few chunks of K
+                    continue
+                assert rc == 0
+                close(out, want, f"{tile} {splits} splits")
+                ran += 1
+        assert ran >= 2
+        if K >= 512:
+            rel = ((out.double() - want).norm() / want.norm()).item() if rc == 0 else 0.0
+            assert rel < 1.5e-7  # (the fp32 instruction: 1.8e-7 at 768 products)
+
+
+@pytest.mark.parametrize("tile", TILES)
+def test_packed_bf16(device, tile):
+    for M, K, N in [(33, 264, 65), (128, 768, 96)]:
+        with Problem(device, M, K, N) as p:
+            want = p.x.bfloat16().double() @ p.w[0].bfloat16().double() + p.b[0].double()
+            p.pack(1)
+            out = p.out()
+            assert p.chain(out, flags_of(tile) | p.cabi.FL_CONTRACT_BF16) == 0
+            close(out, want, "bf16")
+            assert p.chain(out, flags_of(tile)) == UNSUPPORTED  # (packed for the other precision)
+
+
+@pytest.mark.parametrize("tile,splits", [(t, s) for t in TILES for s in (1, 2)])
+def test_packed_epilogues(device, tile, splits):
+    """Bias and elementwise chain, addends, siblings with split columns, both forms of a deferred LayerNormalization,
+    row statistics: each call before packing (any tile) and after (this tile)."""
+    M, K, N = 70, 288, 160
+    print("[case]", tile, splits, flush=True)
+    with Problem(device, M, K, N, count=3) as p:
+        cabi, torch = p.cabi, p.torch
+        e1, e2, x3 = p.rand(M, N), p.rand(M, N), p.rand(M, K)
+        gamma, beta, c1 = p.rand(N), p.rand(N), [w.sum(0) for w in p.w]
+        stats_k = torch.empty(M, K // 32, 2, device=device)
+        stats_n = torch.empty(M, N // 32, 2, device=device)
+        for stats, t in ((stats_k, p.x), (stats_n, e1)):
+            runs = t.reshape(M, -1, 32)
+            stats[..., 0] = runs.mean(-1)
+            stats[..., 1] = ((runs - runs.mean(-1, keepdim=True)) ** 2).sum(-1)
+
+        def norm(deferred, width=0, stats=None, stats_out=None, addend2=None):
+            n = cabi.FlNormFusion()
+            n.deferred, n.width, n.epsilon = deferred, width, 1e-5
+            n.stats = stats.data_ptr() if stats is not None else None
+            n.stats_out = stats_out.data_ptr() if stats_out is not None else None
+            if deferred == cabi.FL_NORM_ADDEND:
+                n.scale, n.shift = ctypes.pointer(p.tensor(gamma)), ctypes.pointer(p.tensor(beta))
+            if addend2 is not None:
+                n.addend2 = ctypes.pointer(p.tensor(addend2))
+            return n
+
+        def calls(flags):
+            res = []
+            out = p.out()
+            gelu = [(cabi.EW_DIV_C, 2 ** 0.5), (cabi.EW_ERF, 0.0), (cabi.EW_ADD_C, 1.0), (cabi.EW_MUL_X, 0.0), (cabi.EW_MUL_C, 0.5)]
+            assert p.chain(out, flags, gelu) == 0
+            res.append(out)
+            out = p.out()
+            none = ctypes.byref(cabi.make_chain([]))
+            assert cabi.lib.fluidml_hip_matmul_chain_add(p.ref(p.x), p.ref(p.w[0]), p.ref(p.b[0]), p.ref(out), none, p.ref(e1), p.ref(e2), flags, None) == 0
+            res.append(out)
+            # siblings, 160 columns as 5 heads of 32 that a transpose moved apart: [5, M, 32]
+            outs = [torch.full((5, M, 32), 9.0, device=device) for _ in range(3)]
+            views = [p.tensor(o, (M, N), (32, 1)) for o in outs]
+            outer = cabi.i64_array([32 * M] * 3)
+            assert cabi.lib.fluidml_hip_matmul_chain_group(3, p.ref(p.x), p.list(p.w), p.list(p.b), p.list(views), 32, outer, none, flags, None) == 0
+            res += outs
+            # LayerNormalization of the left operand, two projections
+            outs = [p.out() for _ in range(2)]
+            n = norm(cabi.FL_NORM_LHS, K, stats_k)
+            assert cabi.lib.fluidml_hip_matmul_chain_group_norm(2, p.ref(p.x), p.list(p.w[:2]), p.list(p.b[:2]), p.list(c1[:2]), p.list(outs), 0, None, none,
+                                                                None, ctypes.byref(n), flags, None) == 0
+            res += outs
+            # LayerNormalization of the addend, a second addend, statistics of the result
+            out, stats = p.out(), torch.full((M, N // 32, 2), 9.0, device=device)
+            n = norm(cabi.FL_NORM_ADDEND, N, stats_n, stats, e2)
+            assert cabi.lib.fluidml_hip_matmul_chain_group_norm(1, p.ref(x3), p.list(p.w[2:]), p.list(p.b[2:]), None, p.list([out]), 0, None, none,
+                                                                p.ref(e1), ctypes.byref(n), flags, None) == 0
+            return res + [out, stats]
+
+        want = calls(0)
+        p.pack()
+        for i, (got, ref) in enumerate(zip(calls(flags_of(tile, splits)), want)):
+            close(got, ref, f"result {i}")
+
+
+def test_packed_gemm(device):
+    with Problem(device, 48, 200, 72, trans_b=True) as p:
+        def call(flags):
+            out = p.out()
+            none = ctypes.byref(p.cabi.make_chain([]))
+            assert p.cabi.lib.fluidml_hip_gemm_chain(p.ref(p.x), p.ref(p.w[0]), p.ref(p.b[0]), p.ref(out), 0.5, 2.0, 0, 1, none, flags, None) == 0
+            return out
+        want = call(0)
+        p.pack()
+        close(call(flags_of("32x64")), want, "gemm")
+
+
+@pytest.mark.parametrize("tile", TILES)
+def test_packed_outside_the_parts(device, tile):
+    """Infinities and NaN behave as in fp32, and operands whose parts would be denormal keep their precision."""
+    with Problem(device, 70, 200, 100) as p:
+        p.x[3, 7], p.x[69, 199], p.w[0][11, 99] = float("inf"), float("nan"), float("-inf")
+        want = p.x.double() @ p.w[0].double() + p.b[0].double()
+        p.pack()
+        out = p.out()
+        assert p.chain(out, flags_of(tile)) == 0
+        assert p.torch.equal(out.isnan(), want.isnan()) and p.torch.equal(out.isinf(), want.isinf())
+        fine = want.isfinite()
+        close(out[fine], want[fine], "finite results beside infinities")
+    with Problem(device, 40, 96, 64, scale=1e-36) as p:
+        p.x.abs_()
+        p.w[0].abs_()
+        p.b[0].zero_()
+        want = p.x.double() @ p.w[0].double()
+        p.pack()
+        out = p.out()
+        assert p.chain(out, flags_of(tile)) == 0
+        np.testing.assert_allclose(out.double().cpu().numpy(), want.cpu().numpy(), rtol=1e-5)
