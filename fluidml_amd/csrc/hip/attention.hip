@@ -5,16 +5,21 @@
 // -> MatMulKernel (reference matmul.cpp:28-59, div.cpp:24-56, mul.cpp, add.cpp:75-137, where.cpp:17-150,
 // softmax.cpp:22-139) without writing the [.., Sq, Skv] score and probability tensors.
 //
-// One workgroup (4 waves) owns 16 query rows of one batch element (head), so that even a single sequence
-// spreads over many compute units; the kernel is latency bound and every phase is kept short:
-//   1. Q block and K^T chunk (128 keys) travel global -> registers -> LDS, 128 bits at a time when the
-//      operands allow it; the V chunk, the mask and the condition are requested before the first MFMA.
-//   2. wave w computes the 16x32 scores of keys [128c + 32w, +32) with v_mfma_f32_16x16x4_f32 and writes them
-//      to an LDS score strip [16][Skv].
-//   3. the strip is re-read row-wise (16 lanes per row, contiguous keys per lane): scale, mask, condition,
-//      maximum, exp and sum with four shuffle steps each; the unnormalised exp goes back to the strip.
-//   4. wave w multiplies the strip with columns [16w, +16) of V (all keys), so no partial sums cross waves,
-//      and divides by the row sum while storing.
+// One workgroup owns 16 query rows of one batch element (head), so that even a single sequence spreads over many
+// compute units, and its waves share out the keys.  The kernel is a chain of latencies more than anything else, so
+// nothing stands in it that could be left out: no operand is staged in LDS, and no value changes its lane.
+//   1. scores, transposed: v_mfma_f32_16x16x4_f32 with the keys as rows and the queries as columns.  A lane feeds it
+//      K^T[d][key lane % 16] and Q[query lane % 16][d] and receives the scores of ITS query (lane % 16) with the keys
+//      16 t + 4 (lane / 16) + i of every key tile t.
+//   2. scale, mask, condition, and the maximum over the wave's own keys: registers and two shuffles.
+//   3. context, transposed: the product with V^T (head columns as rows, queries as columns) wants of a lane
+//      P[key 4 (lane / 16) + i][query lane % 16] in step i -- register i of the scores as they lie.
+//   4. every wave leaves its context, its maximum and its sum of exponentials in LDS; after the only barrier the
+//      contexts are added, each scaled by exp(its maximum - the row's), and divided by the row's sum.
+// All loads leave at once, and none needs more than the alignment of a float, so odd lengths cost nothing.  Measured
+// (us in a replayed graph, heads x queries x keys, 64 columns; before: scores through an LDS strip, K and V staged in LDS):
+//   12 x 128 x 128 6.8 -> 5.5, 12 x 37 x 37 9.6 -> 4.3, 8 x 77 x 77 9.5 -> 5.3, 8 x 256 x 256 11.4 -> 7.8,
+//   12 x 512 x 512 31 (score MatMul, Softmax, MatMul) -> 23
 // Every operand is addressed through element strides, so the head split of the producers and the head merge
 // of the consumer need no copies.
 #include "fl_common.h"
@@ -24,12 +29,9 @@ namespace {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-constexpr int kQ = 16;        // query rows per workgroup
-constexpr int kKeys = 128;    // keys per chunk (32 per wave)
-constexpr int kMaxD = 64;     // head dim limit
-constexpr int kLdQ = kMaxD + 4;
-constexpr int kLdK = kKeys + 4;
-constexpr int kLdV = kMaxD + 4;
+constexpr int kQ = 16;       // query rows per workgroup
+constexpr int kMaxD = 64;    // head dim limit
+constexpr int kMaxKeys = 512;
 
 struct AttentionArgs {
   NestArgs<6> batch;  // operands: 0 out, 1 q, 2 kt, 3 v, 4 mask, 5 cond
@@ -40,20 +42,27 @@ struct AttentionArgs {
   int32_t scale_is_divisor;
   float fill;
   uint32_t q_blocks;
+  int32_t vec_q;  // four consecutive d of a query are 16 aligned bytes
 };
 
-// VEC: q, kt and v are unit-stride along (d, key, d), every other stride, the batch offsets, D and Skv are
-// multiples of four elements and the bases are 16-byte aligned.
-template <int CHUNKS, bool VEC>
-__global__ __launch_bounds__(256) void AttentionKernel(AttentionArgs a, float *__restrict__ out, const float *__restrict__ q,
-                                                       const float *__restrict__ kt, const float *__restrict__ v,
-                                                       const float *__restrict__ mask, const uint8_t *__restrict__ cond) {
-  constexpr int kLdP = CHUNKS * kKeys + 4;
-  constexpr int kNpt = CHUNKS * kKeys / 16;  // keys per lane in the row-wise phase
-  __shared__ __attribute__((aligned(16))) float qs[kQ * kLdQ];
-  __shared__ __attribute__((aligned(16))) float kv[kKeys * kLdV > kMaxD * kLdK ? kKeys * kLdV : kMaxD * kLdK];
-  __shared__ __attribute__((aligned(16))) float ps[kQ * kLdP];
-  __shared__ float row_sum[kQ];
+// Consecutive floats, at any address.
+template <int N>
+struct __attribute__((packed, aligned(4))) Run {
+  float v[N];
+};
+
+// NW waves with KT tiles of 16 keys each, DT tiles of 16 head columns; FULL: D = 16 DT.
+// VEC: head columns lie at unit stride in V (FULL).  Which of them is row r of which tile is free: the tiles are then
+// interleaved, row r of tile j is column DT r + j, so that one load brings a lane its row of every tile (12 heads x 128 x 128
+// 6.0 -> 5.5 us).  The same for the keys, one load for a lane's row of every key tile, was slower (6.1, with 256 keys 9.0
+// instead of 8.1).
+template <int NW, int KT, int DT, bool FULL, bool VEC>
+__global__ __launch_bounds__(64 * NW) void AttentionKernel(AttentionArgs a, float *__restrict__ out, const float *__restrict__ q,
+                                                           const float *__restrict__ kt, const float *__restrict__ v,
+                                                           const float *__restrict__ mask, const uint8_t *__restrict__ cond) {
+  constexpr int kLd = 16 * DT + 4;  // floats per query in LDS: lanes of consecutive queries in different banks
+  __shared__ __attribute__((aligned(16))) float ctx[NW * kQ * kLd];
+  __shared__ float stat[2][NW][kQ];  // the waves' maxima and sums
 
   // Workgroup ids go round the 8 XCDs; renumbered so that each XCD takes a contiguous run of (head, query block)
   // pairs, a head's K and V are fetched by one or two of the L2s instead of all eight.
@@ -62,230 +71,173 @@ __global__ __launch_bounds__(256) void AttentionKernel(AttentionArgs a, float *_
   const uint32_t qb = bid % a.q_blocks;
   int32_t off[6] = {0, 0, 0, 0, 0, 0};
   a.batch.AddOffsets(bid / a.q_blocks, off);
-  const int m0 = static_cast<int>(qb) * kQ;
-  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64, l16 = lane % 16, grp = lane / 16;
+  const int tid = threadIdx.x, lane = tid % 64, l16 = lane % 16, grp = lane / 16;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int m0 = static_cast<int>(qb) * kQ, n0 = wave * KT * 16;
+  const int last_key = a.Skv - 1;
+  auto key = [&](int t, int r) { return n0 + 16 * t + r; };
+  auto column = [&](int j, int r) { return VEC ? DT * r + j : 16 * j + r; };
 
-  // Tiles travel global -> registers -> LDS in two phases so that all of a thread's loads are in flight together
-  // and the next tile's loads overlap the current tile's MFMAs.  Out-of-range elements read the slice's first
-  // element (always present) and are replaced by zero on the way into LDS.
-  constexpr int kPer = kKeys * kMaxD / 256;  // 32 elements of a K^T or V tile per thread
-  float stage[kPer];
-  uint32_t stage_ok = 0;
-  const bool k_lanes_along_d = a.sKd <= a.sKn, v_lanes_along_d = a.sVd <= a.sVn;
-  auto tile_index = [&](int i, bool along_d, int &n, int &k) {
-    const int it = tid + i * 256;
-    n = along_d ? it / kMaxD : it % kKeys;
-    k = along_d ? it % kMaxD : it / kKeys;
-  };
-  auto load_k = [&](int c) {
-    stage_ok = 0;
-    if constexpr (VEC) {
+  // ---- requests: K, Q, mask and condition, then V --------------------------------------------------------------
+  // d runs in the order 16 j + 4 (lane / 16) + e, the same for both operands, so that a lane's Q is four consecutive d
+  float kreg[KT][DT][4], qreg[DT][4];
+  const float *kb = kt + off[2], *qp = q + off[1] + min(m0 + l16, a.Sq - 1) * a.sQm;
 #pragma unroll
-      for (int i = 0; i < kPer / 4; ++i) {
-        const int it = tid + i * 256, k = it / (kKeys / 4), n = it % (kKeys / 4) * 4;
-        const bool ok = c * kKeys + n < a.Skv && k < a.D;
-        const floatx4 x = *reinterpret_cast<const floatx4 *>(kt + off[2] + (ok ? k * a.sKd + c * kKeys + n : 0));
-        stage[4 * i] = x.x, stage[4 * i + 1] = x.y, stage[4 * i + 2] = x.z, stage[4 * i + 3] = x.w;
-        stage_ok |= static_cast<uint32_t>(ok) << i;
-      }
+  for (int j = 0; j < DT; ++j) {
+    const int d0 = 16 * j + 4 * grp;
+    if (a.vec_q) {
+      const floatx4 x = *reinterpret_cast<const floatx4 *>(qp + (FULL || d0 < a.D ? d0 : 0));
+      qreg[j][0] = x.x, qreg[j][1] = x.y, qreg[j][2] = x.z, qreg[j][3] = x.w;
     } else {
 #pragma unroll
-      for (int i = 0; i < kPer; ++i) {
-        int n, k;
-        tile_index(i, k_lanes_along_d, n, k);
-        const bool ok = c * kKeys + n < a.Skv && k < a.D;
-        stage[i] = kt[off[2] + (ok ? k * a.sKd + (c * kKeys + n) * a.sKn : 0)];
-        stage_ok |= static_cast<uint32_t>(ok) << i;
-      }
-    }
-  };
-  auto load_v = [&](int c) {
-    stage_ok = 0;
-    if constexpr (VEC) {
-#pragma unroll
-      for (int i = 0; i < kPer / 4; ++i) {
-        const int it = tid + i * 256, n = it / (kMaxD / 4), k = it % (kMaxD / 4) * 4;
-        const bool ok = c * kKeys + n < a.Skv && k < a.D;
-        const floatx4 x = *reinterpret_cast<const floatx4 *>(v + off[3] + (ok ? (c * kKeys + n) * a.sVn + k : 0));
-        stage[4 * i] = x.x, stage[4 * i + 1] = x.y, stage[4 * i + 2] = x.z, stage[4 * i + 3] = x.w;
-        stage_ok |= static_cast<uint32_t>(ok) << i;
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < kPer; ++i) {
-        int n, k;
-        tile_index(i, v_lanes_along_d, n, k);
-        const bool ok = c * kKeys + n < a.Skv && k < a.D;
-        stage[i] = v[off[3] + (ok ? (c * kKeys + n) * a.sVn + k * a.sVd : 0)];
-        stage_ok |= static_cast<uint32_t>(ok) << i;
-      }
-    }
-  };
-  auto store_stage = [&](bool along_d, bool transposed) {  // transposed: LDS [k][n] (K^T), else [n][k] (V)
-    if constexpr (VEC) {
-#pragma unroll
-      for (int i = 0; i < kPer / 4; ++i) {
-        const int it = tid + i * 256;
-        const bool ok = stage_ok >> i & 1u;
-        floatx4 x = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (ok) x = floatx4{stage[4 * i], stage[4 * i + 1], stage[4 * i + 2], stage[4 * i + 3]};
-        float *dst = transposed ? kv + it / (kKeys / 4) * kLdK + it % (kKeys / 4) * 4
-                                : kv + it / (kMaxD / 4) * kLdV + it % (kMaxD / 4) * 4;
-        *reinterpret_cast<floatx4 *>(dst) = x;
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < kPer; ++i) {
-        int n, k;
-        tile_index(i, along_d, n, k);
-        kv[transposed ? k * kLdK + n : n * kLdV + k] = (stage_ok >> i & 1u) ? stage[i] : 0.0f;
-      }
-    }
-  };
-
-  // ---- Q block -> LDS [m][k], zero padded; the first K^T chunk is requested with it ------------------------
-  {
-    constexpr int kPerQ = kQ * kMaxD / 256;  // 4
-    float qreg[kPerQ];
-    if constexpr (VEC) {
-      const int m = tid / (kMaxD / 4), k = tid % (kMaxD / 4) * 4;
-      const bool ok = m0 + m < a.Sq && k < a.D;
-      floatx4 x = *reinterpret_cast<const floatx4 *>(q + off[1] + (ok ? (m0 + m) * a.sQm + k : 0));
-      if (!ok) x = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-      load_k(0);
-      *reinterpret_cast<floatx4 *>(qs + m * kLdQ + k) = x;
-    } else {
-#pragma unroll
-      for (int i = 0; i < kPerQ; ++i) {
-        const int it = tid + i * 256, m = it / kMaxD, k = it % kMaxD;
-        const bool ok = m0 + m < a.Sq && k < a.D;
-        qreg[i] = q[off[1] + (ok ? (m0 + m) * a.sQm + k * a.sQd : 0)];
-        if (!ok) qreg[i] = 0.0f;
-      }
-      load_k(0);
-#pragma unroll
-      for (int i = 0; i < kPerQ; ++i) {
-        const int it = tid + i * 256;
-        qs[(it / kMaxD) * kLdQ + it % kMaxD] = qreg[i];
-      }
+      for (int e = 0; e < 4; ++e) qreg[j][e] = qp[(FULL ? d0 + e : min(d0 + e, a.D - 1)) * a.sQd];
     }
   }
-  // row-wise phase: lane handles query row tid / 16, keys [kNpt * (tid % 16), +kNpt); its mask and condition
-  // values are requested now
-  const int rw_row = tid / 16, rw_n0 = tid % 16 * kNpt;
-  float mask_v[kNpt];
-  uint32_t keep = ~0u;
-  {
-    const bool row_ok = m0 + rw_row < a.Sq;
-    uint8_t cond_v[kNpt];
 #pragma unroll
-    for (int i = 0; i < kNpt; ++i) {
-      const bool ok = row_ok && rw_n0 + i < a.Skv;
-      mask_v[i] = mask != nullptr ? mask[off[4] + (ok ? (m0 + rw_row) * a.sMm + (rw_n0 + i) * a.sMn : 0)] : 0.0f;
-      cond_v[i] = cond != nullptr ? cond[off[5] + (ok ? (m0 + rw_row) * a.sCm + (rw_n0 + i) * a.sCn : 0)] : uint8_t{1};
-    }
+  for (int t = 0; t < KT; ++t) {
+    const float *at = kb + min(key(t, l16), last_key) * a.sKn;
+#pragma unroll
+    for (int j = 0; j < DT; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int d = 16 * j + 4 * grp + e;
+        kreg[t][j][e] = at[(FULL ? d : min(d, a.D - 1)) * a.sKd];
+      }
+  }
+  float mreg[KT][4];
+  uint32_t keep = ~0u;  // bit 4 t + i
+  {
+    const int m = min(m0 + l16, a.Sq - 1);
+    uint8_t creg[KT][4];
+#pragma unroll
+    for (int t = 0; t < KT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int n = min(key(t, 4 * grp + i), last_key);
+        mreg[t][i] = mask != nullptr ? mask[off[4] + m * a.sMm + n * a.sMn] : 0.0f;
+        creg[t][i] = cond != nullptr ? cond[off[5] + m * a.sCm + n * a.sCn] : uint8_t{1};
+      }
     if (cond != nullptr) {
       keep = 0;
 #pragma unroll
-      for (int i = 0; i < kNpt; ++i) keep |= static_cast<uint32_t>(cond_v[i] != 0) << i;
+      for (int t = 0; t < KT; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) keep |= static_cast<uint32_t>(creg[t][i] != 0) << (4 * t + i);
     }
   }
-
-  // ---- scores -> LDS strip ------------------------------------------------------------------------------
-  // v_mfma_f32_16x16x4_f32: lane supplies A[m = lane % 16][k = lane / 16] and B[k = lane / 16][n = lane % 16] and
-  // receives D[m = 4 * (lane / 16) + i][n = lane % 16], i = 0..3.  The k index is permuted so that lane group g
-  // covers k = kk + 4 g + e in MFMA e: one 128-bit LDS read feeds four MFMAs.
-  const int d16 = (a.D + 15) / 16 * 16;
+  float vreg[KT][4][DT];
+  const float *vb = v + off[3];
 #pragma unroll
-  for (int c = 0; c < CHUNKS; ++c) {
-    if (c > 0) __syncthreads();  // kv free
-    store_stage(k_lanes_along_d, true);
-    if (c + 1 < CHUNKS) load_k(c + 1);
-    else load_v(0);
-    __syncthreads();
-    floatx4 s0 = {0.0f, 0.0f, 0.0f, 0.0f}, s1 = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int kk = 0; kk < d16; kk += 16) {
-      const int kb = kk + 4 * grp;
-      const floatx4 av = *reinterpret_cast<const floatx4 *>(qs + l16 * kLdQ + kb);
-      const float a4[4] = {av.x, av.y, av.z, av.w};
+  for (int t = 0; t < KT; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float *at = vb + min(key(t, 4 * grp + i), last_key) * a.sVn;
+      if constexpr (VEC) {
+        const Run<DT> x = *reinterpret_cast<const Run<DT> *>(at + column(0, l16));
+#pragma unroll
+        for (int j = 0; j < DT; ++j) vreg[t][i][j] = x.v[j];
+      } else {
+#pragma unroll
+        for (int j = 0; j < DT; ++j) vreg[t][i][j] = at[(FULL ? column(j, l16) : min(column(j, l16), a.D - 1)) * a.sVd];
+      }
+    }
+
+  // ---- scores ------------------------------------------------------------------------------------------------------
+  if constexpr (!FULL) {
+    // head columns past D: both operands are zero there
+#pragma unroll
+    for (int j = 0; j < DT; ++j)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[e], kv[(kb + e) * kLdK + wave * 32 + l16], s0, 0, 0, 0);
-        s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[e], kv[(kb + e) * kLdK + wave * 32 + 16 + l16], s1, 0, 0, 0);
+        const bool ok = 16 * j + 4 * grp + e < a.D;
+        qreg[j][e] = ok ? qreg[j][e] : 0.0f;
+#pragma unroll
+        for (int t = 0; t < KT; ++t) kreg[t][j][e] = ok ? kreg[t][j][e] : 0.0f;
       }
-    }
-    const float r0[4] = {s0.x, s0.y, s0.z, s0.w}, r1[4] = {s1.x, s1.y, s1.z, s1.w};
+  }
+  float s[KT][4];
+#pragma unroll
+  for (int t = 0; t < KT; ++t) {
+    floatx4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int j = 0; j < DT; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(kreg[t][j][e], qreg[j][e], acc, 0, 0, 0);
+    s[t][0] = acc.x, s[t][1] = acc.y, s[t][2] = acc.z, s[t][3] = acc.w;
+  }
+
+  // ---- scale, mask, condition; exponentials about the maximum of the wave's keys ---------------------------------
+  float mx = -__FLT_MAX__;
+#pragma unroll
+  for (int t = 0; t < KT; ++t)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      ps[(4 * grp + i) * kLdP + c * kKeys + wave * 32 + l16] = r0[i];
-      ps[(4 * grp + i) * kLdP + c * kKeys + wave * 32 + 16 + l16] = r1[i];
-    }
-  }
-  __syncthreads();  // the strip is complete, the last K^T chunk is consumed
-
-  // ---- scale, mask, condition, row softmax (unnormalised) ------------------------------------------------
-  {
-    float x[kNpt];
-#pragma unroll
-    for (int i = 0; i < kNpt; i += 4) {
-      const floatx4 t = *reinterpret_cast<const floatx4 *>(ps + rw_row * kLdP + rw_n0 + i);
-      x[i] = t.x, x[i + 1] = t.y, x[i + 2] = t.z, x[i + 3] = t.w;
-    }
-    float mx = -__FLT_MAX__;
-#pragma unroll
-    for (int i = 0; i < kNpt; ++i) {
-      float y = a.scale_is_divisor ? x[i] / a.scale : x[i] * a.scale;
-      if (mask != nullptr) y = y + mask_v[i];
-      if ((keep >> i & 1u) == 0) y = a.fill;
-      if (rw_n0 + i >= a.Skv) y = -__FLT_MAX__;
-      x[i] = y;
+      float y = a.scale_is_divisor ? s[t][i] / a.scale : s[t][i] * a.scale;
+      if (mask != nullptr) y = y + mreg[t][i];
+      if ((keep >> (4 * t + i) & 1u) == 0) y = a.fill;
+      if (key(t, 4 * grp + i) > last_key) y = -__FLT_MAX__;
+      s[t][i] = y;
       mx = fmaxf(mx, y);
     }
+  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+  float sum = 0.0f;
 #pragma unroll
-    for (int o = 8; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-    float sum = 0.0f;
-#pragma unroll
-    for (int i = 0; i < kNpt; ++i) {
-      x[i] = rw_n0 + i < a.Skv ? expf(x[i] - mx) : 0.0f;
-      sum += x[i];
-    }
-#pragma unroll
-    for (int o = 8; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
-#pragma unroll
-    for (int i = 0; i < kNpt; i += 4) {
-      *reinterpret_cast<floatx4 *>(ps + rw_row * kLdP + rw_n0 + i) = floatx4{x[i], x[i + 1], x[i + 2], x[i + 3]};
-    }
-    if (tid % 16 == 0) row_sum[rw_row] = sum;
-  }
-
-  // ---- out = (P . V) / row sum: wave w owns head columns [16 w, +16) --------------------------------------
-  floatx4 o = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-  for (int c = 0; c < CHUNKS; ++c) {
-    if (c > 0) __syncthreads();  // kv free
-    store_stage(v_lanes_along_d, false);  // V chunk -> LDS [key][d]
-    if (c + 1 < CHUNKS) load_v(c + 1);
-    __syncthreads();
-    if (wave * 16 < a.D) {
-#pragma unroll 4
-      for (int kk = 0; kk < kKeys; kk += 16) {
-        const int kb = kk + 4 * grp;
-        const floatx4 av = *reinterpret_cast<const floatx4 *>(ps + l16 * kLdP + c * kKeys + kb);
-        const float a4[4] = {av.x, av.y, av.z, av.w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          o = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[e], kv[(kb + e) * kLdV + wave * 16 + l16], o, 0, 0, 0);
-        }
-      }
-    }
-  }
-  {
-    const float r[4] = {o.x, o.y, o.z, o.w};
-    const int k = wave * 16 + l16;
+  for (int t = 0; t < KT; ++t)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int m = 4 * grp + i;
-      if (m0 + m < a.Sq && k < a.D) out[off[0] + (m0 + m) * a.sOm + k * a.sOd] = r[i] / row_sum[m];
+      s[t][i] = key(t, 4 * grp + i) <= last_key ? expf(s[t][i] - mx) : 0.0f;
+      sum += s[t][i];
+    }
+  sum += __shfl_xor(sum, 16, 64);
+  sum += __shfl_xor(sum, 32, 64);
+
+  // ---- the wave's context --------------------------------------------------------------------------------------------
+  floatx4 o[DT];
+#pragma unroll
+  for (int j = 0; j < DT; ++j) o[j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int t = 0; t < KT; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      // (keys past the last one repeat its row of V under a probability of zero; zero themselves, should it hold an infinity)
+      const bool ok = key(t, 4 * grp + i) <= last_key;
+#pragma unroll
+      for (int j = 0; j < DT; ++j) {
+        o[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ok ? vreg[t][i][j] : 0.0f, s[t][i], o[j], 0, 0, 0);
+      }
+    }
+
+  // ---- the waves' contexts meet in LDS --------------------------------------------------------------------------------
+#pragma unroll
+  for (int j = 0; j < DT; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ctx[(wave * kQ + l16) * kLd + column(j, 4 * grp + i)] = o[j][i];
+  if (grp == 0) {
+    stat[0][wave][l16] = mx;
+    stat[1][wave][l16] = sum;
+  }
+  __syncthreads();
+  for (int it = tid; it < kQ * DT * 4; it += 64 * NW) {
+    const int m = it / (4 * DT), k = it % (4 * DT) * 4;
+    float row_max = stat[0][0][m];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) row_max = fmaxf(row_max, stat[0][w][m]);
+    float row_sum = 0.0f;
+    floatx4 r = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float f = expf(stat[0][w][m] - row_max);
+      row_sum += f * stat[1][w][m];
+      const floatx4 x = *reinterpret_cast<const floatx4 *>(ctx + (w * kQ + m) * kLd + k);
+      r.x += f * x.x, r.y += f * x.y, r.z += f * x.z, r.w += f * x.w;
+    }
+    if (m0 + m >= a.Sq) continue;
+    float *at = out + off[0] + (m0 + m) * a.sOm;
+    const float res[4] = {r.x / row_sum, r.y / row_sum, r.z / row_sum, r.w / row_sum};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (FULL || k + e < a.D) at[(k + e) * a.sOd] = res[e];
     }
   }
 }
@@ -314,7 +266,7 @@ int fluidml_hip_attention(const fl_tensor *q, const fl_tensor *kt, const fl_tens
   a.Skv = static_cast<int32_t>(kt->shape[rank - 1]);
   if (kt->shape[rank - 2] != a.D || v->shape[rank - 2] != a.Skv || v->shape[rank - 1] != a.D ||
       out->shape[rank - 2] != a.Sq || out->shape[rank - 1] != a.D) return FL_ERR_SHAPE;
-  if (a.D > kMaxD || a.Skv > 2 * kKeys) return FL_ERR_UNSUPPORTED;
+  if (a.D > kMaxD || a.Skv > kMaxKeys) return FL_ERR_UNSUPPORTED;
   a.sQm = static_cast<int32_t>(q->strides[rank - 2]);
   a.sQd = static_cast<int32_t>(q->strides[rank - 1]);
   a.sKd = static_cast<int32_t>(kt->strides[rank - 2]);
@@ -367,24 +319,37 @@ int fluidml_hip_attention(const fl_tensor *q, const fl_tensor *kt, const fl_tens
   if (blocks > INT32_MAX) return FL_ERR_TOO_LARGE;
   if (blocks == 0 || a.D == 0) return FL_OK;
   if (a.Skv == 0) return FL_ERR_UNSUPPORTED;
-  const dim3 grid(static_cast<uint32_t>(blocks)), block(256);
+  const dim3 grid(static_cast<uint32_t>(blocks));
   float *o = static_cast<float *>(out->base);
   const float *qp = static_cast<const float *>(q->base), *kp = static_cast<const float *>(kt->base),
               *vp = static_cast<const float *>(v->base);
   const float *mp = add_mask ? static_cast<const float *>(add_mask->base) : nullptr;
   const uint8_t *cp = keep_cond ? static_cast<const uint8_t *>(keep_cond->base) : nullptr;
   auto mult4 = [](int64_t x) { return x % 4 == 0; };
-  bool vec = a.sQd == 1 && a.sKn == 1 && a.sVd == 1 && a.D % 4 == 0 && a.Skv % 4 == 0 && mult4(a.sQm) && mult4(a.sKd) &&
-             mult4(a.sVn) && reinterpret_cast<uintptr_t>(qp) % 16 == 0 && reinterpret_cast<uintptr_t>(kp) % 16 == 0 &&
-             reinterpret_cast<uintptr_t>(vp) % 16 == 0;
-  for (int i = 0; i < rank - 2; ++i) vec = vec && mult4(q->strides[i]) && mult4(kt->strides[i]) && mult4(v->strides[i]);
-  if (a.Skv <= kKeys) {
-    if (vec) FL_LAUNCH((AttentionKernel<1, true>), grid, block, 0, AsStream(stream), a, o, qp, kp, vp, mp, cp);
-    else FL_LAUNCH((AttentionKernel<1, false>), grid, block, 0, AsStream(stream), a, o, qp, kp, vp, mp, cp);
-  } else {
-    if (vec) FL_LAUNCH((AttentionKernel<2, true>), grid, block, 0, AsStream(stream), a, o, qp, kp, vp, mp, cp);
-    else FL_LAUNCH((AttentionKernel<2, false>), grid, block, 0, AsStream(stream), a, o, qp, kp, vp, mp, cp);
-  }
+  bool vec = a.sQd == 1 && a.D % 4 == 0 && mult4(a.sQm) && reinterpret_cast<uintptr_t>(qp) % 16 == 0;
+  for (int i = 0; i < rank - 2; ++i) vec = vec && mult4(q->strides[i]);
+  a.vec_q = vec ? 1 : 0;
+  const bool runs = a.sVd == 1;
+#define FL_ATTENTION_D(NW_, KT_, DT_)                                                                                           \
+  do {                                                                                                                          \
+    if (a.D == 16 * DT_ && runs) FL_LAUNCH((AttentionKernel<NW_, KT_, DT_, true, true>), grid, dim3(64 * NW_), 0, AsStream(stream), a, o, qp, kp, vp, mp, cp); \
+    else if (a.D == 16 * DT_) FL_LAUNCH((AttentionKernel<NW_, KT_, DT_, true, false>), grid, dim3(64 * NW_), 0, AsStream(stream), a, o, qp, kp, vp, mp, cp); \
+    else FL_LAUNCH((AttentionKernel<NW_, KT_, DT_, false, false>), grid, dim3(64 * NW_), 0, AsStream(stream), a, o, qp, kp, vp, mp, cp); \
+  } while (0)
+#define FL_ATTENTION(NW_, KT_)                      \
+  do {                                              \
+    if (a.D <= 16) FL_ATTENTION_D(NW_, KT_, 1);     \
+    else if (a.D <= 32) FL_ATTENTION_D(NW_, KT_, 2); \
+    else FL_ATTENTION_D(NW_, KT_, 4);               \
+  } while (0)
+  // enough waves that each has few keys (and its loads are in flight together), no more than have any (512 keys: 16 waves
+  // with two tiles each 23.8 us, 4 with eight 25.3, 8 with four 23.1)
+  if (a.Skv <= 64) FL_ATTENTION(4, 1);
+  else if (a.Skv <= 128) FL_ATTENTION(4, 2);
+  else if (a.Skv <= 256) FL_ATTENTION(8, 2);
+  else FL_ATTENTION(8, 4);
+#undef FL_ATTENTION
+#undef FL_ATTENTION_D
   return LaunchStatus();
 }
 

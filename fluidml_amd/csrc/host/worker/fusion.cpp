@@ -2435,7 +2435,7 @@ class Scheduler {
       return std::nullopt;  // broadcast batch dims
     }
     const int64_t head = qs[rank - 1], keys = shape[rank - 1];
-    if (head > 64 || keys > 256 || head == 0 || keys == 0) return std::nullopt;
+    if (head > 64 || keys > 512 || head == 0 || keys == 0) return std::nullopt;
     Launch l;
     l.kind = Launch::Kind::Attention;
     l.a = scores.in0;
