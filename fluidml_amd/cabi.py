@@ -91,8 +91,8 @@ SIGNATURES = {
     "fluidml_hip_memcpy_d2d": [_vp, _vp, _sz, _vp],
     "fluidml_hip_host_alloc": [_sz, _P(_vp)],
     "fluidml_hip_host_free": [_vp],
-    "fluidml_hip_transfer_in": [_i32, _P(_vp), _P(_vp), _P(_sz), _sz, _vp, _vp],
-    "fluidml_hip_transfer_out": [_i32, _P(_vp), _P(_vp), _P(_sz), _sz, _vp, _vp, _vp, _u32, _vp],
+    "fluidml_hip_transfer_in": [_i32, _P(_vp), _P(_vp), _P(_sz), _vp, _vp],
+    "fluidml_hip_transfer_out": [_i32, _P(_vp), _P(_vp), _P(_sz), _sz, _vp, _vp, _vp, _vp, _u32, _vp],
     "fluidml_hip_clock_khz": [_P(ctypes.c_int)],
     "fluidml_hip_stream_query": [_vp, _P(ctypes.c_int)],
     "fluidml_hip_time_kernels": [_vp, _vp],

@@ -30,12 +30,10 @@ size_t Padded(size_t bytes) { return (bytes + kAlign - 1) / kAlign * kAlign; }
 // bypass the caches (51.5 MB: 1.65 ms with plain stores, 1.1 ms without, on one core).
 constexpr size_t kLargeBytes = size_t{1} << 20;
 constexpr size_t kSmallSlice = 16 << 10, kLargeSlice = 512 << 10;
-// Slice of the way out: a block's round of loads at least (the host starts early), and as large as leaves about a
-// hundred of them (four threads that poll 786 flags while the link fills the memory around them: 1.52 ms for 51.5 MB;
-// 99 flags and eight threads 1.15, the link alone 0.95).
+// Slice of the way out, whole pieces of 16 KiB: as large as leaves about two hundred of them.
 size_t OutSlice(size_t bytes) {
   size_t slice = kSmallSlice;
-  while (slice < kLargeSlice && bytes / (2 * slice) >= 96) slice *= 2;
+  while (slice < kLargeSlice && bytes / (2 * slice) >= 192) slice *= 2;
   return slice;
 }
 // The way in is staged and launched piece by piece: the first one small, so that the link starts early.
@@ -264,6 +262,9 @@ Transfer::Transfer(std::vector<Slot> &&inputs, std::vector<Slot> &&outputs) {
     void *p = nullptr;
     Check(fluidml_hip_arena_create(sizeof(uint64_t), &p), "allocating the transfer clock");  // zero-filled
     clock_ = static_cast<uint64_t *>(p);
+    Check(fluidml_hip_arena_create((flags + outputs_.size() + 1) * sizeof(uint32_t), &p), "allocating the transfer counters");
+    counters_ = static_cast<uint32_t *>(p);
+    Check(fluidml_hip_stream_synchronize(nullptr), "waiting for the cleared counters");
     Check(fluidml_hip_host_alloc(in_bytes_, &p), "allocating pinned memory for the inputs");
     in_ = static_cast<char *>(p);
     Check(fluidml_hip_host_alloc(out_bytes_, &p), "allocating pinned memory for the outputs");
@@ -285,6 +286,7 @@ void Transfer::Release() {
   fluidml_hip_host_free(out_);
   fluidml_hip_host_free(mailbox_);
   fluidml_hip_arena_destroy(clock_);
+  fluidml_hip_arena_destroy(counters_);
 }
 
 void Transfer::In(const std::vector<const void *> &host, void *stream) {
@@ -321,7 +323,7 @@ void Transfer::In(const std::vector<const void *> &host, void *stream) {
         if (!job.One()) _mm_pause();
       }
     }
-    rc = fluidml_hip_transfer_in(n, dst, src, bytes, kSmallSlice, clock_, stream);
+    rc = fluidml_hip_transfer_in(n, dst, src, bytes, clock_, stream);
     launched = end;
     piece = kInPiece;
   } while (rc == 0 && launched < slices.size());
@@ -338,10 +340,10 @@ double Transfer::Out(const std::vector<void *> &host, void *stream) {
   void *dst[FL_MAX_TRANSFER_SEGMENTS];
   const void *src[FL_MAX_TRANSFER_SEGMENTS];
   size_t bytes[FL_MAX_TRANSFER_SEGMENTS];
-  size_t at = 0, flag = 0;
+  size_t at = 0, flag = 0, launches = 0;
   do {
     int32_t n = 0;
-    const size_t first_flag = flag;
+    const size_t first_flag = flag, first_counter = flag + launches++;  // (each launch has a counter of its own besides)
     for (; at < outputs_.size() && n < FL_MAX_TRANSFER_SEGMENTS; ++at) {
       const Slot &s = outputs_[at];
       if (s.bytes == 0) continue;
@@ -351,7 +353,7 @@ double Transfer::Out(const std::vector<void *> &host, void *stream) {
       flag += (s.bytes + out_slice_ - 1) / out_slice_;
     }
     Check(fluidml_hip_transfer_out(n, dst, src, bytes, out_slice_, clock_, first_flag == 0 ? elapsed : nullptr, flags + first_flag,
-                                   value_, stream),
+                                   counters_ + first_counter, value_, stream),
           "copying the outputs to the host");
   } while (at < outputs_.size());
   Helpers &helpers = Helpers::Get();

@@ -42,7 +42,8 @@ class Transfer {
   char *in_ = nullptr, *out_ = nullptr;
   // host: kFlagBase bytes with the elapsed ticks, then one flag per outbound slice
   char *mailbox_ = nullptr;
-  uint64_t *clock_ = nullptr;  // device
+  uint64_t *clock_ = nullptr;     // device
+  uint32_t *counters_ = nullptr;  // device: one per outbound slice and one per outbound launch
   uint32_t value_ = 0;
   double ns_per_tick_ = 10.0;
 };

@@ -215,16 +215,17 @@ int fluidml_hip_memcpy_h2d(void *device, const void *host, size_t bytes, void *s
 int fluidml_hip_memcpy_d2h(void *host, const void *device, size_t bytes, void *stream);
 int fluidml_hip_memcpy_d2d(void *dst, const void *src, size_t bytes, void *stream);
 /* Arguments of a run through pinned host memory (fluidml_hip_host_alloc).  Both calls launch one kernel that copies
- * up to FL_MAX_TRANSFER_SEGMENTS ranges in slices of `slice_bytes` (a multiple of 16); all addresses are 16-byte
- * aligned and both sides of a range are readable / writable up to the next multiple of 16 bytes.  `clock` is a device
+ * up to FL_MAX_TRANSFER_SEGMENTS ranges, on the way out in slices of `slice_bytes` (a multiple of 16384) one after the
+ * other; all addresses are 16-byte aligned and both sides of a range are readable / writable up to the next multiple of 16
+ * bytes.  `counters`: one device word per slice and one more, zero before their first use.  `clock` is a device
  * word, zero before its first use.  transfer_out stores `value` in flags[i] (host memory) once slice i is there (slices
  * are counted through the ranges in order; at least one flag is written) and, with `elapsed` (host memory), the ticks of
  * fluidml_hip_clock_khz between the end of the latest transfer_in and its own start. */
 #define FL_MAX_TRANSFER_SEGMENTS 8
 int fluidml_hip_host_alloc(size_t bytes, void **host);
 int fluidml_hip_host_free(void *host);
-int fluidml_hip_transfer_in(int32_t n, void *const *device, const void *const *host, const size_t *bytes, size_t slice_bytes, uint64_t *clock, void *stream);
-int fluidml_hip_transfer_out(int32_t n, void *const *host, const void *const *device, const size_t *bytes, size_t slice_bytes, uint64_t *clock, uint64_t *elapsed, uint32_t *flags, uint32_t value, void *stream);
+int fluidml_hip_transfer_in(int32_t n, void *const *device, const void *const *host, const size_t *bytes, uint64_t *clock, void *stream);
+int fluidml_hip_transfer_out(int32_t n, void *const *host, const void *const *device, const size_t *bytes, size_t slice_bytes, uint64_t *clock, uint64_t *elapsed, uint32_t *flags, uint32_t *counters, uint32_t value, void *stream);
 int fluidml_hip_clock_khz(int *khz);
 /* *idle = 1 once everything issued on `stream` is done; never waits. */
 int fluidml_hip_stream_query(void *stream, int *idle);
