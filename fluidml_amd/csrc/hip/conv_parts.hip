@@ -435,7 +435,8 @@ int fluidml_hip_conv3x3_packed_chain(const fl_tensor *in, const fl_tensor *weigh
     const int64_t before = pads ? pads[d] : 0, after = pads ? pads[d + 2] : 0;
     if (before < 0 || after < 0) return FL_ERR_ATTR;
     if (before > 0x3fffffff) return FL_ERR_TOO_LARGE;
-    if (out->shape[2 + d] + 2 > in->shape[2 + d] + before + after) return FL_ERR_SHAPE;
+    // (the whole output and nothing else: a smaller one would be a convolution with other strides or dilations, or a crop)
+    if (out->shape[2 + d] != in->shape[2 + d] + before + after - 2) return FL_ERR_SHAPE;
   }
   if (Numel(in) > 0x7fffffff || Numel(out) > 0x7fffffff) return FL_ERR_UNSUPPORTED;
   for (int d = 0; d < 4; ++d) {

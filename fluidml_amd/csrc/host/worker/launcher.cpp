@@ -288,6 +288,22 @@ void LaunchPlan::FoldNorms() {
   }
 }
 
+namespace {
+// Whether a convolution step that reads its weights through `weights` is one the packed form is for.  Asked of every launch
+// for itself, when the weights are packed and when it is issued: another reader of the same constant may have other strides
+// or dilations, read it through a view, or be no convolution at all.
+bool IsPackableConv(const Step &step, const Operand &weights) {
+  const flow::OpKind kind = step.node->GetKind();
+  if (kind != flow::OpKind::ConvWithPadding && kind != flow::OpKind::ConvWithoutPadding) return false;
+  if (weights.space != Operand::Space::Constant || weights.viewed) return false;
+  const flow::Attrs &at = step.node->GetAttrs();
+  const std::vector<int64_t> &shape = weights.meta.GetShape();
+  const std::vector<int64_t> ones{1, 1};
+  // (fewer than sixteen channels would mostly multiply padding)
+  return at.group == 1 && at.strides == ones && at.dilations == ones && shape.size() == 4 && shape[1] >= 16;
+}
+}  // namespace
+
 // Environment FLUIDML_CONV_PACKED=0 (read at every compile) leaves all weights as they stand.
 void LaunchPlan::PackConvWeights() {
   const char *env = std::getenv("FLUIDML_CONV_PACKED");
@@ -296,20 +312,13 @@ void LaunchPlan::PackConvWeights() {
   if (flags_ != 0) return;  // (literal-reference semantics)
   for (const Launch &l : GetSchedule()) {
     const Step &step = steps_[l.kind == Launch::Kind::ConvChain ? l.owner : l.members.front()];
-    const flow::OpKind kind = step.node->GetKind();
-    if (kind != flow::OpKind::ConvWithPadding && kind != flow::OpKind::ConvWithoutPadding) continue;
     if (l.kind == Launch::Kind::ConvChain ? l.has_gate || l.has_skip || l.has_out2 : l.kind != Launch::Kind::Step) continue;
     const Operand &op = l.kind == Launch::Kind::ConvChain || l.rewired ? l.b : step.in1;
-    if (op.space != Operand::Space::Constant || op.viewed || packed_.count(op.name)) continue;
-    const flow::Attrs &at = step.node->GetAttrs();
-    const std::vector<int64_t> &shape = op.meta.GetShape();
-    const std::vector<int64_t> ones{1, 1};
-    // (fewer than sixteen channels would mostly multiply padding)
-    if (at.group != 1 || at.strides != ones || at.dilations != ones || shape.size() != 4 || shape[1] < 16) continue;
+    if (!IsPackableConv(step, op) || packed_.count(op.name)) continue;
     const kernel::TensorView w = ViewOf(Resolve(op), op);
     PackedSlot slot;
     // bf16 contractions need one part; channels that do not come in sixteens stay fp32 there
-    slot.parts = bf16_ && shape[1] % 16 == 0 ? 1 : 3;
+    slot.parts = bf16_ && op.meta.GetShape()[1] % 16 == 0 ? 1 : 3;
     const int rc = fluidml_hip_conv3x3_packed_bytes(&w.t, slot.parts, &slot.bytes);
     if (rc == FL_ERR_UNSUPPORTED) continue;
     Check(rc, "sizing packed convolution weights");
@@ -360,7 +369,7 @@ void LaunchPlan::PackContractionWeights() {
 
 int LaunchPlan::IssuePackedConv(const Step &step, const Operand &weights, const fl_tensor &in, const fl_tensor &out,
                                 const fl_ew_program *chain, void *stream) const {
-  const auto it = weights.space == Operand::Space::Constant ? packed_.find(weights.name) : packed_.end();
+  const auto it = IsPackableConv(step, weights) ? packed_.find(weights.name) : packed_.end();
   if (it == packed_.end()) return FL_ERR_UNSUPPORTED;
   const kernel::TensorView w = ViewOf(Resolve(weights), weights);
   const kernel::DeviceConstant *bias = step.kernel->GetConstant(0);

@@ -1,0 +1,27 @@
+"""Arguments that the C entry points refuse before anything is launched (no GPU: the addresses are never read)."""
+import ctypes
+
+import pytest
+
+from fluidml_amd import cabi
+
+FL_ERR_SHAPE = -3
+HERE = ctypes.create_string_buffer(4096)
+
+
+def tensor(*shape):
+    base = (ctypes.addressof(HERE) + 255) // 256 * 256
+    return cabi.make_tensor(base, cabi.FL_FLOAT32, shape)
+
+
+@pytest.mark.parametrize("size,pads,out", [
+    ((13, 15), (1, 1, 1, 1), (7, 8)),    # what stride 2 leaves
+    ((13, 15), (2, 2, 2, 2), (13, 15)),  # what dilation 2 leaves
+    ((13, 15), (0, 0, 0, 0), (11, 12)),
+    ((13, 15), (0, 0, 0, 0), (12, 13)),
+])
+def test_packed_convolution_has_one_output_size(size, pads, out):
+    x, w, o = tensor(1, 32, *size), tensor(32, 32, 3, 3), tensor(1, 32, *out)
+    rc = cabi.lib.fluidml_hip_conv3x3_packed_chain(ctypes.byref(x), ctypes.byref(w), x.base, 3, None, ctypes.byref(o),
+                                                   cabi.i64_array(pads), None, 0, None)
+    assert rc == FL_ERR_SHAPE

@@ -1,10 +1,12 @@
 """3x3 convolutions against packed weights (fluidml_hip_conv3x3_packed_chain) on the GPU, at the edges of its tiles,
 channel chunks, filter groups and splits, against the oracle; and the values its bf16 parts cannot carry."""
 import ctypes
+import os
 
 import numpy as np
 import pytest
 
+from oracle import graph_runner
 from oracle import kernels as ok
 from tests.util import DeviceView, assert_close, some_layouts
 
@@ -107,3 +109,38 @@ def test_packed_conv_is_as_exact_as_fp32(device):
         for kw in range(3):
             want[0] += np.einsum("fc,chw->fhw", w[:, :, kh, kw].astype(np.float64), padded[0, :, kh:kh + 14, kw:kw + 14])
     assert np.linalg.norm(got - want) / np.linalg.norm(want) < 3e-7  # (fp32 sums of 4608 products: 4e-7 .. 1.2e-6)
+
+
+@pytest.mark.parametrize("fuse", ["1", "0"])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_weights_that_other_operations_read_too(device, tmp_path, monkeypatch, fuse, bf16):
+    """One initializer read by the convolution the packed form is for, by ones with another stride or dilation, by a
+    convolution of another tensor and by an Add."""
+    from fluidml_amd import fluidml, models
+
+    monkeypatch.setenv("FLUIDML_FUSE", fuse)
+    net = models.Net("shared", 3)
+    w = net.normal((32, 32, 3, 3), std=0.06)
+    x = net.input("x", np.float32, (1, 32, 13, 15))
+    z = net.input("z", np.float32, (32, 32, 3, 3))
+    y = net.input("y", np.float32, (2, 32, 9, 20))
+    net.output(net.relu(net.conv(x, w, None, [1, 1], [1, 1, 1, 1])))
+    net.output(net.relu(net.conv(x, w, None, [2, 2], [1, 1, 1, 1])))
+    net.output(net.relu(net.conv(x, w, None, [1, 1], [2, 2, 2, 2], dilations=[2, 2])))
+    net.output(net.conv(x, w, None, [2, 1], [0, 0, 0, 0]))
+    net.output(net.relu(net.conv(y, w, None, [1, 1], [0, 0, 0, 0])))
+    net.output(net.add(z, w))
+    rng = np.random.default_rng(4)
+    feeds = {v.name: rng.standard_normal(v.shape, np.float32) for v in net.inputs}
+    want = graph_runner.run_graph(net, feeds)
+    ex = fluidml.Executor.make_plain_greedy("shared")
+    ex.context().set_bf16(bf16)
+    ex.compile(net.save(os.path.join(tmp_path, "shared.onnx")))
+    outs = {v.name: np.full(v.shape, 9.0, np.float32) for v in net.outputs}
+    print("[case]", fuse, bf16, flush=True)
+    ex.invoke({**feeds, **outs})
+    for i, v in enumerate(net.outputs):
+        if bf16 and i < 5:  # 288 products of operands rounded to 8 bits: 2^-9 each way, results about 1.7
+            assert np.abs(outs[v.name] - want[v.name]).max() < 0.06, i
+        else:
+            assert_close(outs[v.name], want[v.name], what=f"output {i}")
