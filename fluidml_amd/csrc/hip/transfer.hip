@@ -37,17 +37,22 @@ struct TransferArgs {
   Segment segments[FL_MAX_TRANSFER_SEGMENTS];
 };
 
+// The time of the replays, for the host.  By the block that takes piece 0, before it counts that piece: the flag of the
+// first slice says then that it has been written (a block that only carried the first index could start after all others
+// had raised every flag, and the host would read the previous run's time).
+__device__ __forceinline__ void LeaveElapsed(const TransferArgs &args) {
+  if (threadIdx.x != 0 || args.elapsed == nullptr) return;
+  const uint64_t now = wall_clock64();
+  const uint64_t since = *args.clock;
+  *args.clock = 0;
+  *args.elapsed = since != 0 && now > since ? now - since : 0;
+}
+
 // Bound by the link (about 55 GB/s each way: 51.5 MB take 0.93 ms, the copy engine needs 0.91) and, for the few
 // kilobytes of a text request, by the launch (an asynchronous copy of pageable memory costs 13 us in and 21 us out per
 // argument and a stream wait 11 us; one launch plus a polled flag 6 us).  Four 16-byte loads are in flight per lane.
 template <bool OUTBOUND>
 __global__ __launch_bounds__(kThreads) void TransferKernel(TransferArgs args) {
-  if (OUTBOUND && blockIdx.x == 0 && threadIdx.x == 0 && args.elapsed != nullptr) {
-    const uint64_t now = wall_clock64();
-    const uint64_t since = *args.clock;
-    *args.clock = 0;
-    *args.elapsed = since != 0 && now > since ? now - since : 0;
-  }
   __shared__ uint32_t taken;
   const bool in_turn = OUTBOUND && args.n_pieces > gridDim.x;
   uint32_t s = 0, piece = blockIdx.x;
@@ -62,6 +67,7 @@ __global__ __launch_bounds__(kThreads) void TransferKernel(TransferArgs args) {
       piece = taken;
     }
     if (piece >= args.n_pieces) break;
+    if (OUTBOUND && piece == 0) LeaveElapsed(args);
     while (s + 1 < args.n_segments && piece >= args.segments[s + 1].first_piece) ++s;
     const Segment g = args.segments[s];
     const uint32_t local = piece - g.first_piece, i = local * kPiece16 + threadIdx.x;
@@ -92,7 +98,9 @@ __global__ __launch_bounds__(kThreads) void TransferKernel(TransferArgs args) {
     if (!in_turn) break;  // (a block per piece)
   }
   if (OUTBOUND) {
-    if (args.n_pieces == 0 && threadIdx.x == 0) __hip_atomic_store(args.flags, args.value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (args.n_pieces != 0) return;
+    LeaveElapsed(args);  // (one block, nothing but the flag)
+    if (threadIdx.x == 0) __hip_atomic_store(args.flags, args.value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     return;
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");

@@ -32,3 +32,56 @@ def test_arguments_arrive(tmp_path, sizes):
         assert ex.invoke({**args, **outs}) >= 0
         for i, v in enumerate(net.outputs):
             np.testing.assert_array_equal(outs[v.name], np.maximum(args[f"x{i}"], 0))
+
+
+@pytest.mark.parametrize("pieces", [0, 1, 64, 65, 1000])  # (64 blocks: from 65 pieces on they take them in turn)
+def test_elapsed_belongs_to_the_run_whose_flags_are_up(device, pieces):
+    """The time that a transfer_out leaves is there once all flags are, and is that of its own run: runs of nothing
+    and of a few milliseconds in turn."""
+    import ctypes
+
+    import torch
+
+    from fluidml_amd import cabi
+
+    def alloc(name, size):
+        p = ctypes.c_void_p()
+        cabi.call(name, size, ctypes.byref(p))
+        return p.value
+
+    size, slice_bytes = pieces * 16384, 32768
+    slices = max(1, -(-size // slice_bytes))
+    src, clock, counters = (alloc("arena_create", max(n, 1)) for n in (size, 8, 4 * (slices + 1)))
+    dst, mailbox = (alloc("host_alloc", n) for n in (size, 64 + 4 * slices))
+    ctypes.memset(mailbox, 0, 64 + 4 * slices)
+    flags = np.ctypeslib.as_array((ctypes.c_uint32 * slices).from_address(mailbox + 64))
+    elapsed = ctypes.c_uint64.from_address(mailbox)
+    khz = ctypes.c_int()
+    cabi.call("clock_khz", ctypes.byref(khz))
+    a = torch.randn(4096, 4096, device=device)
+    out = torch.empty_like(a)
+    torch.mm(a, a, out=out)
+    torch.cuda.synchronize()
+    stream = torch.cuda.current_stream().cuda_stream
+    n = 1 if pieces else 0
+    lists = [(ctypes.c_void_p * 1)(dst), (ctypes.c_void_p * 1)(src), (ctypes.c_size_t * 1)(size)]
+    print("[case]", pieces, flush=True)
+    for turn in range(1, 13):
+        begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        cabi.call("transfer_in", 0, None, None, None, clock, stream)
+        begin.record()
+        for _ in range(8 if turn % 2 else 0):
+            torch.mm(a, a, out=out)
+        end.record()
+        cabi.call("transfer_out", n, *lists, slice_bytes, clock, mailbox, mailbox + 64, counters, turn, stream)
+        while not (flags == turn).all():
+            if torch.cuda.current_stream().query():
+                assert (flags == turn).all(), "the stream is idle but a flag is missing"
+        ms = elapsed.value / khz.value
+        torch.cuda.synchronize()
+        want = begin.elapsed_time(end)
+        assert want - 0.05 < ms < want + 0.5, (turn, ms, want)
+    for p in (src, clock, counters):
+        cabi.call("arena_destroy", p)
+    for p in (dst, mailbox):
+        cabi.call("host_free", p)
