@@ -356,9 +356,11 @@ double Transfer::Out(const std::vector<void *> &host, void *stream) {
                                    counters_ + first_counter, value_, stream),
           "copying the outputs to the host");
   } while (at < outputs_.size());
+  job.Wait(0, true);  // (also without an output: the launch leaves one flag)
+  // Not before: what is queued in front of the launch may take any time, and they would poll through all of it.  They wake
+  // while the caller takes over the first slices.
   Helpers &helpers = Helpers::Get();
   const bool helped = large && helpers.Call(&job);
-  job.Wait(0, true);  // (also without an output: the launch leaves one flag)
   job.Work(true);
   if (helped) {
     uint32_t spins = 0;
