@@ -73,6 +73,7 @@ __global__ __launch_bounds__(kThreads, 2) void ConvPartsKernel(float *out, const
   constexpr int kItems = 2 * kPix;  // (channel half, pixel): eight channels each
   constexpr int kPer = (kItems + kThreads - 1) / kThreads;
   __shared__ u32x4 lds[2 * PARTS * kItems];
+  __shared__ uint32_t tiny_inputs;  // (BadSum)
   const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
   const int lrow = lane % 32, half = lane / 32;
   const int wf = wave % WF, wp = wave / WF;
@@ -110,6 +111,8 @@ __global__ __launch_bounds__(kThreads, 2) void ConvPartsKernel(float *out, const
     x_at[t] = x_ok[t] ? 4u * (ih * p.sXh + iw * p.sXw + (RAGGED ? 0 : 8 * h * p.sXc)) : 0u;
   }
   float xr[kPer][8];
+  uint32_t tiny_key = 0xffffffffu;
+  if (PARTS == 3 && tid == 0) tiny_inputs = 0;
   auto load_patch = [&](int c) {
 #pragma unroll
     for (int t = 0; t < kPer; ++t) {
@@ -140,6 +143,7 @@ __global__ __launch_bounds__(kThreads, 2) void ConvPartsKernel(float *out, const
           const bool ok = x_ok[t] && (!RAGGED || c * kChunk + 8 * (i / kPix) + e < p.C);
           x[e] = ok ? xr[t][e] : 0.0f;
         }
+        if constexpr (PARTS == 3) tiny_key = TinyKey(tiny_key, x);
         u32x4 parts[PARTS];
         SplitParts<PARTS>(x, parts);
 #pragma unroll
@@ -198,6 +202,9 @@ __global__ __launch_bounds__(kThreads, 2) void ConvPartsKernel(float *out, const
   }
 
   if constexpr (PARTS == 3) {
+    if (tiny_key < kTinyKey) tiny_inputs = 1;
+    __syncthreads();
+    const bool tiny = tiny_inputs != 0;
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
@@ -206,7 +213,7 @@ __global__ __launch_bounds__(kThreads, 2) void ConvPartsKernel(float *out, const
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) bad |= BadSum(acc[j][e]);
+      for (int e = 0; e < 16; ++e) bad |= BadSum(acc[j][e], tiny);
     if (__any(bad)) {
       // the same channels once more with the fp32 instruction, operands straight from memory
 #pragma unroll
@@ -399,6 +406,7 @@ int fluidml_hip_conv3x3_pack(const fl_tensor *weights, int32_t parts, void *pack
   size_t bytes = 0;
   FL_CHECK(fluidml_hip_conv3x3_packed_bytes(weights, parts, &bytes));
   if (!IsAligned(packed, 16)) return FL_ERR_ATTR;
+  if (parts == 3) FL_CHECK(PartsCanCarry(weights, weights->shape[1] * 9, AsStream(stream)));
   const int F = static_cast<int>(weights->shape[0]), C = static_cast<int>(weights->shape[1]);
   const int chunks = static_cast<int>(Ceil(C, kChunk));
   const uint32_t items = static_cast<uint32_t>(Ceil(F, 32) * chunks * 9 * 64);

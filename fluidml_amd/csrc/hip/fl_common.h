@@ -81,6 +81,10 @@ constexpr size_t kWorkspaceTileFloats = 1024;
 // The stream's workspace, created on first use.  nullptr when it does not exist yet and cannot be created
 // now (the stream is being captured into a graph) or the allocation fails; callers then do without.
 StreamWorkspace *GetStreamWorkspace(hipStream_t stream);  // runtime.hip
+
+// Whether weights that sums of `terms` products read can stand as three bf16 parts (see below): FL_OK or
+// FL_ERR_UNSUPPORTED.  Waits for the stream.  matmul_parts.hip
+int PartsCanCarry(const fl_tensor *weights, int64_t terms, hipStream_t stream);
 void DropStreamWorkspace(hipStream_t stream);
 // Device address of the current device's fixed split-K scratch (fluidml_hip_matmul_no_alloc), looked up on
 // the first call per device; `ptr` may be null.  matmul.hip
@@ -122,9 +126,13 @@ __host__ __device__ __forceinline__ void StaticFor(F &&body) {
 // over twenty powers of ten the same to within the run of the draw.  The six
 // v_mfma_f32_32x32x16_bf16 take 192 cycles per 16 values of k, the eight fp32 instructions 512; measured with operands
 // in registers on the whole chip 287 against 130-136 TFLOP/s.
-// What the parts cannot carry (an infinity minus itself is no number; a result so small that parts of its operands
-// may have been denormal) shows in the sum: BadSum tells, and the kernels then multiply that wave's tile again with
-// the fp32 instruction.
+// What the parts cannot carry shows in the sum (an infinity minus itself is no number; a result so small that parts of its
+// operands may have been denormal): BadSum tells, and the kernels then multiply that wave's tile again with the fp32
+// instruction.  An exact zero is taken for one only where the workgroup has staged no activation that is smaller than
+// 2^-40 and not zero (TinyKey): products of such values may have vanished, which the fp32 instruction would keep as
+// denormal numbers.  The weights are looked at when they are packed (PartsCanCarry): zero or at least 2^-60, so that
+// their parts are exact and products with activations from 2^-40 on stay normal, and the sums of their magnitudes at most
+// 2^20, so that the 2^-126 a denormal part may lose stays below the rounding of a result of 2^-80.
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -163,10 +171,21 @@ __device__ __forceinline__ void MfmaParts(const u32x4 (&a)[PARTS], const u32x4 (
   mul(0, 0, acc);
 }
 
-// a sum that is not finite, or neither zero nor at least 2^-80
-__device__ __forceinline__ bool BadSum(float v) {
+// a sum that is not finite, or neither zero nor at least 2^-80; with `tiny` also zero
+__device__ __forceinline__ bool BadSum(float v, bool tiny) {
   const uint32_t bits = __builtin_bit_cast(uint32_t, v) & 0x7fffffffu;
-  return bits != 0 && bits - 0x17800000u >= 0x7f800000u - 0x17800000u;
+  return bits == 0 ? tiny : bits - 0x17800000u >= 0x7f800000u - 0x17800000u;
+}
+
+// The smallest magnitude other than zero, as twice its bits minus one (zero wraps to the largest); below kTinyKey: below 2^-40
+constexpr uint32_t kTinyKey = 2 * 0x2b800000u - 1;
+__device__ __forceinline__ uint32_t TinyKey(uint32_t seen, const float (&x)[8]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t a = (__builtin_bit_cast(uint32_t, x[2 * i]) << 1) - 1, b = (__builtin_bit_cast(uint32_t, x[2 * i + 1]) << 1) - 1;
+    seen = min(seen, min(a, b));
+  }
+  return seen;
 }
 
 // Interpreter of fl_ew_program, shared by the elementwise-chain kernel and the contraction epilogues.

@@ -49,8 +49,9 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
   constexpr int kRed = KS > 1 ? TM * kWaves * 256 : 0;   // 16-byte places of the K slices' partial tiles
   constexpr int kLds = 2 * kStage > kRed ? 2 * kStage : kRed;
   constexpr bool NORM = EXTRA == 1;
-  __shared__ u32x4 lds[kLds + (NORM ? BM / 2 : 0)];
+  __shared__ u32x4 lds[kLds + (NORM ? BM / 2 : 0) + (PARTS == 3 ? 1 : 0)];
   float *const ln_rows = reinterpret_cast<float *>(lds + kLds);  // mean, then 1 / sqrt(var + eps), per row
+  uint32_t *const tiny_inputs = reinterpret_cast<uint32_t *>(lds + kLds + (NORM ? BM / 2 : 0));  // (BadSum; three parts)
 
   float *C = C_;
   const float *B = B_;
@@ -124,6 +125,8 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
       for (int s = 0; s < PARTS; ++s) br[S][u][s] = *reinterpret_cast<const u32x4 *>(from + s * 1024 + lane * 16u);
     }
   };
+  uint32_t tiny_key = 0xffffffffu;
+  if (PARTS == 3 && tid == 0) *tiny_inputs = 0;
   // item t of chunk c: its parts, into LDS
   auto store_item = [&](int c, int buf, auto set_c, int t) {
     constexpr int S = decltype(set_c)::value;
@@ -131,6 +134,7 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
     const floatx4 lo = ar[S][t][0], hi = ar[S][t][1];
     const float x[8] = {live ? lo.x : 0.0f, live ? lo.y : 0.0f, live ? lo.z : 0.0f, live ? lo.w : 0.0f,
                         live ? hi.x : 0.0f, live ? hi.y : 0.0f, live ? hi.z : 0.0f, live ? hi.w : 0.0f};
+    if constexpr (PARTS == 3) tiny_key = TinyKey(tiny_key, x);
     u32x4 parts[PARTS];
     SplitParts<PARTS>(x, parts);
 #pragma unroll
@@ -270,13 +274,16 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
   });
 
   if constexpr (PARTS == 3) {
+    if (tiny_key < kTinyKey) *tiny_inputs = 1;
+    __syncthreads();
+    const bool tiny = *tiny_inputs != 0;
     bool bad = false;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         acc[i][e] += low[i][e];
-        bad |= BadSum(acc[i][e]);
+        bad |= BadSum(acc[i][e], tiny);
       }
     if (__any(bad)) {
       // this wave's steps once more with the fp32 instruction, operands straight from memory
@@ -452,6 +459,36 @@ __global__ __launch_bounds__(kPackThreads) void MatmulPackKernel(u32x4 *__restri
   for (int s = 0; s < PARTS; ++s) packed[(block * PARTS + s) * 64 + lane] = parts[s];
 }
 
+// range[0]: the smallest magnitude but zero, as TinyKey has it; range[1]: the bits of the largest finite one.
+struct RangeArgs {
+  uint32_t n;
+  int32_t rank;
+  FastDiv shape[4];
+  int32_t strides[4];
+};
+__global__ __launch_bounds__(kPackThreads) void WeightRangeKernel(uint32_t *range, const float *__restrict__ w, RangeArgs a) {
+  uint32_t low = 0xffffffffu, high = 0;
+  for (uint32_t i = blockIdx.x * kPackThreads + threadIdx.x; i < a.n; i += gridDim.x * kPackThreads) {
+    uint32_t rem = i;
+    int32_t at = 0;
+    for (int d = a.rank - 1; d >= 0; --d) {
+      uint32_t q, r;
+      a.shape[d].DivMod(rem, q, r);
+      at += static_cast<int32_t>(r) * a.strides[d];
+      rem = q;
+    }
+    const uint32_t bits = __builtin_bit_cast(uint32_t, w[at]) & 0x7fffffffu;
+    low = min(low, 2 * bits - 1);
+    if (bits < 0x7f800000u) high = max(high, bits);
+  }
+  low = WaveReduce(low, [](uint32_t x, uint32_t y) { return min(x, y); });
+  high = WaveReduce(high, [](uint32_t x, uint32_t y) { return max(x, y); });
+  if (threadIdx.x % kWave == 0) {
+    atomicMin(range, low);
+    atomicMax(range + 1, high);
+  }
+}
+
 // ---- which weights have a packed form -----------------------------------------------------------------------------
 struct PackedWeights {
   void *packed;
@@ -513,6 +550,33 @@ int LaunchTiles(const MatmulArgs &p, uint32_t n_batch, float *C, const float *A,
 }
 
 }  // namespace
+
+int PartsCanCarry(const fl_tensor *weights, int64_t terms, hipStream_t s) {
+  if (weights->rank < 1 || weights->rank > 4) return FL_ERR_RANK;
+  RangeArgs a;
+  std::memset(&a, 0, sizeof(a));
+  a.n = static_cast<uint32_t>(Numel(weights));
+  a.rank = weights->rank;
+  for (int d = 0; d < a.rank; ++d) {
+    a.shape[d] = FastDiv(static_cast<uint32_t>(weights->shape[d]));
+    a.strides[d] = static_cast<int32_t>(weights->strides[d]);
+  }
+  uint32_t range[2] = {0xffffffffu, 0}, *device = nullptr;
+  FL_HIP_CHECK(hipMalloc(&device, sizeof(range)));
+  hipError_t err = hipMemcpyAsync(device, range, sizeof(range), hipMemcpyHostToDevice, s);
+  if (err == hipSuccess) {
+    const uint32_t blocks = std::min<uint32_t>((a.n + kPackThreads - 1) / kPackThreads, 1024);
+    FL_LAUNCH(WeightRangeKernel, dim3(blocks), dim3(kPackThreads), 0, s, device, static_cast<const float *>(weights->base), a);
+    err = hipGetLastError();
+  }
+  if (err == hipSuccess) err = hipMemcpyAsync(range, device, sizeof(range), hipMemcpyDeviceToHost, s);
+  if (err == hipSuccess) err = hipStreamSynchronize(s);
+  (void)hipFree(device);
+  FL_HIP_CHECK(err);
+  const float largest = __builtin_bit_cast(float, range[1]);
+  const bool ok = range[0] >= 2 * 0x21800000u - 1 && static_cast<double>(terms) * largest <= 0x1p20;  // (2^-60)
+  return ok ? FL_OK : FL_ERR_UNSUPPORTED;
+}
 
 int LaunchPacked(const MatmulArgs &args, uint32_t n_batch, bool extra, int parts, float *C, const float *A, const float *B,
                  hipStream_t s, TileChoice choice) {
@@ -584,6 +648,7 @@ int fluidml_hip_contract_pack(const fl_tensor *rhs, int32_t trans_b, int64_t row
     std::lock_guard<std::mutex> lock(g_packed_mutex);
     if (g_packed.count(rhs->base)) return FL_ERR_UNSUPPORTED;  // (packed already)
   }
+  if (parts == 3) FL_CHECK(PartsCanCarry(rhs, w.K, AsStream(stream)));
   *bytes = static_cast<size_t>(items) * 16 * parts;
   FL_HIP_CHECK(hipMalloc(&w.packed, *bytes));
   const dim3 grid(static_cast<uint32_t>((items + kPackThreads - 1) / kPackThreads));

@@ -308,7 +308,12 @@ bool IsPackableConv(const Step &step, const Operand &weights) {
 void LaunchPlan::PackConvWeights() {
   const char *env = std::getenv("FLUIDML_CONV_PACKED");
   if (env != nullptr && std::strtol(env, nullptr, 10) == 0) return;
-  std::vector<std::pair<kernel::TensorView, PackedSlot>> jobs;
+  struct Job {
+    std::string name;
+    kernel::TensorView weights;
+    PackedSlot slot;
+  };
+  std::vector<Job> jobs;
   if (flags_ != 0) return;  // (literal-reference semantics)
   for (const Launch &l : GetSchedule()) {
     const Step &step = steps_[l.kind == Launch::Kind::ConvChain ? l.owner : l.members.front()];
@@ -324,12 +329,18 @@ void LaunchPlan::PackConvWeights() {
     Check(rc, "sizing packed convolution weights");
     Check(fluidml_hip_arena_create(slot.bytes, &slot.device), "allocating packed convolution weights");
     packed_[op.name] = slot;
-    jobs.emplace_back(w, slot);
+    jobs.push_back({op.name, w, slot});
   }
   // (the allocations are cleared on the null stream, which the plan's stream does not wait for)
   Check(fluidml_hip_stream_synchronize(nullptr), "waiting for the cleared buffers");
-  for (const auto &job : jobs) {
-    Check(fluidml_hip_conv3x3_pack(&job.first.t, job.second.parts, job.second.device, stream_), "packing convolution weights");
+  for (const Job &job : jobs) {
+    const int rc = fluidml_hip_conv3x3_pack(&job.weights.t, job.slot.parts, job.slot.device, stream_);
+    if (rc == FL_ERR_UNSUPPORTED) {  // (values that the parts cannot carry)
+      fluidml_hip_free(job.slot.device);
+      packed_.erase(job.name);
+      continue;
+    }
+    Check(rc, "packing convolution weights");
   }
 }
 

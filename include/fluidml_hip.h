@@ -494,7 +494,10 @@ int fluidml_hip_matmul_chain_group_norm(int32_t count, const fl_tensor *lhs, con
  * results) or 1 (rounded to bf16, for calls with FL_CONTRACT_BF16).  From then on every contraction of this library
  * whose right operand is `rhs` (address, extents and strides) may use the packed form, which therefore has to be current:
  * the weights must not change before fluidml_hip_contract_unpack(*packed), which frees it.  The packing runs on `stream`;
- * a contraction on another stream has to be ordered behind it by the caller.  `*bytes`: size of the packed form. */
+ * a contraction on another stream has to be ordered behind it by the caller.  `*bytes`: size of the packed form.  With
+ * three parts the weights are looked at first, which waits for the stream: FL_ERR_UNSUPPORTED where one is smaller than
+ * 2^-60 and not zero, or K times the largest finite one exceeds 2^20 (parts of such values do not give what the fp32
+ * instruction gives; infinities and NaN do). */
 int fluidml_hip_contract_pack(const fl_tensor *rhs, int32_t trans_b, int64_t rows, int32_t parts, void *stream, void **packed, size_t *bytes);
 int fluidml_hip_contract_unpack(void *packed);
 /* GemmConstantWeightsBiasKernel -> elementwise chain (reference gemm.cpp:39-182); `flags` = fl_contract_flags. */
@@ -506,7 +509,8 @@ int fluidml_hip_conv_chain(const fl_tensor *in, const fl_tensor *weights, const 
  * have been laid out for the matrix cores: `packed` holds them as `parts` bf16 values each, 3 (every fp32 value is the
  * sum of its three parts: fp32 results) or 1 (rounded to bf16: the FL_CONTRACT_BF16 precision).
  * ..._packed_bytes: size of `packed` for these weights (FL_ERR_UNSUPPORTED where there is no such layout); ..._pack
- * fills it, once, on `stream`; ..._packed_chain runs the convolution, `weights` are the ones that were packed.  `flags`:
+ * fills it, once, on `stream` (FL_ERR_UNSUPPORTED, `packed` unchanged, for values fluidml_hip_contract_pack refuses too);
+ * ..._packed_chain runs the convolution, `weights` are the ones that were packed.  `flags`:
  * 0, or FL_CONTRACT_TILE(1 | 2) (2 or 4 tiles of 2 x 16 pixels per wave) and FL_CONTRACT_SPLITS(n) instead of the
  * library's rule. */
 int fluidml_hip_conv3x3_packed_bytes(const fl_tensor *weights, int32_t parts, size_t *bytes);

@@ -144,3 +144,36 @@ def test_weights_that_other_operations_read_too(device, tmp_path, monkeypatch, f
             assert np.abs(outs[v.name] - want[v.name]).max() < 0.06, i
         else:
             assert_close(outs[v.name], want[v.name], what=f"output {i}")
+
+
+@pytest.mark.parametrize("tile,splits", [(1, 1), (2, 1), (1, 2)])
+def test_packed_conv_products_that_vanish(device, tile, splits):
+    """Results of denormal numbers (see test_packed_products_that_vanish), and zeros where the input has nothing else."""
+    x, w, _ = _operands(13, 1, 32, 12, 40, 64)
+    for x_scale, w_scale in ((1e-42, 1.0), (1e-26, 1e-16)):
+        tiny, weights = ((np.abs(x) + 0.5).astype(np.float64) * x_scale).astype(np.float32), (np.abs(w) + np.float32(0.5)) * np.float32(w_scale)
+        tiny[..., 20:] = 0
+        want = _oracle(tiny.astype(np.float32), weights, None, [1, 1, 1, 1], relu=False)
+        got = _run(device, tiny, weights, None, [1, 1, 1, 1], 3, tile, splits, chain=[])
+        assert want.max() > 0 and (np.abs(got.astype(np.float64) - want) <= 2 * 288 * 2.0 ** -150 + 1e-5 * want).all()  # (both round)
+        assert (got[..., 21:] == 0).all()
+
+
+def test_conv_weights_the_parts_cannot_carry(device, tmp_path):
+    """Refused by the library, left as they stand by a plan."""
+    from fluidml_amd import cabi, fluidml, models
+
+    x, w, bias = _operands(14, 1, 32, 12, 18, 64)
+    for value in (2.0 ** -61, 1e-40, 2.0 ** 20):
+        v = w.copy()
+        v[63, 31, 2, 2] = value
+        with pytest.raises(cabi.FluidmlHipError) as e:
+            _run(device, x, v, bias, [1, 1, 1, 1], 3)
+        assert e.value.code == cabi.FL_ERR_UNSUPPORTED
+        net = models.Net("refused", 3)
+        net.output(net.relu(net.conv(net.input("x", np.float32, x.shape), net.const(v), net.const(bias), [1, 1], [1, 1, 1, 1])))
+        ex = fluidml.Executor.make_plain_greedy("refused")
+        ex.compile(net.save(os.path.join(tmp_path, "refused.onnx")))
+        out = np.zeros(net.outputs[0].shape, np.float32)
+        ex.invoke({"x": x, net.outputs[0].name: out})
+        assert_close(out, _oracle(x, v, bias, [1, 1, 1, 1]), what=str(value))

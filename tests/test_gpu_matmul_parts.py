@@ -206,3 +206,45 @@ def test_packed_outside_the_parts(device, tile):
         out = p.out()
         assert p.chain(out, flags_of(tile)) == 0
         np.testing.assert_allclose(out.double().cpu().numpy(), want.cpu().numpy(), rtol=1e-5)
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("x_scale,w_scale", [(1e-42, 1.0), (1e-41, 1e-3), (1e-21, 2e-18), (1e-26, 1e-16)])
+def test_packed_products_that_vanish(device, tile, x_scale, w_scale):
+    """Results of denormal numbers: where parts or their products come to nothing, the fp32 instruction has the word.
+    Its sums round to multiples of 2^-149, half of one per product; without the second pass they were all zero."""
+    M, K, N = 40, 96, 64
+    with Problem(device, M, K, N) as p:
+        # (no exact zeros, weights from 2^-60 on)
+        p.x.copy_((p.x.abs() + 0.5).double() * x_scale)
+        p.w[0].copy_((p.w[0].abs() + 0.5) * w_scale)
+        p.x[3] = 0
+        p.x[5, :7] = 0
+        p.x[7, 1:] = 0
+        p.b[0].zero_()
+        want = p.x.double() @ p.w[0].double()
+        p.pack()
+        out = p.out()
+        assert p.chain(out, flags_of(tile)) == 0
+        err = (out.double() - want).abs()
+        assert (err <= K * 2.0 ** -150 + 1e-6 * want.abs()).all(), err.max().item()
+        assert (out[3] == 0).all() and (out[7] != 0).any()
+
+
+@pytest.mark.parametrize("element,value", [(0, 2.0 ** -61), (95 * 64 + 63, -1e-40), (77, 2.0 ** 20), (6143, -3e38)])
+def test_weights_the_parts_cannot_carry_are_not_packed(device, element, value):
+    """Refused, and the contraction runs on them as they stand; zeros, infinities and NaN are no reason."""
+    with Problem(device, 40, 96, 64, scale=1e-35) as p:
+        p.w[0].view(-1)[5] = 0.0
+        keep = p.w[0].view(-1)[element].item()
+        p.w[0].view(-1)[element] = value
+        want = p.x.double() @ p.w[0].double() + p.b[0].double()
+        with pytest.raises(p.cabi.FluidmlHipError) as e:
+            p.pack()
+        assert e.value.code == UNSUPPORTED
+        out = p.out()
+        assert p.chain(out, flags_of("32x64")) == UNSUPPORTED and p.chain(out, 0) == 0
+        close(out, want, "as they stand")
+        p.w[0].view(-1)[element] = keep
+        p.w[0].view(-1)[6], p.w[0].view(-1)[7] = float("inf"), float("nan")
+        p.pack()
