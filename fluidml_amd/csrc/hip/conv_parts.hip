@@ -507,6 +507,7 @@ int fluidml_hip_conv3x3_packed_chain(const fl_tensor *in, const fl_tensor *weigh
   if (parts == 3) FL_PARTS(3);
   else FL_PARTS(1);
 #undef FL_PARTS
+  NotePackedParts(parts);
   return LaunchStatus();
 }
 

@@ -82,6 +82,9 @@ constexpr size_t kWorkspaceTileFloats = 1024;
 // now (the stream is being captured into a graph) or the allocation fails; callers then do without.
 StreamWorkspace *GetStreamWorkspace(hipStream_t stream);  // runtime.hip
 
+// What fluidml_hip_take_packed_parts tells the calling thread.  runtime.hip
+void NotePackedParts(int32_t parts);
+
 // Whether weights that sums of `terms` products read can stand as three bf16 parts (see below): FL_OK or
 // FL_ERR_UNSUPPORTED.  Waits for the stream.  matmul_parts.hip
 int PartsCanCarry(const fl_tensor *weights, int64_t terms, hipStream_t stream);

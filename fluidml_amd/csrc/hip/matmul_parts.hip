@@ -617,10 +617,10 @@ int LaunchPacked(const MatmulArgs &args, uint32_t n_batch, bool extra, int parts
     const int64_t chunk = tile == FL_TILE_PACKED_32x64 ? 128 : 64, chunks = (p.K + chunk - 1) / chunk;
     while (splits > 1 && (chunks + splits - 1) / splits * (splits - 1) >= chunks) --splits;
   }
-  if (parts == 3) {
-    return extra ? LaunchTiles<3, 1>(p, n_batch, C, A, B, s, tile, splits) : LaunchTiles<3, 0>(p, n_batch, C, A, B, s, tile, splits);
-  }
-  return extra ? LaunchTiles<1, 1>(p, n_batch, C, A, B, s, tile, splits) : LaunchTiles<1, 0>(p, n_batch, C, A, B, s, tile, splits);
+  const int rc = parts == 3 ? (extra ? LaunchTiles<3, 1>(p, n_batch, C, A, B, s, tile, splits) : LaunchTiles<3, 0>(p, n_batch, C, A, B, s, tile, splits))
+                            : (extra ? LaunchTiles<1, 1>(p, n_batch, C, A, B, s, tile, splits) : LaunchTiles<1, 0>(p, n_batch, C, A, B, s, tile, splits));
+  if (rc == FL_OK) NotePackedParts(parts);
+  return rc;
 }
 
 }  // namespace fl

@@ -28,7 +28,15 @@ namespace fl {
 namespace {
 std::mutex g_workspace_mutex;
 std::unordered_map<hipStream_t, StreamWorkspace> g_workspaces;
+thread_local int32_t t_packed_parts = 0;
 }  // namespace
+
+void NotePackedParts(int32_t parts) { t_packed_parts = parts; }
+int32_t TakePackedParts() {
+  const int32_t parts = t_packed_parts;
+  t_packed_parts = 0;
+  return parts;
+}
 
 StreamWorkspace *GetStreamWorkspace(hipStream_t stream) {
   std::lock_guard<std::mutex> lock(g_workspace_mutex);
@@ -87,6 +95,12 @@ __global__ __launch_bounds__(256) void MfmaRateKernel(int count, uint64_t *out) 
 }  // namespace fl
 
 extern "C" {
+
+int fluidml_hip_take_packed_parts(int32_t *parts) {
+  if (parts == nullptr) return FL_ERR_NULL;
+  *parts = TakePackedParts();
+  return FL_OK;
+}
 
 int fluidml_hip_abi_version(void) { return 3; }
 

@@ -5,6 +5,7 @@
 #include <limits>
 #include <cstdlib>
 #include <map>
+#include <set>
 #include <sstream>
 #include <stdexcept>
 
@@ -186,6 +187,7 @@ void LaunchPlan::Materialize() {
   transfer_ = std::make_unique<Transfer>(std::move(in), std::move(out));
   Check(fluidml_hip_arena_create(arena_bytes_, &arena_), "allocating the arena");
   TuneContractions();
+  UnpackUnusedWeights();
 }
 
 void *LaunchPlan::Resolve(const Operand &op) const {
@@ -375,6 +377,35 @@ void LaunchPlan::PackContractionWeights() {
       const bool gemm = kind == flow::OpKind::GemmConstantWeightsBias, own = l.kind != Launch::Kind::Step || l.rewired;
       pack(own ? l.a : step.in0, own ? l.b : step.in1, gemm && at.trans_a, gemm && at.trans_b);
     }
+  }
+}
+
+// Which launches take the packed form is the library's to say, with the operands and the configuration each really has:
+// the schedule runs once, on whatever lies in memory.
+void LaunchPlan::UnpackUnusedWeights() {
+  if (contract_packed_.empty()) return;
+  kernel::LaunchContext ctx;
+  ctx.stream = stream_;
+  ctx.flags = flags_;
+  ctx.bf16 = bf16_;
+  std::set<std::string> used;
+  for (const Launch &l : GetSchedule()) {
+    int32_t parts = 0;
+    Check(fluidml_hip_take_packed_parts(&parts), "packed launches");
+    Issue(ctx, l);
+    Check(fluidml_hip_take_packed_parts(&parts), "packed launches");
+    if (parts == 0) continue;
+    for (const Launch &m : l.group) used.insert(m.b.name);
+    if (l.group.empty()) used.insert(l.kind == Launch::Kind::Step && !l.rewired ? steps_[l.members[0]].in1.name : l.b.name);
+  }
+  Check(fluidml_hip_stream_synchronize(stream_), "waiting for the launches");
+  for (auto it = contract_packed_.begin(); it != contract_packed_.end();) {
+    if (used.count(it->first)) {
+      ++it;
+      continue;
+    }
+    Check(fluidml_hip_contract_unpack(it->second.device), "freeing packed weights");
+    it = contract_packed_.erase(it);
   }
 }
 

@@ -301,6 +301,8 @@ class LaunchPlan {
   void PackConvWeights();
   // The same for the weights of MatMul and Gemm (fluidml_hip_contract_pack); the library finds them by their address.
   void PackContractionWeights();
+  // Frees those of them that no launch takes, once the tile configurations are picked.
+  void UnpackUnusedWeights();
   // (FL_ERR_UNSUPPORTED, nothing launched, where they are not, or the operands do not fit)
   int IssuePackedConv(const Step &step, const Operand &weights, const fl_tensor &in, const fl_tensor &out,
                       const fl_ew_program *chain, void *stream) const;

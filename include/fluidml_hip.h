@@ -500,6 +500,9 @@ int fluidml_hip_matmul_chain_group_norm(int32_t count, const fl_tensor *lhs, con
  * instruction gives; infinities and NaN do). */
 int fluidml_hip_contract_pack(const fl_tensor *rhs, int32_t trans_b, int64_t rows, int32_t parts, void *stream, void **packed, size_t *bytes);
 int fluidml_hip_contract_unpack(void *packed);
+/* The parts of the packed weights (contractions and 3x3 convolutions) the calling thread's latest launch against such
+ * weights ran with, 0 if there was none since the last call of this function. */
+int fluidml_hip_take_packed_parts(int32_t *parts);
 /* GemmConstantWeightsBiasKernel -> elementwise chain (reference gemm.cpp:39-182); `flags` = fl_contract_flags. */
 int fluidml_hip_gemm_chain(const fl_tensor *lhs, const fl_tensor *rhs, const fl_tensor *bias, const fl_tensor *out, double alpha, double beta, int32_t trans_a, int32_t trans_b, const fl_ew_program *chain, uint32_t flags, void *stream);
 /* Conv{With,Without}PaddingKernel -> elementwise chain (reference conv.cpp:27-280);

@@ -248,3 +248,40 @@ def test_weights_the_parts_cannot_carry_are_not_packed(device, element, value):
         p.w[0].view(-1)[element] = keep
         p.w[0].view(-1)[6], p.w[0].view(-1)[7] = float("inf"), float("nan")
         p.pack()
+
+
+def test_a_plan_frees_the_packed_weights_no_launch_takes(device, tmp_path, monkeypatch):
+    """The tile configuration of a contraction is picked after its weights have been packed."""
+    import json
+    import os
+
+    from fluidml_amd import fluidml, models
+
+    net = models.Net("two", 1)
+    x = net.input("x", np.float32, (512, 768))
+    net.output(net.add(net.matmul(x, net.normal((768, 3072))), net.zeros((3072,))))
+    net.output(net.matmul(net.relu(x), net.normal((768, 2560))))
+    path = net.save(os.path.join(tmp_path, "two.onnx"))
+    feed = {"x": np.random.default_rng(2).standard_normal((512, 768), np.float32)}
+    want = [feed["x"] @ net.initializers[0].const, np.maximum(feed["x"], 0) @ net.initializers[2].const]
+
+    def compiled(tune, packed="1"):
+        monkeypatch.setenv("FLUIDML_TUNE", tune)
+        monkeypatch.setenv("FLUIDML_MATMUL_PACKED", packed)
+        ex = fluidml.Executor.make_plain_greedy("two")
+        ex.compile(path)
+        outs = {v.name: np.zeros(v.shape, np.float32) for v in net.outputs}
+        ex.invoke({**feed, **outs})
+        for v, w in zip(net.outputs, want):
+            np.testing.assert_allclose(outs[v.name], w, rtol=1e-4, atol=1e-5)
+        return ex, ex.plan()["private_bytes"]
+
+    _, none = compiled("0", "0")
+    ex, both = compiled("0")
+    assert both - none == 768 * (3072 + 2560) * 6
+    signature = next(sig for sig, _, _ in ex.contraction_choices() if "3072" in sig)
+    table = os.path.join(tmp_path, "picks.json")
+    with open(table, "w") as f:
+        json.dump({signature: {"tile": 2, "splits": 0}}, f)
+    _, one = compiled(table)
+    assert one - none == 768 * 2560 * 6
