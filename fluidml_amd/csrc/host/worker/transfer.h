@@ -45,6 +45,7 @@ class Transfer {
   uint64_t *clock_ = nullptr;     // device
   uint32_t *counters_ = nullptr;  // device: one per outbound slice and one per outbound launch
   uint32_t value_ = 0;
+  double wait_ns_ = 0;  // from queueing the last outbound copy to its first flag
   double ns_per_tick_ = 10.0;
 };
 
