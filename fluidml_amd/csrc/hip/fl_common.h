@@ -131,9 +131,9 @@ __host__ __device__ __forceinline__ void StaticFor(F &&body) {
 // in registers on the whole chip 287 against 130-136 TFLOP/s.
 // What the parts cannot carry shows in the sum (an infinity minus itself is no number; a result so small that parts of its
 // operands may have been denormal): BadSum tells, and the kernels then multiply that wave's tile again with the fp32
-// instruction.  An exact zero is taken for one only where the workgroup has staged no activation that is smaller than
-// 2^-40 and not zero (TinyKey): products of such values may have vanished, which the fp32 instruction would keep as
-// denormal numbers.  The weights are looked at when they are packed (PartsCanCarry): zero or at least 2^-60, so that
+// instruction.  An exact zero is taken for one only where no activation behind it is smaller than 2^-40 and not zero
+// (TinyKey; noted while the workgroup stages them, or looked up once a zero has come out): products of such values may have
+// vanished, which the fp32 instruction would keep as denormal numbers.  The weights are looked at when they are packed (PartsCanCarry): zero or at least 2^-60, so that
 // their parts are exact and products with activations from 2^-40 on stay normal, and the sums of their magnitudes at most
 // 2^20, so that the 2^-126 a denormal part may lose stays below the rounding of a result of 2^-80.
 typedef float floatx16 __attribute__((ext_vector_type(16)));

@@ -49,9 +49,8 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
   constexpr int kRed = KS > 1 ? TM * kWaves * 256 : 0;   // 16-byte places of the K slices' partial tiles
   constexpr int kLds = 2 * kStage > kRed ? 2 * kStage : kRed;
   constexpr bool NORM = EXTRA == 1;
-  __shared__ u32x4 lds[kLds + (NORM ? BM / 2 : 0) + (PARTS == 3 ? 1 : 0)];
+  __shared__ u32x4 lds[kLds + (NORM ? BM / 2 : 0)];
   float *const ln_rows = reinterpret_cast<float *>(lds + kLds);  // mean, then 1 / sqrt(var + eps), per row
-  uint32_t *const tiny_inputs = reinterpret_cast<uint32_t *>(lds + kLds + (NORM ? BM / 2 : 0));  // (BadSum; three parts)
 
   float *C = C_;
   const float *B = B_;
@@ -125,8 +124,6 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
       for (int s = 0; s < PARTS; ++s) br[S][u][s] = *reinterpret_cast<const u32x4 *>(from + s * 1024 + lane * 16u);
     }
   };
-  uint32_t tiny_key = 0xffffffffu;
-  if (PARTS == 3 && tid == 0) *tiny_inputs = 0;
   // item t of chunk c: its parts, into LDS
   auto store_item = [&](int c, int buf, auto set_c, int t) {
     constexpr int S = decltype(set_c)::value;
@@ -134,7 +131,6 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
     const floatx4 lo = ar[S][t][0], hi = ar[S][t][1];
     const float x[8] = {live ? lo.x : 0.0f, live ? lo.y : 0.0f, live ? lo.z : 0.0f, live ? lo.w : 0.0f,
                         live ? hi.x : 0.0f, live ? hi.y : 0.0f, live ? hi.z : 0.0f, live ? hi.w : 0.0f};
-    if constexpr (PARTS == 3) tiny_key = TinyKey(tiny_key, x);
     u32x4 parts[PARTS];
     SplitParts<PARTS>(x, parts);
 #pragma unroll
@@ -274,17 +270,35 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
   });
 
   if constexpr (PARTS == 3) {
-    if (tiny_key < kTinyKey) *tiny_inputs = 1;
-    __syncthreads();
-    const bool tiny = *tiny_inputs != 0;
-    bool bad = false;
+    bool bad = false, zero = false;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         acc[i][e] += low[i][e];
-        bad |= BadSum(acc[i][e], tiny);
+        bad |= BadSum(acc[i][e], false);
+        zero |= acc[i][e] == 0.0f;
       }
+    if (!__any(bad) && __any(zero && n < p.N)) {
+      // Exact zeros: look for activations of this wave's steps whose products may have vanished.  Here and not while they are
+      // staged, since only rows (or columns) of zeros come this way: noting it there cost 0.6 of 26 us at 512 rows.
+      uint32_t tiny_key = 0xffffffffu;
+      for (int cc = c_begin; cc < c_end; ++cc) {
+#pragma unroll
+        for (int u = 0; u < kSteps; ++u) {
+          const int k = (cc * kChunkSteps + ks * kSteps + u) * 16 + 8 * half;
+          if (k >= p.K) continue;
+#pragma unroll
+          for (int i = 0; i < TM; ++i) {
+            const float *at = A + static_cast<int64_t>(min(m0 + 32 * i + lrow, p.M - 1)) * p.sAm + k;
+            const floatx4 lo = *reinterpret_cast<const floatx4 *>(at), hi = *reinterpret_cast<const floatx4 *>(at + 4);
+            const float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+            tiny_key = TinyKey(tiny_key, x);
+          }
+        }
+      }
+      bad = tiny_key < kTinyKey;
+    }
     if (__any(bad)) {
       // this wave's steps once more with the fp32 instruction, operands straight from memory
 #pragma unroll
