@@ -520,13 +520,22 @@ const void *FindPacked(const float *b, const MatmulArgs &p, int parts) {
   return w.K == p.K && w.N == p.N && w.sBk == p.sBk && w.sBn == p.sBn && w.parts == parts ? w.packed : nullptr;
 }
 
-// Whether the packed form is the faster one.  Three parts: with few rows a launch is bound by bringing the weights in, and
-// the packed form is half as large again; it wins from about 64 rows and 390000 results on (us, packed against the best other
-// tile: 512 x 768 9.2 / 11.3, 512 x 3072 21.2 / 27.7, 256 x 1536 8.0 / 8.7, 128 x 3072 11.3 / 11.9, but 256 x 768 8.9 / 7.3,
-// 64 x 3072 10.1 / 8.0; 77 x 50304 57 / 72, but 20 x 50304 38 / 32).  One part: half the bytes, faster throughout (128 x 3072 6.1 / 10.7, 256 x
-// 512 4.6 / 5.2); at most eight rows stream the fp32 weights instead, whatever the precision asked for.
-bool WorthPacking(int64_t rows, int64_t cols, int parts) {
-  return parts == 1 ? rows > 8 : rows >= 64 && rows * cols >= 390000;
+// Whether the packed form is worth having: `cols` are those of all members of a launch together.
+// Three parts cost six bytes per weight beside the four that stay for the other kernels, so it is taken where a launch gets
+// about a tenth faster against the best of the other tiles, as a tuner would pick it: from 65 rows, 280000 results and
+// 580 million products on.  Measured with weights that come from HBM, gain of the best packed tile:
+//   K =  512: 512x1536 5 %, 512x2048 4 %, 77x50304 15 %, 128x50304 18 %, 256x50304 23 %; but 20x50304 -14 %, 64x50304 10 %
+//   K =  768: 128x2304 2 %, 512x768 6 %, 128x3072 5 %, 192x3072 6 %, 320x2304 4 %, 224x3072 7 % (528 million products);
+//             256x3072 13 %, 512x1536 12 % (604 million), 288x3072 12 %, 384x2304 13 %, 512x2304 19 %, 512x3072 23 %
+//   K = 1024: 128x3072 4 %, 128x4096 7 %, 384x1024 10 %, 512x1024 9 %; 192x4096 9 %, 256x4096 13 %, 300x3072 13 %; 64x32000 -8 %
+//   K = 2048: 128x2048 -8 %, 512x512 -8 %; 256x2048 14 %, 384x2048 15 %, 128x8192 17 %; 64x8192 1 %
+//   K = 3072: 256x768 1 %, 320x768 0 % (245760 results); 384x768 10 % (294912), 448x768 12 %, 512x768 10 %
+//   K = 4096: 64x4096 -3 %, 64x11008 4 %, 256x1024 6 % (262144 results); 96x4096 19 %, 128x4096 14 %, 384x1024 22 %, 256x4096 31 %
+// One part: two bytes per weight and half the traffic, faster throughout (128x3072 6.1 / 10.7 us, 256x512 4.6 / 5.2); at most
+// eight rows stream the fp32 weights instead, whatever the precision asked for.
+bool WorthPacking(int64_t rows, int64_t cols, int64_t K, int parts) {
+  if (parts == 1) return rows > 8;
+  return rows > 64 && rows * cols >= 280000 && static_cast<double>(rows) * static_cast<double>(cols) * static_cast<double>(K) >= 5.8e8;
 }
 
 template <int PARTS, int TM, int WN, int KS, int DEPTH, int EXTRA>
@@ -607,7 +616,7 @@ int LaunchPacked(const MatmulArgs &args, uint32_t n_batch, bool extra, int parts
   }
   int tile = choice.tile, splits = choice.splits > 0 ? choice.splits : 1;
   if (tile == FL_TILE_RULE) {
-    if (choice.splits != 0 || !WorthPacking(p.M, p.N, parts)) return FL_ERR_UNSUPPORTED;
+    if (choice.splits != 0 || !WorthPacking(p.M, static_cast<int64_t>(p.N) * std::max(1, p.n_groups), p.K, parts)) return FL_ERR_UNSUPPORTED;
     // 64x128 tiles while they give two thirds of the compute units a workgroup (four waves each from one per compute unit
     // on: two of them fit one then), else smaller ones, and K split over workgroups where it is long (measured, us: K = 768,
     // 512 x 3072: 64x128_K2 21.2, 64x128 23.2, 64x64 23.8; 256 x 3072: 64x64 15.9, 64x128_K2 with two splits 17.0; 512 x
@@ -654,7 +663,7 @@ int fluidml_hip_contract_pack(const fl_tensor *rhs, int32_t trans_b, int64_t row
   w.K = rhs->shape[trans_b ? 1 : 0], w.sBk = rhs->strides[trans_b ? 1 : 0];
   w.N = rhs->shape[trans_b ? 0 : 1], w.sBn = rhs->strides[trans_b ? 0 : 1];
   w.parts = parts;
-  if (!WorthPacking(rows, w.N, parts)) return FL_ERR_UNSUPPORTED;
+  if (!WorthPacking(rows, w.N, w.K, parts)) return FL_ERR_UNSUPPORTED;
   if (w.K <= 0 || w.N <= 0 || w.K > 0x3fffffff || w.N > 0x3fffffff || w.sBk < 0 || w.sBn < 0) return FL_ERR_UNSUPPORTED;
   const int64_t steps = (w.K + 15) / 16, items = (w.N + 31) / 32 * steps * 64;
   if ((items + kPackThreads - 1) / kPackThreads > 0x7fffffff) return FL_ERR_TOO_LARGE;

@@ -350,11 +350,11 @@ void LaunchPlan::PackConvWeights() {
 void LaunchPlan::PackContractionWeights() {
   const char *env = std::getenv("FLUIDML_MATMUL_PACKED");
   if (flags_ != 0 || (env != nullptr && std::strtol(env, nullptr, 10) == 0)) return;
-  auto pack = [&](const Operand &lhs, const Operand &rhs, bool trans_a, bool trans_b) {
+  auto pack = [&](const Operand &lhs, const Operand &rhs, bool trans_a, bool trans_b, size_t members = 1) {
     if (rhs.space != Operand::Space::Constant || rhs.viewed || contract_packed_.count(rhs.name)) return;
     const std::vector<int64_t> &shape = lhs.meta.GetShape();
     if (rhs.meta.GetShape().size() != 2 || shape.size() < 2 || trans_a) return;
-    int64_t rows = 1;
+    int64_t rows = static_cast<int64_t>(members);
     for (size_t d = 0; d + 1 < shape.size(); ++d) rows *= shape[d];
     if (shape.back() % 8 != 0) return;
     const kernel::TensorView w = ViewOf(Resolve(rhs), rhs);
@@ -366,7 +366,7 @@ void LaunchPlan::PackContractionWeights() {
   };
   for (const Launch &l : GetSchedule()) {
     if (l.kind == Launch::Kind::MatMulGroup) {
-      for (const Launch &m : l.group) pack(l.a, m.b, false, false);
+      for (const Launch &m : l.group) pack(l.a, m.b, false, false, l.group.size());
     } else if (l.kind == Launch::Kind::MatMulChain) {
       pack(l.a, l.b, false, false);
     } else if (l.kind == Launch::Kind::GemmChain || l.kind == Launch::Kind::Step) {

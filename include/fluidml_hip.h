@@ -489,8 +489,8 @@ typedef struct fl_norm_fusion {
  * (FL_TILE_128x128_STAGED: deferred rows of at most 512 elements). */
 int fluidml_hip_matmul_chain_group_norm(int32_t count, const fl_tensor *lhs, const fl_tensor *const *rhs, const fl_tensor *const *bias, const fl_tensor *const *col_sum, const fl_tensor *const *out, int64_t n_inner, const int64_t *stride_outer, const fl_ew_program *chain, const fl_tensor *addend, const fl_norm_fusion *norm, uint32_t flags, void *stream);
 /* Lays constant weights out for the matrix cores, once: `rhs` is the rank-2 right operand of a MatMul ([K, N]) or, with
- * `trans_b`, of a Gemm ([N, K]) whose left operand has `rows` rows (FL_ERR_UNSUPPORTED where the other kernels are the
- * faster ones at that size).  Every value is stored as `parts` bf16 values, 3 (it is the sum of the three: fp32
+ * `trans_b`, of a Gemm ([N, K]) whose left operand has `rows` rows, times the members of the launch where there are
+ * several (FL_ERR_UNSUPPORTED where the packed form is not worth its memory at that size; each launch decides again).  Every value is stored as `parts` bf16 values, 3 (it is the sum of the three: fp32
  * results) or 1 (rounded to bf16, for calls with FL_CONTRACT_BF16).  From then on every contraction of this library
  * whose right operand is `rhs` (address, extents and strides) may use the packed form, which therefore has to be current:
  * the weights must not change before fluidml_hip_contract_unpack(*packed), which frees it.  The packing runs on `stream`;

@@ -25,3 +25,14 @@ def test_packed_convolution_has_one_output_size(size, pads, out):
     rc = cabi.lib.fluidml_hip_conv3x3_packed_chain(ctypes.byref(x), ctypes.byref(w), x.base, 3, None, ctypes.byref(o),
                                                    cabi.i64_array(pads), None, 0, None)
     assert rc == FL_ERR_SHAPE
+
+
+@pytest.mark.parametrize("rows,K,N", [
+    (128, 768, 3072), (192, 768, 3072), (512, 768, 768),  # a twentieth faster, for half as much memory again
+    (64, 4096, 4096), (20, 512, 50304),                   # slower
+    (256, 3072, 768), (320, 3072, 768), (128, 2048, 2048),
+])
+def test_weights_not_worth_packing(rows, K, N):
+    w, packed, size = tensor(K, N), ctypes.c_void_p(), ctypes.c_size_t()
+    rc = cabi.lib.fluidml_hip_contract_pack(ctypes.byref(w), 0, rows, 3, None, ctypes.byref(packed), ctypes.byref(size))
+    assert rc == cabi.FL_ERR_UNSUPPORTED and not packed.value

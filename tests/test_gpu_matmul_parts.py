@@ -285,3 +285,22 @@ def test_a_plan_frees_the_packed_weights_no_launch_takes(device, tmp_path, monke
         json.dump({signature: {"tile": 2, "splits": 0}}, f)
     _, one = compiled(table)
     assert one - none == 768 * 2560 * 6
+
+
+@pytest.mark.parametrize("M,K,N,count,packed", [
+    (65, 768, 11648, 1, True), (64, 768, 12288, 1, False),                                # rows
+    (384, 3072, 768, 1, True), (364, 3072, 768, 1, False),                                # results
+    (246, 768, 3072, 1, True), (245, 768, 3072, 1, False), (328, 768, 768, 3, True), (327, 768, 768, 3, False),  # products
+])
+def test_the_rule_counts_rows_results_and_products_of_all_members(device, M, K, N, count, packed):
+    with Problem(device, M, K, N, count=count) as p:
+        p.pack()
+        parts = ctypes.c_int32()
+        p.cabi.call("take_packed_parts", ctypes.byref(parts))
+        outs = [p.out() for _ in range(count)]
+        none = ctypes.byref(p.cabi.make_chain([]))
+        assert p.cabi.lib.fluidml_hip_matmul_chain_group(count, p.ref(p.x), p.list(p.w), p.list(p.b), p.list(outs), 0, None, none, 0, None) == 0
+        p.cabi.call("take_packed_parts", ctypes.byref(parts))
+        assert (parts.value == 3) == packed
+        for o, w, b in zip(outs, p.w, p.b):
+            close(o, p.x.double() @ w.double() + b.double(), "members")
