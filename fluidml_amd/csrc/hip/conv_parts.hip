@@ -53,8 +53,6 @@ struct PartsArgs {
   uint32_t n_splits;
   int32_t chunks_per_split;
   int32_t weight_major;  // consecutive workgroups share weights (else: the patch)
-  int32_t sWf, sWc, sWh, sWw;  // the weights as they stand in the graph, for the tiles that BadSum sends back
-  const float *weights;
   const float *bias;
   int32_t sB;
   float *partials;
@@ -215,17 +213,18 @@ __global__ __launch_bounds__(kThreads, 2) void ConvPartsKernel(float *out, const
 #pragma unroll
       for (int e = 0; e < 16; ++e) bad |= BadSum(acc[j][e], tiny);
     if (__any(bad)) {
-      // the same channels once more with the fp32 instruction, operands straight from memory
+      // the same channels once more with the fp32 instruction, operands straight from memory (filters and channels that do
+      // not exist are zero in the packed weights)
+      const uint16_t *w_src = reinterpret_cast<const uint16_t *>(packed) +
+                              static_cast<int64_t>(min(ftile, p.ftiles - 1)) * p.chunks * (9 * PARTS * 512) + lrow * 8;
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[j][e] = 0.0f;
-      const int f = ftile * 32 + lrow;
       for (int c0 = c_first * kChunk; c0 < min(p.C, c_end * kChunk); c0 += 2) {
         const int ch = c0 + half;
         for (int tap = 0; tap < 9; ++tap) {
-          const bool live = ch < p.C && f < p.F;
-          const float w = live ? p.weights[static_cast<int64_t>(f) * p.sWf + static_cast<int64_t>(ch) * p.sWc + tap / 3 * p.sWh + tap % 3 * p.sWw] : 0.0f;
+          const float w = JoinParts(w_src + (ch / 16 * 9 + tap) * (PARTS * 512) + ch % 16 / 8 * 256 + ch % 8, 512);
 #pragma unroll
           for (int j = 0; j < TN; ++j) {
             const int ih = oh0 + py + 2 * j - p.ph + tap / 3, iw = ow0 + px - p.pw + tap % 3;
@@ -461,9 +460,6 @@ int fluidml_hip_conv3x3_packed_chain(const fl_tensor *in, const fl_tensor *weigh
   p.sXh = static_cast<int32_t>(in->strides[2]), p.sXw = static_cast<int32_t>(in->strides[3]);
   p.sOn = static_cast<int32_t>(out->strides[0]), p.sOf = static_cast<int32_t>(out->strides[1]);
   p.sOh = static_cast<int32_t>(out->strides[2]), p.sOw = static_cast<int32_t>(out->strides[3]);
-  p.sWf = static_cast<int32_t>(weights->strides[0]), p.sWc = static_cast<int32_t>(weights->strides[1]);
-  p.sWh = static_cast<int32_t>(weights->strides[2]), p.sWw = static_cast<int32_t>(weights->strides[3]);
-  p.weights = static_cast<const float *>(weights->base);
   if (bias != nullptr) {
     FL_CHECK(CheckView(bias));
     if (bias->dtype != FL_FLOAT32) return FL_ERR_DTYPE;

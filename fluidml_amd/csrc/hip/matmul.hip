@@ -1606,7 +1606,8 @@ int Contract(const fl_tensor *lhs, const fl_tensor *rhs, const fl_tensor *out, b
   // at most 8 rows against k-contiguous weights: HBM-bound weight streaming, fp32 whatever `bf16` says (a caller
   // that names a tile configuration gets the tiled kernel)
   const bool free_choice = choice.tile == FL_TILE_RULE && choice.splits == 0;
-  if (!extra && free_choice && TrySkinnyGemm(p, n_batch, C, A, B, s)) return LaunchStatus();
+  const bool only_packed = OnlyPacked(p, B);
+  if (!extra && free_choice && !only_packed && TrySkinnyGemm(p, n_batch, C, A, B, s)) return LaunchStatus();
   const uint32_t nb = static_cast<uint32_t>(n_batch);
   int rc = FL_ERR_UNSUPPORTED;
   if (choice.tile == FL_TILE_RULE || choice.tile >= FL_TILE_PACKED_32x64) {
@@ -1614,6 +1615,7 @@ int Contract(const fl_tensor *lhs, const fl_tensor *rhs, const fl_tensor *out, b
     if (rc != FL_ERR_UNSUPPORTED) return rc != FL_OK ? rc : LaunchStatus();
     if (choice.tile != FL_TILE_RULE) return rc;
   }
+  if (only_packed) return FL_ERR_UNSUPPORTED;
   if (extra) {
 #define FL_MM_EXTRA(E_)                                                                 \
   do {                                                                                  \

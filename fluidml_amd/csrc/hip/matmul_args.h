@@ -110,6 +110,9 @@ struct TileChoice {
 int LaunchPacked(const MatmulArgs &p, uint32_t n_batch, bool extra, int parts, float *C, const float *A, const float *B,
                  hipStream_t s, TileChoice choice);
 
+// Whether B, or that of a member, exists in its packed form only: no other kernel can read it.
+bool OnlyPacked(const MatmulArgs &p, const float *B);
+
 }  // namespace fl
 
 #endif

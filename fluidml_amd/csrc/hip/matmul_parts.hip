@@ -567,7 +567,6 @@ int LaunchTiles(const MatmulArgs &p, uint32_t n_batch, float *C, const float *A,
     case FL_TILE_PACKED_64x64: return LaunchTile<PARTS, 2, 2, 2, 2, EXTRA>(p, n_batch, C, A, B, s, splits);
     case FL_TILE_PACKED_64x128: return LaunchTile<PARTS, 2, 4, 1, 3, EXTRA>(p, n_batch, C, A, B, s, splits);
     case FL_TILE_PACKED_64x128_K2: return LaunchTile<PARTS, 2, 4, 2, 2, EXTRA>(p, n_batch, C, A, B, s, splits);
-    case FL_TILE_PACKED_128x128_K2: return LaunchTile<PARTS, 4, 4, 2, 1, EXTRA>(p, n_batch, C, A, B, s, splits);
     default: return FL_ERR_UNSUPPORTED;
   }
 }

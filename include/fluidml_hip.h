@@ -139,8 +139,7 @@ enum fl_contract_tile {
   FL_TILE_PACKED_32x64 = 9,       /* two waves side by side times four K slices */
   FL_TILE_PACKED_64x64 = 10,      /* two times two, two row tiles per wave */
   FL_TILE_PACKED_64x128 = 11,     /* four waves side by side, two row tiles each */
-  FL_TILE_PACKED_64x128_K2 = 12,  /* the same times two K slices */
-  FL_TILE_PACKED_128x128_K2 = 13  /* four row tiles each */
+  FL_TILE_PACKED_64x128_K2 = 12   /* the same times two K slices */
 };
 #define FL_CONTRACT_TILE_SHIFT 4
 #define FL_CONTRACT_SPLIT_SHIFT 8

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
-TILES = {"32x64": 9, "64x64": 10, "64x128": 11, "64x128_K2": 12, "128x128_K2": 13}
+TILES = {"32x64": 9, "64x64": 10, "64x128": 11, "64x128_K2": 12}
 UNSUPPORTED = -8
 
 
