@@ -5,7 +5,8 @@ Executor (plain_greedy by default) and replayed as HIP launches over one HBM are
 A "step" is one inference: one replay of the whole launch plan (416 graph nodes issued as a few dozen kernel
 launches after launch-level fusion) on inputs that are already resident in HBM.  Prints ONE JSON line:
 `value` = inferences/s over the timed replays; `roofline` = the contraction kernel's flops over its launch
-durations (dispatch begin/end timestamps) against the fp32 MFMA peak, `roofline.traffic` = the HBM bytes per
+durations (dispatch begin/end timestamps) against the peak of the matrix instruction each launch runs on (fp32 MFMA;
+for launches against packed weights bf16 MFMA, a sixth of it where six products give an fp32 result), `roofline.traffic` = the HBM bytes per
 launch the tracked profiler summary (`roofline.traffic_source`) holds for exactly this workload, else null;
 `cpu_baseline` = the oracle's scalar loop nests on one host core for a bounded sample;
 `peak_hbm_bytes` = arena + constants + interface staging.  The default run adds `configs`: the same
@@ -27,6 +28,10 @@ if ROOT not in sys.path:
 
 FP32_MFMA_PEAK_TFLOPS = 157.3  # MI355X dense fp32 matrix peak
 HBM_PEAK_GBS = 8000.0
+# Launches against packed weights multiply on the bf16 matrix instruction: one product per pair of values with weights of
+# one part (the opt-in bf16 precision), six with three parts (fp32 results).
+BF16_MFMA_PEAK_TFLOPS = 2500.0  # MI355X dense bf16 matrix peak
+MATRIX_PEAK_TFLOPS = {0: FP32_MFMA_PEAK_TFLOPS, 1: BF16_MFMA_PEAK_TFLOPS, 3: BF16_MFMA_PEAK_TFLOPS / 6}
 
 # HBM bytes per launch of the contraction kernel come from the tracked profiler summary of the default workload
 # (BERT-base, seq 128, 12 layers, plain_greedy, fusion on): rocprofv3 FETCH_SIZE / WRITE_SIZE per dispatch, each
@@ -195,7 +200,9 @@ def measure(args, config, executor, per_kernel=False, per_launch=False):
             family = "AttentionKernel"  # scores, softmax and context product in one launch: its own device kernel
         if family in ("TransposeKernel", "ReshapeKernel") and "+" in t["kernel"]:
             family = "ReshapeKernel"
-        k = by_kernel.setdefault(family, {"ns": 0.0, "bytes": 0.0, "flops": 0.0, "launches": 0})
+        k = by_kernel.setdefault(family, {"ns": 0.0, "bytes": 0.0, "flops": 0.0, "launches": 0, "packed": 0, "ideal_ns": 0.0})
+        k["packed"] += t["packed_parts"] != 0
+        k["ideal_ns"] += t["flops"] / MATRIX_PEAK_TFLOPS[t["packed_parts"]] / 1e3
         k["ns"] += t["ns"]
         k["bytes"] += t["bytes"]
         k["flops"] += t["flops"]
@@ -204,12 +211,15 @@ def measure(args, config, executor, per_kernel=False, per_launch=False):
     dname, d = dominant
     if d["flops"] > 0:
         achieved = d["flops"] / d["ns"] / 1e3  # flop/ns = GFLOP/s -> TFLOP/s
+        # the rate at which these flops would run with every launch at the peak of its own matrix instruction
+        peak = d["flops"] / d["ideal_ns"] / 1e3
         default_workload = (args.config, args.layers, args.seq, args.executor) == ("bert_base", 12, 128, "plain_greedy") and \
             os.environ.get("FLUIDML_FUSE", "1") != "0"
         roofline = {"bound": "mfma", "kernel": dname + " (all launches of the contraction kernel, fused epilogues included)",
-                    "achieved": achieved, "peak": FP32_MFMA_PEAK_TFLOPS,
-                    "unit": "TFLOP/s", "frac": achieved / FP32_MFMA_PEAK_TFLOPS,
-                    "traffic": traffic_from_summary() if default_workload and dname == "MatMulKernel" else None,
+                    "achieved": achieved, "peak": peak, "unit": "TFLOP/s", "frac": achieved / peak,
+                    "launches_on_packed_weights": d["packed"],
+                    # (the summary's launches are the ones against weights as they stand)
+                    "traffic": traffic_from_summary() if default_workload and dname == "MatMulKernel" and d["packed"] == 0 else None,
                     "traffic_source": TRAFFIC_SUMMARY + (" (rocprofv3 FETCH_SIZE + WRITE_SIZE per dispatch, scaled by the "
                                                          "identity-copy kernel's readings)" if default_workload else
                                                          " covers the default workload only: not measured for this one"),

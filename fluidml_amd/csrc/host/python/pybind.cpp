@@ -379,6 +379,7 @@ PYBIND11_MODULE(fluidml, m) {
                d["ns"] = t.ns;
                d["bytes"] = t.bytes;
                d["flops"] = t.flops;
+               d["packed_parts"] = t.packed_parts;
                out.append(d);
              }
              return out;

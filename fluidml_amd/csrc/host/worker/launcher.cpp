@@ -1442,6 +1442,9 @@ std::vector<StepTime> LaunchPlan::Profile(size_t warmup, size_t iters) {
   ctx.bf16 = bf16_;
   const std::vector<Launch> &schedule = GetSchedule();
   std::vector<std::vector<double>> samples(schedule.size());
+  std::vector<int32_t> packed_parts(schedule.size(), 0);
+  int32_t before = 0;
+  Check(fluidml_hip_take_packed_parts(&before), "packed launches");
   // one start/stop pair per launch, stamped by the dispatch itself (kernel-exact durations)
   std::vector<void *> events(2 * schedule.size(), nullptr);
   for (void *&e : events) Check(fluidml_hip_event_create(&e), "event");
@@ -1451,6 +1454,7 @@ std::vector<StepTime> LaunchPlan::Profile(size_t warmup, size_t iters) {
         if (schedule[i].kind == Launch::Kind::View || schedule[i].kind == Launch::Kind::Placed) continue;
         Check(fluidml_hip_time_kernels(events[2 * i], events[2 * i + 1]), "kernel timing on");
         Issue(ctx, schedule[i]);
+        Check(fluidml_hip_take_packed_parts(&packed_parts[i]), "packed launches");
       }
     } catch (...) {
       fluidml_hip_time_kernels(nullptr, nullptr);
@@ -1482,6 +1486,7 @@ std::vector<StepTime> LaunchPlan::Profile(size_t warmup, size_t iters) {
     t.ns = v.empty() ? 0 : v[v.size() / 2];
     t.bytes = l.bytes;
     t.flops = l.flops;
+    t.packed_parts = packed_parts[i];
     out.push_back(std::move(t));
   }
   return out;

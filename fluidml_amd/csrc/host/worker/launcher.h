@@ -178,6 +178,7 @@ struct Argument {
 struct StepTime {
   std::string node, kernel;
   double ns = 0, bytes = 0, flops = 0;
+  int32_t packed_parts = 0;  // bf16 parts of the packed weights it ran with, 0: none
 };
 
 class LaunchPlan {
