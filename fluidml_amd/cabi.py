@@ -162,6 +162,7 @@ SIGNATURES = {
     # contractions
     "fluidml_hip_contract_pack": [_T, _i32, _i64, _i32, _vp, _P(_vp), _P(_sz)],
     "fluidml_hip_contract_unpack": [_vp],
+    "fluidml_hip_contract_adopt": [_vp],
     "fluidml_hip_take_packed_parts": [_P(_i32)],
     "fluidml_hip_matmul": [_T, _T, _T, _vp],
     "fluidml_hip_matmul_no_alloc": [_T, _T, _T, _vp],

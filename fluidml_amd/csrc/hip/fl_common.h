@@ -157,6 +157,14 @@ __device__ __forceinline__ void SplitParts(const float (&x)[8], u32x4 (&parts)[P
   }
 }
 
+// The value whose three parts lie `step` values apart: exact for what PartsCanCarry lets through, infinities and NaN.
+__device__ __forceinline__ float JoinParts(const uint16_t *at, int step) {
+  float part[3];
+#pragma unroll
+  for (int q = 0; q < 3; ++q) part[q] = __builtin_bit_cast(float, static_cast<uint32_t>(at[q * step]) << 16);
+  return fabsf(part[0]) < __builtin_inff() ? part[0] + part[1] + part[2] : part[0];
+}
+
 // acc + low += A(32 x 16) B(16 x 32), every operand as its PARTS parts: the products of the leading parts go to acc, all
 // others (a 256th of them at most) to low, so that acc sees one rounding per sixteen values of k
 template <int PARTS>

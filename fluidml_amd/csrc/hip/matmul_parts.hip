@@ -32,7 +32,7 @@ constexpr int kPackThreads = 256;
 constexpr int kSteps = 2;  // steps of 16 k per wave and chunk
 
 template <int PARTS, int TM, int WN, int KS, int DEPTH, int EXTRA>
-__global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, const float *A, const float *B_, MatmulArgs p) {
+__global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, const float *A, MatmulArgs p) {
   // (no __restrict__ on what is loaded ahead of its use: see conv_parts.hip)
   constexpr int kWaves = WN * KS, kThreads = 64 * kWaves;
   constexpr int BM = 32 * TM, BN = 32 * WN;
@@ -53,13 +53,12 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
   float *const ln_rows = reinterpret_cast<float *>(lds + kLds);  // mean, then 1 / sqrt(var + eps), per row
 
   float *C = C_;
-  const float *B = B_;
   const int tid = threadIdx.x, lane = tid % 64;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int ks = wave / WN, wn = wave % WN;
   const int lrow = lane % 32, half = lane / 32;
 
-  asm volatile("" ::"s"(p.M), "s"(p.N), "s"(p.K), "s"(p.sAm), "s"(p.sBk), "s"(p.sBn), "s"(p.sCm), "s"(p.sCn), "s"(p.tiles_m),
+  asm volatile("" ::"s"(p.M), "s"(p.N), "s"(p.K), "s"(p.sAm), "s"(p.sCm), "s"(p.sCn), "s"(p.tiles_m),
                "s"(p.tiles_n), "s"(p.n_splits), "s"(p.chunks_per_split), "s"(p.n_groups), "s"(p.n_inner), "s"(p.sCn_outer),
                "s"(p.bias), "s"(p.sDm), "s"(p.sDn), "s"(p.ca), "s"(p.cb), "s"(p.partials), "s"(p.counters), "s"(p.chain_n),
                "s"(p.packed));
@@ -75,7 +74,6 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
   int32_t sCm = p.sCm, sCn = p.sCn, sCn_outer = p.sCn_outer;
   if (p.n_groups > 1 && blockIdx.y > 0) {
     const uint32_t g = blockIdx.y - 1;
-    B = p.gB[g];
     C = p.gC[g];
     packed = static_cast<const u32x4 *>(p.g_packed[g]);
     bias = p.gbias[g];
@@ -301,6 +299,7 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
     }
     if (__any(bad)) {
       // this wave's steps once more with the fp32 instruction, operands straight from memory
+      const uint16_t *b_src = reinterpret_cast<const uint16_t *>(b_base) + lrow * 8;
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -309,7 +308,7 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
         const int k0 = (cc * kChunkSteps + ks * kSteps) * 16;
         for (int k = k0; k < min(p.K, k0 + 16 * kSteps); k += 2) {
           const bool live = k + half < p.K;
-          const float b = live && n < p.N ? B[static_cast<int64_t>(k + half) * p.sBk + static_cast<int64_t>(n) * p.sBn] : 0.0f;
+          const float b = live && n < p.N ? JoinParts(b_src + (k + half) / 16 * (PARTS * 512) + (k + half) % 16 / 8 * 256 + (k + half) % 8, 512) : 0.0f;
 #pragma unroll
           for (int i = 0; i < TM; ++i) {
             const int m = m0 + 32 * i + lrow;
@@ -520,9 +519,16 @@ const void *FindPacked(const float *b, const MatmulArgs &p, int parts) {
   return w.K == p.K && w.N == p.N && w.sBk == p.sBk && w.sBn == p.sBn && w.parts == parts ? w.packed : nullptr;
 }
 
+// B (or a member's) is the packed form itself
+bool StandsPacked(const float *b) {
+  std::lock_guard<std::mutex> lock(g_packed_mutex);
+  const auto it = g_packed.find(b);
+  return it != g_packed.end() && it->second.packed == b;
+}
+
 // Whether the packed form is worth having: `cols` are those of all members of a launch together.
-// Three parts cost six bytes per weight beside the four that stay for the other kernels, so it is taken where a launch gets
-// about a tenth faster against the best of the other tiles, as a tuner would pick it: from 65 rows, 280000 results and
+// Three parts cost six bytes per weight instead of four (beside them, where somebody reads the weights as they stand too), so it
+// is taken where a launch gets about a tenth faster against the best of the other tiles, as a tuner would pick it: from 65 rows, 280000 results and
 // 580 million products on.  Measured with weights that come from HBM, gain of the best packed tile:
 //   K =  512: 512x1536 5 %, 512x2048 4 %, 77x50304 15 %, 128x50304 18 %, 256x50304 23 %; but 20x50304 -14 %, 64x50304 10 %
 //   K =  768: 128x2304 2 %, 512x768 6 %, 128x3072 5 %, 192x3072 6 %, 320x2304 4 %, 224x3072 7 % (528 million products);
@@ -539,7 +545,7 @@ bool WorthPacking(int64_t rows, int64_t cols, int64_t K, int parts) {
 }
 
 template <int PARTS, int TM, int WN, int KS, int DEPTH, int EXTRA>
-int LaunchTile(MatmulArgs q, uint32_t n_batch, float *C, const float *A, const float *B, hipStream_t s, int splits) {
+int LaunchTile(MatmulArgs q, uint32_t n_batch, float *C, const float *A, hipStream_t s, int splits) {
   constexpr int BK = 16 * kSteps * KS, kWaves = WN * KS;
   q.chain_n = q.chain.n;
   q.tiles_m = static_cast<uint32_t>((q.M + 32 * TM - 1) / (32 * TM));
@@ -556,22 +562,28 @@ int LaunchTile(MatmulArgs q, uint32_t n_batch, float *C, const float *A, const f
     q.partials = ws->partials;
     q.counters = ws->counters;
   }
-  FL_LAUNCH((MatmulPartsKernel<PARTS, TM, WN, KS, DEPTH, EXTRA>), dim3(q.tiles_m * q.tiles_n, n_batch, splits), dim3(64 * kWaves), 0, s, C, A, B, q);
+  FL_LAUNCH((MatmulPartsKernel<PARTS, TM, WN, KS, DEPTH, EXTRA>), dim3(q.tiles_m * q.tiles_n, n_batch, splits), dim3(64 * kWaves), 0, s, C, A, q);
   return FL_OK;
 }
 
 template <int PARTS, int EXTRA>
-int LaunchTiles(const MatmulArgs &p, uint32_t n_batch, float *C, const float *A, const float *B, hipStream_t s, int tile, int splits) {
+int LaunchTiles(const MatmulArgs &p, uint32_t n_batch, float *C, const float *A, hipStream_t s, int tile, int splits) {
   switch (tile) {
-    case FL_TILE_PACKED_32x64: return LaunchTile<PARTS, 1, 2, 4, 2, EXTRA>(p, n_batch, C, A, B, s, splits);
-    case FL_TILE_PACKED_64x64: return LaunchTile<PARTS, 2, 2, 2, 2, EXTRA>(p, n_batch, C, A, B, s, splits);
-    case FL_TILE_PACKED_64x128: return LaunchTile<PARTS, 2, 4, 1, 3, EXTRA>(p, n_batch, C, A, B, s, splits);
-    case FL_TILE_PACKED_64x128_K2: return LaunchTile<PARTS, 2, 4, 2, 2, EXTRA>(p, n_batch, C, A, B, s, splits);
+    case FL_TILE_PACKED_32x64: return LaunchTile<PARTS, 1, 2, 4, 2, EXTRA>(p, n_batch, C, A, s, splits);
+    case FL_TILE_PACKED_64x64: return LaunchTile<PARTS, 2, 2, 2, 2, EXTRA>(p, n_batch, C, A, s, splits);
+    case FL_TILE_PACKED_64x128: return LaunchTile<PARTS, 2, 4, 1, 3, EXTRA>(p, n_batch, C, A, s, splits);
+    case FL_TILE_PACKED_64x128_K2: return LaunchTile<PARTS, 2, 4, 2, 2, EXTRA>(p, n_batch, C, A, s, splits);
     default: return FL_ERR_UNSUPPORTED;
   }
 }
 
 }  // namespace
+
+bool OnlyPacked(const MatmulArgs &p, const float *B) {
+  bool only = StandsPacked(B);
+  for (int g = 1; g < p.n_groups; ++g) only |= StandsPacked(p.gB[g - 1]);
+  return only;
+}
 
 int PartsCanCarry(const fl_tensor *weights, int64_t terms, hipStream_t s) {
   if (weights->rank < 1 || weights->rank > 4) return FL_ERR_RANK;
@@ -639,8 +651,8 @@ int LaunchPacked(const MatmulArgs &args, uint32_t n_batch, bool extra, int parts
     const int64_t chunk = tile == FL_TILE_PACKED_32x64 ? 128 : 64, chunks = (p.K + chunk - 1) / chunk;
     while (splits > 1 && (chunks + splits - 1) / splits * (splits - 1) >= chunks) --splits;
   }
-  const int rc = parts == 3 ? (extra ? LaunchTiles<3, 1>(p, n_batch, C, A, B, s, tile, splits) : LaunchTiles<3, 0>(p, n_batch, C, A, B, s, tile, splits))
-                            : (extra ? LaunchTiles<1, 1>(p, n_batch, C, A, B, s, tile, splits) : LaunchTiles<1, 0>(p, n_batch, C, A, B, s, tile, splits));
+  const int rc = parts == 3 ? (extra ? LaunchTiles<3, 1>(p, n_batch, C, A, s, tile, splits) : LaunchTiles<3, 0>(p, n_batch, C, A, s, tile, splits))
+                            : (extra ? LaunchTiles<1, 1>(p, n_batch, C, A, s, tile, splits) : LaunchTiles<1, 0>(p, n_batch, C, A, s, tile, splits));
   if (rc == FL_OK) NotePackedParts(parts);
   return rc;
 }
@@ -692,6 +704,19 @@ int fluidml_hip_contract_pack(const fl_tensor *rhs, int32_t trans_b, int64_t row
   std::lock_guard<std::mutex> lock(g_packed_mutex);
   g_packed[rhs->base] = w;
   *packed = w.packed;
+  return FL_OK;
+}
+
+int fluidml_hip_contract_adopt(void *packed) {
+  using namespace fl;
+  if (packed == nullptr) return FL_ERR_NULL;
+  std::lock_guard<std::mutex> lock(g_packed_mutex);
+  auto it = g_packed.begin();
+  while (it != g_packed.end() && it->second.packed != packed) ++it;
+  if (it == g_packed.end()) return FL_ERR_ATTR;
+  const PackedWeights w = it->second;
+  g_packed.erase(it);
+  g_packed[packed] = w;
   return FL_OK;
 }
 

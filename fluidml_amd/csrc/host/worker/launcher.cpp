@@ -43,7 +43,9 @@ LaunchPlan::~LaunchPlan() {
   for (void *e : region_events_) fluidml_hip_event_destroy(e);
   if (side_stream_) fluidml_hip_stream_destroy(side_stream_);
   for (auto &kv : contract_packed_) fluidml_hip_contract_unpack(kv.second.device);
-  for (auto &kv : constants_) fluidml_hip_free(kv.second.device);
+  for (auto &kv : constants_) {
+    if (!kv.second.packed_only) fluidml_hip_free(kv.second.device);
+  }
   for (auto &kv : privates_) fluidml_hip_free(kv.second.device);
   for (auto &kv : interfaces_) fluidml_hip_free(kv.second.device);
   for (auto &kv : packed_) fluidml_hip_free(kv.second.device);
@@ -57,7 +59,7 @@ void LaunchPlan::AddArgument(Argument &&arg) {
 }
 
 void LaunchPlan::AddConstant(const std::string &name, const Tensor &tensor, const std::vector<size_t> &layout) {
-  constants_.insert({name, ConstantSlot{tensor, layout, nullptr}});
+  constants_.insert({name, ConstantSlot{tensor, layout, nullptr, false}});
 }
 
 void LaunchPlan::AddPrivate(const std::string &name, size_t bytes) { privates_[name].bytes = bytes; }
@@ -66,7 +68,7 @@ void LaunchPlan::AddStep(Step &&step) { steps_.push_back(std::move(step)); }
 
 size_t LaunchPlan::GetConstantBytes() const {
   size_t n = 0;
-  for (const auto &kv : constants_) n += kv.second.tensor.GetMeta().GetSize();
+  for (const auto &kv : constants_) n += kv.second.packed_only ? 0 : kv.second.tensor.GetMeta().GetSize();
   for (const Step &s : steps_) n += s.kernel->GetConstantBytes();
   return n;
 }
@@ -187,7 +189,6 @@ void LaunchPlan::Materialize() {
   transfer_ = std::make_unique<Transfer>(std::move(in), std::move(out));
   Check(fluidml_hip_arena_create(arena_bytes_, &arena_), "allocating the arena");
   TuneContractions();
-  UnpackUnusedWeights();
 }
 
 void *LaunchPlan::Resolve(const Operand &op) const {
@@ -276,8 +277,8 @@ void LaunchPlan::FoldNorms() {
       for (size_t n = 0; n < N; ++n) c2[n] += bias[n];
     }
     w.tensor = Tensor(Type::kFloat32, std::vector<int64_t>(shape), std::move(scaled));
-    constants_.insert({"norm_c1:" + wname, ConstantSlot{Tensor(Type::kFloat32, {static_cast<int64_t>(N)}, std::move(c1)), {0}, nullptr}});
-    constants_.insert({"norm_c2:" + wname, ConstantSlot{Tensor(Type::kFloat32, {static_cast<int64_t>(N)}, std::move(c2)), {0}, nullptr}});
+    constants_.insert({"norm_c1:" + wname, ConstantSlot{Tensor(Type::kFloat32, {static_cast<int64_t>(N)}, std::move(c1)), {0}, nullptr, false}});
+    constants_.insert({"norm_c2:" + wname, ConstantSlot{Tensor(Type::kFloat32, {static_cast<int64_t>(N)}, std::move(c2)), {0}, nullptr, false}});
     folded_[wname] = owner;
   };
   for (const Launch &l : GetSchedule()) {
@@ -382,30 +383,67 @@ void LaunchPlan::PackContractionWeights() {
 
 // Which launches take the packed form is the library's to say, with the operands and the configuration each really has:
 // the schedule runs once, on whatever lies in memory.
-void LaunchPlan::UnpackUnusedWeights() {
-  if (contract_packed_.empty()) return;
+void LaunchPlan::SettleWeights() {
+  if (packed_.empty() && contract_packed_.empty()) return;
   kernel::LaunchContext ctx;
   ctx.stream = stream_;
   ctx.flags = flags_;
   ctx.bf16 = bf16_;
-  std::set<std::string> used;
+  std::set<std::string> packed, raw;  // constants read in the one form and in the other
   for (const Launch &l : GetSchedule()) {
+    if (l.kind == Launch::Kind::View || l.kind == Launch::Kind::Placed) continue;
     int32_t parts = 0;
     Check(fluidml_hip_take_packed_parts(&parts), "packed launches");
     Issue(ctx, l);
     Check(fluidml_hip_take_packed_parts(&parts), "packed launches");
-    if (parts == 0) continue;
-    for (const Launch &m : l.group) used.insert(m.b.name);
-    if (l.group.empty()) used.insert(l.kind == Launch::Kind::Step && !l.rewired ? steps_[l.members[0]].in1.name : l.b.name);
-  }
-  Check(fluidml_hip_stream_synchronize(stream_), "waiting for the launches");
-  for (auto it = contract_packed_.begin(); it != contract_packed_.end();) {
-    if (used.count(it->first)) {
-      ++it;
+    auto reads = [&](std::initializer_list<const Operand *> operands, std::set<std::string> &as) {
+      for (const Operand *op : operands) {
+        if (op->space == Operand::Space::Constant) as.insert(op->name);
+      }
+    };
+    std::set<std::string> &weights = parts != 0 ? packed : raw;
+    if (l.kind == Launch::Kind::Step && !l.rewired) {
+      const Step &s = steps_[l.members[0]];
+      reads({&s.in0}, raw);
+      reads({&s.in1}, weights);
       continue;
     }
-    Check(fluidml_hip_contract_unpack(it->second.device), "freeing packed weights");
-    it = contract_packed_.erase(it);
+    reads({&l.a, &l.c, &l.d, &l.e}, raw);
+    if (l.group.empty()) reads({&l.b}, weights);
+    for (const Launch &m : l.group) {
+      reads({&m.a, &m.c, &m.d, &m.e}, raw);
+      reads({&m.b}, l.kind == Launch::Kind::MatMulGroup ? weights : raw);
+    }
+  }
+  Check(fluidml_hip_stream_synchronize(stream_), "waiting for the launches");
+  auto settle = [&](const std::string &name, void *device, auto &&drop, auto &&adopt) {
+    if (packed.count(name) == 0) {
+      drop();
+      return true;
+    }
+    if (raw.count(name) != 0) return false;
+    ConstantSlot &slot = constants_.at(name);
+    adopt();
+    fluidml_hip_free(slot.device);
+    slot.device = device;
+    slot.packed_only = true;
+    return false;
+  };
+  for (auto it = contract_packed_.begin(); it != contract_packed_.end();) {
+    void *device = it->second.device;
+    const bool dropped = settle(
+        it->first, device, [&] { Check(fluidml_hip_contract_unpack(device), "freeing packed weights"); },
+        [&] { Check(fluidml_hip_contract_adopt(device), "keeping packed weights"); });
+    it = dropped ? contract_packed_.erase(it) : std::next(it);
+  }
+  for (auto it = packed_.begin(); it != packed_.end();) {
+    void *device = it->second.device;
+    const bool dropped = settle(it->first, device, [&] { fluidml_hip_free(device); }, [] {});
+    it = dropped ? packed_.erase(it) : std::next(it);
+  }
+  if (graph_ != nullptr) {  // (its launches hold the addresses)
+    fluidml_hip_graph_destroy(graph_);
+    graph_ = nullptr;
   }
 }
 
@@ -418,8 +456,12 @@ int LaunchPlan::IssuePackedConv(const Step &step, const Operand &weights, const 
   kernel::TensorView c;
   if (bias != nullptr) c = bias->View();
   const bool padded = step.node->GetKind() == flow::OpKind::ConvWithPadding;
-  return fluidml_hip_conv3x3_packed_chain(&in, &w.t, it->second.device, it->second.parts, bias ? &c.t : nullptr, &out,
-                                          padded ? step.node->GetAttrs().pads.data() : nullptr, chain, 0, stream);
+  const int rc = fluidml_hip_conv3x3_packed_chain(&in, &w.t, it->second.device, it->second.parts, bias ? &c.t : nullptr, &out,
+                                                  padded ? step.node->GetAttrs().pads.data() : nullptr, chain, 0, stream);
+  if (rc == FL_ERR_UNSUPPORTED && constants_.at(weights.name).packed_only) {
+    throw std::logic_error("plan: weights " + weights.name + " are packed, their convolution is not");
+  }
+  return rc;
 }
 
 namespace {
@@ -1107,13 +1149,18 @@ size_t LaunchPlan::Run(const std::unordered_map<std::string, void *> &args, size
   return static_cast<size_t>(transfer_->Out(out, stream_)) / epoch;
 }
 
+void LaunchPlan::DecideBranches() {
+  if (branches_decided_) return;
+  branches_decided_ = true;
+  ChooseBranches();
+  SettleWeights();
+}
+
 // Which kernels gain from running beside each other is not something the estimate above can tell (GPT-NeoX: its MLP
 // beside the attention block gains nothing, the next layer's first projections beside an attention block 12 us;
 // ConvBERT loses with every region), so the schedule with its regions and the one without them are both replayed on
 // the first inputs and the faster one stays.
-void LaunchPlan::DecideBranches() {
-  if (branches_decided_) return;
-  branches_decided_ = true;
+void LaunchPlan::ChooseBranches() {
   had_regions_ = !regions_.empty();
   const char *env = std::getenv("FLUIDML_BRANCH_CHECK");
   const bool env_check = env == nullptr || std::strtol(env, nullptr, 10) != 0;

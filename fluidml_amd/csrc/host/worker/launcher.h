@@ -195,7 +195,7 @@ class LaunchPlan {
 
   const std::string &GetName() const { return name_; }
   size_t GetArenaBytes() const { return arena_bytes_; }
-  size_t GetConstantBytes() const;   // constant regions + constants kernels own
+  size_t GetConstantBytes() const;   // constant regions + constants kernels own; without those that are kept packed only
   size_t GetInterfaceBytes() const;  // device staging of graph inputs and outputs
   size_t GetPrivateBytes() const;    // buffers outside the arena: regions no Memory edge uses, outputs of side branches,
                                      // packed weights (once materialised)
@@ -280,6 +280,7 @@ class LaunchPlan {
     Tensor tensor;
     std::vector<size_t> layout;
     void *device = nullptr;
+    bool packed_only = false;  // `device` is the packed form, which packed_ or contract_packed_ owns
   };
   struct RawSlot {
     size_t bytes = 0;
@@ -302,8 +303,9 @@ class LaunchPlan {
   void PackConvWeights();
   // The same for the weights of MatMul and Gemm (fluidml_hip_contract_pack); the library finds them by their address.
   void PackContractionWeights();
-  // Frees those of them that no launch takes, once the tile configurations are picked.
-  void UnpackUnusedWeights();
+  // Once the schedule and its tile configurations are final: frees the packed weights that no launch takes, and the weights
+  // as they stand of which every launch takes the packed form.
+  void SettleWeights();
   // (FL_ERR_UNSUPPORTED, nothing launched, where they are not, or the operands do not fit)
   int IssuePackedConv(const Step &step, const Operand &weights, const fl_tensor &in, const fl_tensor &out,
                       const fl_ew_program *chain, void *stream) const;
@@ -311,6 +313,7 @@ class LaunchPlan {
   void Replay(kernel::LaunchContext &ctx);
   void PlanBranches() const;
   void DecideBranches();
+  void ChooseBranches();
 
   std::string name_;
   size_t arena_bytes_;

@@ -499,6 +499,10 @@ int fluidml_hip_matmul_chain_group_norm(int32_t count, const fl_tensor *lhs, con
  * instruction gives; infinities and NaN do). */
 int fluidml_hip_contract_pack(const fl_tensor *rhs, int32_t trans_b, int64_t rows, int32_t parts, void *stream, void **packed, size_t *bytes);
 int fluidml_hip_contract_unpack(void *packed);
+/* The weights behind `packed` may be freed or changed from here on: their packed form stands for them.  Calls name it by a
+ * tensor of the weights' extents and strides whose address is `packed`; a call that would not take the packed form
+ * returns FL_ERR_UNSUPPORTED. */
+int fluidml_hip_contract_adopt(void *packed);
 /* The parts of the packed weights (contractions and 3x3 convolutions) the calling thread's latest launch against such
  * weights ran with, 0 if there was none since the last call of this function. */
 int fluidml_hip_take_packed_parts(int32_t *parts);
@@ -512,7 +516,7 @@ int fluidml_hip_conv_chain(const fl_tensor *in, const fl_tensor *weights, const 
  * sum of its three parts: fp32 results) or 1 (rounded to bf16: the FL_CONTRACT_BF16 precision).
  * ..._packed_bytes: size of `packed` for these weights (FL_ERR_UNSUPPORTED where there is no such layout); ..._pack
  * fills it, once, on `stream` (FL_ERR_UNSUPPORTED, `packed` unchanged, for values fluidml_hip_contract_pack refuses too);
- * ..._packed_chain runs the convolution, `weights` are the ones that were packed.  `flags`:
+ * ..._packed_chain runs the convolution; of `weights` it takes the extents only, the values are in `packed`.  `flags`:
  * 0, or FL_CONTRACT_TILE(1 | 2) (2 or 4 tiles of 2 x 16 pixels per wave) and FL_CONTRACT_SPLITS(n) instead of the
  * library's rule. */
 int fluidml_hip_conv3x3_packed_bytes(const fl_tensor *weights, int32_t parts, size_t *bytes);

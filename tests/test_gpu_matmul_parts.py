@@ -274,17 +274,109 @@ def test_a_plan_frees_the_packed_weights_no_launch_takes(device, tmp_path, monke
         ex.invoke({**feed, **outs})
         for v, w in zip(net.outputs, want):
             np.testing.assert_allclose(outs[v.name], w, rtol=1e-4, atol=1e-5)
-        return ex, ex.plan()["private_bytes"]
+        plan = ex.plan()
+        assert plan["peak_device_bytes"] == plan["arena_bytes"] + plan["constant_bytes"] + plan["interface_bytes"] + plan["private_bytes"]
+        return ex, plan["private_bytes"], plan["constant_bytes"]
 
-    _, none = compiled("0", "0")
-    ex, both = compiled("0")
-    assert both - none == 768 * (3072 + 2560) * 6
+    _, none, full = compiled("0", "0")
+    ex, both, rest = compiled("0")
+    assert both - none == 768 * (3072 + 2560) * 6 and full - rest == 768 * (3072 + 2560) * 4
     signature = next(sig for sig, _, _ in ex.contraction_choices() if "3072" in sig)
     table = os.path.join(tmp_path, "picks.json")
     with open(table, "w") as f:
         json.dump({signature: {"tile": 2, "splits": 0}}, f)
-    _, one = compiled(table)
-    assert one - none == 768 * 2560 * 6
+    _, one, rest = compiled(table)
+    assert one - none == 768 * 2560 * 6 and full - rest == 768 * 2560 * 4
+
+
+@pytest.mark.parametrize("graph", ["1", "0"])
+def test_weights_that_exist_packed_only(device, tmp_path, monkeypatch, graph):
+    """A plan keeps the one form of its weights that its launches read, both where somebody reads them as they stand; the
+    second pass of what the parts cannot carry works from either."""
+    import os
+
+    from fluidml_amd import fluidml, models
+
+    monkeypatch.setenv("FLUIDML_TUNE", "0")
+    monkeypatch.setenv("FLUIDML_HIP_GRAPH", graph)
+    net = models.Net("forms", 1)
+    x = net.input("x", np.float32, (512, 768))
+    y = net.input("y", np.float32, (768, 2560))
+    few = net.input("few", np.float32, (9, 768))
+    w = [net.normal((768, n)) for n in (3072, 2560, 2816)]
+    net.output(net.matmul(x, w[0]))                    # packed only
+    net.output(net.matmul(net.relu(x), w[1]))
+    net.output(net.add(y, w[1]))                       # as they stand too
+    net.output(net.relu(net.matmul(x, w[2])))
+    net.output(net.matmul(few, w[2]))                  # too few rows for the packed form
+    conv = net.normal((64, 32, 3, 3), std=0.06)
+    img = net.input("img", np.float32, (1, 32, 30, 30))
+    net.output(net.relu(net.conv(img, conv, None, [1, 1], [1, 1, 1, 1])))
+    ex = fluidml.Executor.make_plain_greedy("forms")
+    ex.compile(net.save(os.path.join(tmp_path, "forms.onnx")))
+    plan = ex.plan()
+    assert plan["constant_bytes"] == 768 * (2560 + 2816) * 4
+    assert plan["private_bytes"] >= 768 * (3072 + 2560 + 2816) * 6 + 64 * 32 * 9 * 6
+    rng = np.random.default_rng(2)
+    for turn in range(3):
+        feed = {v.name: rng.standard_normal(v.shape, np.float32) for v in net.inputs}
+        if turn == 1:
+            feed["x"] *= np.float32(1e-37)
+            feed["img"][:] *= np.float32(1e-37)
+        if turn == 2:
+            feed["x"][5, 7], feed["img"][0, 3, 3, 3] = np.inf, np.nan
+        outs = {v.name: np.full(v.shape, 9.0, np.float32) for v in net.outputs}
+        ex.invoke({**feed, **outs})
+        f64 = {k: v.astype(np.float64) for k, v in feed.items()}
+        c = [v.const.astype(np.float64) for v in w]
+        with np.errstate(invalid="ignore"):
+            pad = np.pad(f64["img"][0], ((0, 0), (1, 1), (1, 1)))
+            image = sum(np.tensordot(conv.const[:, :, i, j].astype(np.float64), pad[:, i:i + 30, j:j + 30], 1) for i in range(3) for j in range(3))
+            want = [f64["x"] @ c[0], np.maximum(f64["x"], 0) @ c[1], f64["y"] + c[1], np.maximum(f64["x"] @ c[2], 0), f64["few"] @ c[2],
+                    np.maximum(image, 0)[None]]
+        scale = 1e-37 if turn == 1 else 1.0
+        for i, (v, ref) in enumerate(zip(net.outputs, want)):
+            got, s = outs[v.name], scale if i in (0, 1, 3, 5) else 1.0
+            assert np.array_equal(np.isfinite(got), np.isfinite(ref)), (turn, i)
+            fine = np.isfinite(ref)
+            assert (np.abs(got[fine] - ref[fine]) <= 1e-5 * s + 1e-5 * np.abs(ref[fine])).all(), (turn, i)
+
+
+@pytest.mark.parametrize("tile", TILES)
+def test_adopted_weights(device, tile):
+    """The packed form stands for the weights; calls that would read them as they stood are refused."""
+    for trans_b in (False, True):
+        with Problem(device, 70, 200, 100, trans_b=trans_b) as p:
+            cabi = p.cabi
+            w = p.w[0].t() if trans_b else p.w[0]
+            p.x[3, 7], p.x[69, 199] = float("inf"), float("nan")
+            w[11, 99] = float("-inf")
+            want = p.x.double() @ w.double()
+            tiny = p.x.clone().nan_to_num_(0, 0, 0).abs_() * 1e-36
+            want_tiny = tiny.double() @ w.double()
+            p.pack()
+            cabi.call("contract_adopt", p.packed[0])
+            rhs = cabi.make_tensor(p.packed[0].value, cabi.FL_FLOAT32, p.w[0].shape, p.w[0].stride())
+            p.w[0].fill_(float("nan"))
+            none, zero = ctypes.byref(cabi.make_chain([])), p.torch.zeros(100, device=device)
+
+            def call(x, flags, rows=70):
+                out = p.out()
+                rc = cabi.lib.fluidml_hip_gemm_chain(p.ref(x, (rows, 200)), ctypes.byref(rhs), p.ref(zero), p.ref(out, (rows, 100)), 1.0, 1.0, 0,
+                                                     int(trans_b), none, flags, None)
+                return rc, out
+
+            rc, out = call(p.x, flags_of(tile))
+            assert rc == 0 and p.torch.equal(out.isnan(), want.isnan()) and p.torch.equal(out.isinf(), want.isinf())
+            fine = want.isfinite()
+            close(out[fine], want[fine], "finite results beside infinities")
+            rc, out = call(tiny, flags_of(tile))
+            fine = want_tiny.isfinite()
+            assert rc == 0 and not out[~fine].isfinite().any()
+            # (the weights' signs differ: against sums of magnitudes, about 200 times 0.8 times 0.06)
+            assert ((out[fine].double() - want_tiny[fine]).abs() <= 1e-6 * 10 * 1e-36).all()
+            for flags, rows in ((0, 70), (0, 3), (1 << 4, 70), (3 << 4, 70), (cabi.FL_CONTRACT_BF16, 70)):
+                assert call(p.x, flags, rows)[0] == UNSUPPORTED
 
 
 @pytest.mark.parametrize("M,K,N,count,packed", [
