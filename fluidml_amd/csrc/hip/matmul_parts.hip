@@ -496,10 +496,9 @@ __global__ __launch_bounds__(kPackThreads) void WeightRangeKernel(uint32_t *rang
   }
   low = WaveReduce(low, [](uint32_t x, uint32_t y) { return min(x, y); });
   high = WaveReduce(high, [](uint32_t x, uint32_t y) { return max(x, y); });
-  if (threadIdx.x % kWave == 0) {
-    atomicMin(range, low);
-    atomicMax(range + 1, high);
-  }
+  // (all waves of a large matrix at one address took 99 us; a stale value here only costs the atomic it was to spare)
+  if (threadIdx.x % kWave == 0 && low < __hip_atomic_load(range, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(range, low);
+  if (threadIdx.x % kWave == 0 && high > __hip_atomic_load(range + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(range + 1, high);
 }
 
 // ---- which weights have a packed form -----------------------------------------------------------------------------
