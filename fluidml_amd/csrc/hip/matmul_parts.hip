@@ -627,20 +627,26 @@ int LaunchPacked(const MatmulArgs &args, uint32_t n_batch, bool extra, int parts
   int tile = choice.tile, splits = choice.splits > 0 ? choice.splits : 1;
   if (tile == FL_TILE_RULE) {
     if (choice.splits != 0 || !WorthPacking(p.M, static_cast<int64_t>(p.N) * std::max(1, p.n_groups), p.K, parts)) return FL_ERR_UNSUPPORTED;
-    // 64x128 tiles while they give two thirds of the compute units a workgroup (four waves each from one per compute unit
-    // on: two of them fit one then), else smaller ones, and K split over workgroups where it is long (measured, us: K = 768,
-    // 512 x 3072: 64x128_K2 21.2, 64x128 23.2, 64x64 23.8; 256 x 3072: 64x64 15.9, 64x128_K2 with two splits 17.0; 512 x
-    // 768: 32x64 9.2, the others above 11; K = 3072, 512 x 768: 64x128_K2 with four splits 24.7, 64x64 with four 26.0;
-    // K = 512, 256 x 50304: 64x128 93, 64x64 106, both with two K slices 118).
+    // One workgroup per compute unit is the aim.  More 64x128 tiles than compute units: four waves each, two of them fit one.
+    // Half as many and more: eight waves each (a second K slice).  Fewer: K split over workgroups until they fill the chip,
+    // from a length on at which the exchange of the partial tiles pays; below it smaller tiles.  Measured (us):
+    //   three parts  512x3072, K = 768: 64x128_K2 21.8, 64x128 23.6, 64x64 24.9; 256x50304, K = 512: 64x128 94, 64x64 106, K2 124;
+    //                512x4096, K = 4096 (256 tiles): K2 98, 64x128 112
+    //                256x3072, K = 768: 64x64 16.1, K2 in two 17.3; 256x4096, K = 1024: 64x64 20.8, K2 in two 22.4, in one 26.6;
+    //                640x1280, K = 1280: 22.5 both; 512x2048, K = 2048: K2 in two 32.7, 64x64 35.4, K2 in one 44.5
+    //                256x4096: K = 4096 K2 in two 55, in one 81, K = 11008 137, 223; 512x1024, K = 4096: K2 in four 33.1, in three 36.5
+    //                512x768, K = 3072: K2 in four 24.9, 64x64 in four 26.7; 256x2048, K = 2048: K2 in three 23.3, in four 24.1
+    //   one part     512x768, K = 3072 (192 tiles of 32x64): 32x64 14.9, K2 in four 14.6; 256x4096, K = 4096 (512): K2 in two 26.6, in
+    //                one 36.3; 640x1280, K = 5120 (400): K2 in two 29, 32x64 38; 256x4096, K = 1024: 32x64 10.1, K2 10.7
     auto tiles = [&](int bm, int bn) { return static_cast<int64_t>((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn) * n_batch; };
     const int64_t t128 = tiles(64, 128), t64 = tiles(64, 64), t32 = tiles(32, 64);
-    if (t128 >= 256) {
+    if (t128 > 256) {
       tile = FL_TILE_PACKED_64x128;
-    } else if (t128 >= 128) {
+    } else if (t128 > 128) {
       tile = FL_TILE_PACKED_64x128_K2;
-    } else if (parts == 3 && p.K >= 2048 && t128 >= 32) {
+    } else if (parts == 3 ? p.K >= 1280 && t128 >= 32 : p.K >= 2048 && t32 > 256) {
       tile = FL_TILE_PACKED_64x128_K2;
-      splits = static_cast<int>(std::min<int64_t>(192 / t128, 4));
+      splits = static_cast<int>(std::min<int64_t>({256 / t128, 4, p.K / 640}));
     } else if (parts == 3 && t64 >= 144) {
       tile = FL_TILE_PACKED_64x64;
     } else {

@@ -250,6 +250,30 @@ def test_weights_the_parts_cannot_carry_are_not_packed(device, element, value):
         p.pack()
 
 
+@pytest.mark.parametrize("M,K,N", [  # 64x128 tiles times splits of the rule
+    (77, 768, 16512),                   # more than 256
+    (256, 640, 8192), (192, 768, 5504),  # 256, 129
+    (256, 1280, 4096), (256, 1272, 4096),  # 128 x 2, the next shorter K
+    (150, 1920, 4000), (140, 2560, 2048), (68, 2560, 4224),  # 96 x 2, 48 x 4, 66 x 3
+    (96, 1288, 2060),                   # not packed in three parts
+])
+def test_packed_tiles_of_the_rule(device, M, K, N):
+    for parts in (3, 1):
+        with Problem(device, M, K, N) as p:
+            x, w = (p.x, p.w[0]) if parts == 3 else (p.x.bfloat16(), p.w[0].bfloat16())
+            want = x.double() @ w.double() + p.b[0].double()
+            p.pack(parts)
+            got = ctypes.c_int32()
+            p.cabi.call("take_packed_parts", ctypes.byref(got))
+            print("[case]", M, K, N, parts, flush=True)
+            for _ in range(2):
+                out = p.out()
+                assert p.chain(out, 0 if parts == 3 else p.cabi.FL_CONTRACT_BF16) == 0
+                close(out, want, f"{parts} parts")
+            p.cabi.call("take_packed_parts", ctypes.byref(got))
+            assert got.value == (parts if parts == 1 or (M * N >= 280000 and float(M) * K * N >= 5.8e8) else 0)
+
+
 def test_a_plan_frees_the_packed_weights_no_launch_takes(device, tmp_path, monkeypatch):
     """The tile configuration of a contraction is picked after its weights have been packed."""
     import json
