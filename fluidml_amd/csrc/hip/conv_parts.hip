@@ -12,8 +12,8 @@
 //     TN = 4), and the next two taps' loads are in flight;
 //   * the input patch of 16 channels is split into its parts once per workgroup, on its way into LDS, where it lies as
 //     [part][channel half][pixel][8 channels]: a lane's B operand is one 128-bit read at a per-lane base plus a
-//     compile-time offset, consecutive pixels in consecutive 16-byte places (no bank conflicts), and a row of the
-//     patch serves all the taps;
+//     compile-time offset, consecutive pixels in consecutive 16-byte places, and a row of the patch serves all the
+//     taps (3.8 conflict cycles per LDS instruction, reads and writes of 16 bytes per lane together);
 //   * per chunk of 16 channels one barrier, TN x 54 products per wave; LDS is double buffered and the next chunk's
 //     loads are in flight across the products;
 //   * the loads that run ahead are held in their place by scheduling barriers (the compiler moves them down to their use);
