@@ -1616,6 +1616,10 @@ int Contract(const fl_tensor *lhs, const fl_tensor *rhs, const fl_tensor *out, b
     if (choice.tile != FL_TILE_RULE) return rc;
   }
   if (only_packed) return FL_ERR_UNSUPPORTED;
+  if ((!bf16 || k_scale != nullptr) && free_choice) {  // (a scale per row of B: fp32 in any case, see below)
+    rc = LaunchRows(p, nb, extra, C, A, B, s);
+    if (rc != FL_ERR_UNSUPPORTED) return rc != FL_OK ? rc : LaunchStatus();
+  }
   if (extra) {
 #define FL_MM_EXTRA(E_)                                                                 \
   do {                                                                                  \

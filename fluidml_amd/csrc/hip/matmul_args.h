@@ -110,6 +110,10 @@ struct TileChoice {
 int LaunchPacked(const MatmulArgs &p, uint32_t n_batch, bool extra, int parts, float *C, const float *A, const float *B,
                  hipStream_t s, TileChoice choice);
 
+// matmul_rows.hip: the contraction of few rows and short sums.  FL_ERR_UNSUPPORTED, with nothing launched, where the operands
+// do not fit or its rule leaves the problem to the other kernels.
+int LaunchRows(const MatmulArgs &p, uint32_t n_batch, bool extra, float *C, const float *A, const float *B, hipStream_t s);
+
 // Whether B, or that of a member, exists in its packed form only: no other kernel can read it.
 bool OnlyPacked(const MatmulArgs &p, const float *B);
 
