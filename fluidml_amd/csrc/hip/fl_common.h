@@ -149,7 +149,8 @@ __device__ __forceinline__ void SplitParts(const float (&x)[8], u32x4 (&parts)[P
     float a = x[2 * i], b = x[2 * i + 1];
 #pragma unroll
     for (int q = 0; q < PARTS; ++q) {
-      const uint32_t packed = __builtin_bit_cast(uint32_t, bf16x2{static_cast<__bf16>(a), static_cast<__bf16>(b)});
+      uint32_t packed = __builtin_bit_cast(uint32_t, bf16x2{static_cast<__bf16>(a), static_cast<__bf16>(b)});
+      if (q + 1 < PARTS) asm("" : "+v"(packed));  // (one conversion for both uses: the compiler makes a second one of each half)
       parts[q][i] = packed;
       a -= __builtin_bit_cast(float, packed << 16);
       b -= __builtin_bit_cast(float, packed & 0xffff0000u);
