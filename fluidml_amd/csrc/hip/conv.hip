@@ -244,6 +244,10 @@ int ConvImplicitGemm(const fl_tensor *in, const fl_tensor *weights, const fl_ten
 int ConvHalo3x3(const fl_tensor *in, const fl_tensor *weights, const fl_tensor *bias, const fl_tensor *out,
                 const int64_t *pads, const int64_t *strides, const int64_t *dilations, const fl_ew_program *chain,
                 void *stream, bool bf16);  // conv_halo.hip
+bool ConvHaloEnabled();
+
+int ConvShort(const fl_tensor *in, const fl_tensor *weights, const fl_tensor *bias, const fl_tensor *out, const int64_t *pads,
+              const int64_t *strides, const int64_t *dilations, const fl_ew_program *chain, void *stream);  // conv_short.hip
 
 namespace {
 
@@ -341,6 +345,13 @@ int Conv(const fl_tensor *in, const fl_tensor *weights, const fl_tensor *bias, c
     return ConvImplicitGemm(in, weights, bias, out, pads, strides, dilations, chain, bf16, stream, extras);
   }
   if (!depthwise && flags == 0 && ns == 2) {
+    // sums of at most 32 terms (with the opt-in bf16 precision only the kind that the next kernel leaves in fp32)
+    const bool unit_3x3 = p.k_shape[0] == 3 && p.k_shape[1] == 3 && p.stride[0] == 1 && p.stride[1] == 1 && p.dilation[0] == 1 &&
+                          p.dilation[1] == 1;
+    if (ConvHaloEnabled() && (!bf16 || (unit_3x3 && F >= 32))) {
+      const int rc = ConvShort(in, weights, bias, out, pads, strides, dilations, chain, stream);
+      if (rc != FL_ERR_UNSUPPORTED) return rc;
+    }
     // 3x3, unit stride: the input patch is staged once per workgroup instead of gathered tap by tap (with bf16
     // operands where they are allowed and the channels come in chunks of 16, else fp32)
     const int rc = ConvHalo3x3(in, weights, bias, out, pads, strides, dilations, chain, stream, bf16);

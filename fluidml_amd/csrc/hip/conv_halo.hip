@@ -74,9 +74,9 @@ struct HaloArgs {
 
 // NV: pixel tiles (4 rows x 8 columns each) a wave owns, one below the other: the workgroup covers 4 NV x 16 pixels.
 // With two, the weights a wave reads from LDS serve twice the products and a barrier separates twice the work.
-// FEW: fewer than eight input channels (the first layer of an image network): one chunk whose missing channels read
-// as zero; the filters' rows are then shorter than a chunk and not 16-byte aligned, so the weights are loaded
-// value by value.
+// FEW: fewer than eight input channels (the first layer of an image network, where conv_short.hip does not take it): one
+// chunk whose missing channels read as zero; the filters' rows are then shorter than a chunk and not 16-byte aligned, so
+// the weights are loaded value by value.
 template <int NV, bool FEW>
 __global__ __launch_bounds__(kThreads) void ConvHalo3x3Kernel(float *__restrict__ out, const float *__restrict__ in,
                                                               const float *__restrict__ weights, HaloArgs p) {
@@ -498,20 +498,20 @@ __global__ __launch_bounds__(kThreads) void ConvHalo3x3Bf16Kernel(float *__restr
   }
 }
 
+}  // namespace
+
 // Environment FLUIDML_CONV_HALO=0 keeps every convolution on the implicit-GEMM path.
-bool HaloEnabled() {
+bool ConvHaloEnabled() {
   const char *v = std::getenv("FLUIDML_CONV_HALO");  // (read at every call)
   return v == nullptr || std::strtol(v, nullptr, 10) != 0;
 }
-
-}  // namespace
 
 // FL_ERR_UNSUPPORTED (nothing launched) when the convolution does not fit this kernel: the caller goes on to the
 // implicit-GEMM path.  Operands were validated by the caller.
 int ConvHalo3x3(const fl_tensor *in, const fl_tensor *weights, const fl_tensor *bias, const fl_tensor *out,
                 const int64_t *pads, const int64_t *strides, const int64_t *dilations, const fl_ew_program *chain,
                 void *stream, bool bf16) {
-  if (!HaloEnabled() || out->rank != 4) return FL_ERR_UNSUPPORTED;
+  if (!ConvHaloEnabled() || out->rank != 4) return FL_ERR_UNSUPPORTED;
   if (weights->shape[2] != 3 || weights->shape[3] != 3) return FL_ERR_UNSUPPORTED;
   for (int d = 0; d < 2; ++d) {
     if ((strides && strides[d] != 1) || (dilations && dilations[d] != 1)) return FL_ERR_UNSUPPORTED;
