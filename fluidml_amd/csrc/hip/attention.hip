@@ -11,7 +11,7 @@
 //   1. scores, transposed: v_mfma_f32_16x16x4_f32 with the keys as rows and the queries as columns.  A lane feeds it
 //      K^T[d][key lane % 16] and Q[query lane % 16][d] and receives the scores of ITS query (lane % 16) with the keys
 //      16 t + 4 (lane / 16) + i of every key tile t.
-//   2. scale, mask, condition, and the maximum over the wave's own keys: registers and two shuffles.
+//   2. scale, mask, condition, and the maximum over the wave's own keys: registers and two swaps of rows.
 //   3. context, transposed: the product with V^T (head columns as rows, queries as columns) wants of a lane
 //      P[key 4 (lane / 16) + i][query lane % 16] in step i -- register i of the scores as they lie.
 //   4. every wave leaves its context, its maximum and its sum of exponentials in LDS; after the only barrier the
@@ -179,8 +179,7 @@ __global__ __launch_bounds__(64 * NW) void AttentionKernel(AttentionArgs a, floa
       s[t][i] = y;
       mx = fmaxf(mx, y);
     }
-  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+  mx = AcrossHalves(AcrossRows(mx, MaxOp{}), MaxOp{});
   float sum = 0.0f;
 #pragma unroll
   for (int t = 0; t < KT; ++t)
@@ -189,8 +188,7 @@ __global__ __launch_bounds__(64 * NW) void AttentionKernel(AttentionArgs a, floa
       s[t][i] = key(t, 4 * grp + i) <= last_key ? expf(s[t][i] - mx) : 0.0f;
       sum += s[t][i];
     }
-  sum += __shfl_xor(sum, 16, 64);
-  sum += __shfl_xor(sum, 32, 64);
+  sum = AcrossHalves(AcrossRows(sum, SumOp{}), SumOp{});
 
   // ---- the wave's context --------------------------------------------------------------------------------------------
   floatx4 o[DT];

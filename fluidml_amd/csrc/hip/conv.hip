@@ -588,8 +588,7 @@ __global__ __launch_bounds__(kBlock) void PointwiseOnePixelKernel(int32_t channe
   } else {
     for (int c = lane; c < channels; c += LANES) acc += row[c * w_c] * x[c * in_c];
   }
-#pragma unroll
-  for (int off = LANES / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, kWave);
+  acc = GroupReduce<LANES>(acc, SumOp{});
   if (live && lane == 0) {
     if (b != nullptr) acc += b[f * b_stride];
     if (chain.n != 0) acc = RunChain(chain, acc);

@@ -561,17 +561,41 @@ inline NestArgs<NOPS> MakeNestArgs(const LoopNest &nest) {
 // ---- device-side reductions -------------------------------------------------
 
 #if defined(__HIPCC__)
-// The value of another lane through the data-parallel-primitive path of the vector ALU (a few cycles, against the
-// round trip through the LDS crossbar that a shuffle by lane index costs).  `CTRL`: 0xB1 / 0x4E swap neighbours /
-// pairs inside every four lanes, 0x141 / 0x140 mirror every 8 / 16 lanes.
-template <int CTRL>
-__device__ __forceinline__ float DppMove(float v) {
+// Values of other lanes without the LDS crossbar: a shuffle by lane index goes through it and takes its round trip, more than
+// a hundred cycles in a chain of six.  The vector ALU reads other lanes of a row of sixteen as it moves a value (`CTRL`: 0xB1 /
+// 0x4E swap neighbours / pairs inside every four lanes, 0x141 / 0x140 mirror every 8 / 16 lanes, 0x128 turns a row by eight), and
+// swaps rows, or halves of the wave, between two registers.  Every lane that takes part has to be active.
+template <int CTRL, typename T>
+__device__ __forceinline__ T DppMove(T v) {
+  static_assert(sizeof(T) == 4, "a register");
   const int bits = __builtin_bit_cast(int, v);
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(bits, bits, CTRL, 0xf, 0xf, false));
+  return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(bits, bits, CTRL, 0xf, 0xf, false));
 }
 
+// f(v of rows 0 and 2, v of rows 1 and 3), to the lanes of both
+template <typename T, typename F>
+__device__ __forceinline__ T AcrossRows(T v, F f) {
+  static_assert(sizeof(T) == 4, "a register");
+  const uint32_t bits = __builtin_bit_cast(uint32_t, v);
+  const auto both = __builtin_amdgcn_permlane16_swap(bits, bits, false, false);
+  const uint32_t first = both[0], second = both[1];  // (a bit cast of an element of a vector reads the first one)
+  return f(__builtin_bit_cast(T, first), __builtin_bit_cast(T, second));
+}
+// f(v of the lower half of the wave, v of the upper half), to both
+template <typename T, typename F>
+__device__ __forceinline__ T AcrossHalves(T v, F f) {
+  static_assert(sizeof(T) == 4, "a register");
+  const uint32_t bits = __builtin_bit_cast(uint32_t, v);
+  const auto both = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
+  const uint32_t first = both[0], second = both[1];  // (a bit cast of an element of a vector reads the first one)
+  return f(__builtin_bit_cast(T, first), __builtin_bit_cast(T, second));
+}
+
+struct SumOp {
+  __device__ __forceinline__ float operator()(float a, float b) const { return a + b; }
+};
+
 // Sum over every aligned group of W consecutive lanes (W a power of two), delivered to all lanes of the group.
-// Every lane of the wave has to be active.
 template <int W>
 __device__ __forceinline__ float GroupSum(float v) {
   static_assert(W >= 1 && W <= kWave && (W & (W - 1)) == 0, "groups are powers of two");
@@ -579,23 +603,29 @@ __device__ __forceinline__ float GroupSum(float v) {
   if constexpr (W >= 4) v += DppMove<0x4E>(v);
   if constexpr (W >= 8) v += DppMove<0x141>(v);
   if constexpr (W >= 16) v += DppMove<0x140>(v);
-  if constexpr (W >= 32) v += __shfl_xor(v, 16, kWave);
-  if constexpr (W >= 64) v += __shfl_xor(v, 32, kWave);
+  if constexpr (W >= 32) v = AcrossRows(v, SumOp{});
+  if constexpr (W >= 64) v = AcrossHalves(v, SumOp{});
+  return v;
+}
+
+// The same for any associative and commutative f, the far lanes first.
+template <int W, typename T, typename F>
+__device__ __forceinline__ T GroupReduce(T v, F f) {
+  static_assert(W >= 1 && W <= kWave && (W & (W - 1)) == 0, "groups are powers of two");
+  if constexpr (W >= 64) v = AcrossHalves(v, f);
+  if constexpr (W >= 32) v = AcrossRows(v, f);
+  if constexpr (W >= 16) v = f(v, DppMove<0x128>(v));
+  if constexpr (W >= 8) v = f(v, DppMove<0x141>(v));
+  if constexpr (W >= 4) v = f(v, DppMove<0x4E>(v));
+  if constexpr (W >= 2) v = f(v, DppMove<0xB1>(v));
   return v;
 }
 
 template <typename T, typename F>
 __device__ __forceinline__ T WaveReduce(T v, F f) {
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) {
-    v = f(v, __shfl_xor(v, off, kWave));
-  }
-  return v;
+  return GroupReduce<kWave>(v, f);
 }
 
-struct SumOp {
-  __device__ __forceinline__ float operator()(float a, float b) const { return a + b; }
-};
 struct MaxOp {
   __device__ __forceinline__ float operator()(float a, float b) const { return fmaxf(a, b); }
 };

@@ -137,13 +137,6 @@ struct alignas(16) Quad {
   float v[4];
 };
 
-template <int LANES, typename F>
-__device__ __forceinline__ float GroupReduce(float v, F f) {
-#pragma unroll
-  for (int off = LANES / 2; off > 0; off >>= 1) v = f(v, __shfl_xor(v, off, kWave));
-  return v;
-}
-
 template <int LANES, int ITEMS>
 __global__ __launch_bounds__(kBlock) void SoftmaxRowVec(RowArgs<3> a, float *__restrict__ out,
                                                         const float *__restrict__ in, SoftmaxPre pre) {
@@ -397,13 +390,11 @@ __global__ __launch_bounds__(kBlock) void GatherStatsKernel(uint32_t len, int64_
     const uint32_t first = j & ~31u;
     const float cols = static_cast<float>(first < len ? min(32u, len - first) : 1u);
     float sum = x;
-#pragma unroll
-    for (int o = 16; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+    sum = GroupReduce<32>(sum, SumOp{});
     const float mean = sum / cols;
     const float d = in ? x - mean : 0.0f;
     float sq = d * d;
-#pragma unroll
-    for (int o = 16; o > 0; o >>= 1) sq += __shfl_xor(sq, o, 64);
+    sq = GroupReduce<32>(sq, SumOp{});
     if ((threadIdx.x & 31u) == 0 && in) {
       float *at = stats + (static_cast<size_t>(row) * parts + j / 32) * 2;
       at[0] = mean;
