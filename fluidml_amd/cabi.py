@@ -179,6 +179,7 @@ SIGNATURES = {
     "fluidml_hip_conv3x3_packed_bytes": [_T, _i32, _P(_sz)],
     "fluidml_hip_conv3x3_pack": [_T, _i32, _vp, _vp],
     "fluidml_hip_conv3x3_packed_chain": [_T, _T, _vp, _i32, _T, _T, _i64p, _vp, _u32, _vp],
+    "fluidml_hip_conv3x3_packed_chain_pool": [_T, _T, _vp, _i32, _T, _T, _i64p, _vp, _u32, _vp],
     "fluidml_hip_conv_chain_scale_add": [_T, _T, _T, _T, _i64p, _i64p, _i64p, _i64, _vp, _T, _T, _u32, _vp],
     "fluidml_hip_conv_chain_mean": [_T, _T, _T, _T, _i64p, _i64p, _i64p, _i64, _vp, _T, _u32, _vp],
     "fluidml_hip_pointwise_conv_pair": [_T, _T, _T, _vp, _T, _T, _vp, _T, _vp],

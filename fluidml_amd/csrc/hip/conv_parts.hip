@@ -28,6 +28,9 @@
 //   8 x 512 x  14^2 -> 512                      92 ->  50 (147)               35 -> 27 (276)
 //   1 x 256 x  56^2 -> 256                      52 ->  31 (118)               23 -> 16 (230)
 //   4 x 256 x  37^2 -> 256                     156 ->  46 (142)              106 -> 20 (327)
+// A 2 x 2 pool behind the chain is taken in the epilogue, where neighbouring lanes hold whole windows: a quarter of the result
+// is written and nothing read back (us, convolution and pool): 8 x 64 x 224^2 fp32 166 + 18 -> 162, bf16 70 + 18 -> 64;
+// 8 x 256 x 56^2 fp32 158 + 6 -> 153; the five pools of VGG-16 at batch 8 43 -> 0 altogether.
 // (the tiles of 28^2 and 56^2 images are seven eighths full: 220 TFLOP/s of the 287 the instructions reach alone)
 #include <algorithm>
 
@@ -53,6 +56,7 @@ struct PartsArgs {
   uint32_t n_splits;
   int32_t chunks_per_split;
   int32_t weight_major;  // consecutive workgroups share weights (else: the patch)
+  int32_t pooled;        // the result is the maximum of each 2 x 2 pixels (the strides are the pooled tensor's)
   const float *bias;
   int32_t sB;
   float *partials;
@@ -302,6 +306,38 @@ __global__ __launch_bounds__(kThreads, 2) void ConvPartsKernel(float *out, const
 #pragma unroll
     for (int e = 0; e < 16; ++e) vals[e] = acc[j][e] + bias_v[e];
     if (p.chain.n != 0) RunChainBlock<16>(p.chain, vals);
+    if (p.pooled) {
+      // The four pixels of a window are a lane's neighbour and the two in the next row of sixteen.  Each exchange halves the
+      // filters a lane goes on with instead of computing every maximum twice, and all lanes store in the end: lane r of
+      // the upper (0) and the lower row (1), column parity c, has the filters e = 4 k + 2 r + c.
+      float rows[8], four[4];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        // (e = 4 (k / 2) + k % 2 stays with the upper row, the one two further with the lower)
+        const int e = k / 2 * 4 + k % 2;
+        const uint32_t a = __builtin_bit_cast(uint32_t, vals[e]), b = __builtin_bit_cast(uint32_t, vals[e + 2]);
+        const auto both = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+        const uint32_t first = both[0], second = both[1];
+        rows[k] = MaximumF(__builtin_bit_cast(float, first), __builtin_bit_cast(float, second));
+      }
+      const bool odd = (lane & 1) != 0;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float keep = odd ? rows[2 * k + 1] : rows[2 * k], give = odd ? rows[2 * k] : rows[2 * k + 1];
+        four[k] = MaximumF(keep, DppMove<0xB1>(give));
+      }
+      // (an odd last row or column belongs to no window)
+      const int row = oh / 2, col = ow / 2;
+      if (row < p.OH / 2 && col < p.OW / 2) {
+        float *dst = out + static_cast<int64_t>(img) * p.sOn + static_cast<int64_t>(row) * p.sOh + static_cast<int64_t>(col) * p.sOw;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int f = ftile * 32 + k * 8 + half * 4 + lrow / 16 * 2 + (lane & 1);
+          if (f < p.F) dst[static_cast<int64_t>(f) * p.sOf] = four[k];
+        }
+      }
+      return;
+    }
     if (oh < p.OH && ow < p.OW) {
       float *dst = out + static_cast<int64_t>(img) * p.sOn + static_cast<int64_t>(oh) * p.sOh + static_cast<int64_t>(ow) * p.sOw;
 #pragma unroll
@@ -422,9 +458,9 @@ int fluidml_hip_conv3x3_pack(const fl_tensor *weights, int32_t parts, void *pack
   return LaunchStatus();
 }
 
-int fluidml_hip_conv3x3_packed_chain(const fl_tensor *in, const fl_tensor *weights, const void *packed, int32_t parts,
-                                     const fl_tensor *bias, const fl_tensor *out, const int64_t *pads,
-                                     const fl_ew_program *chain, uint32_t flags, void *stream) {
+static int PackedChain(const fl_tensor *in, const fl_tensor *weights, const void *packed, int32_t parts, const fl_tensor *bias,
+                       const fl_tensor *out, const int64_t *pads, const fl_ew_program *chain, uint32_t flags, bool pooled,
+                       void *stream) {
   using namespace fl;
   FL_CHECK(CheckChain(chain));
   FL_CHECK(CheckView(in));
@@ -438,14 +474,16 @@ int fluidml_hip_conv3x3_packed_chain(const fl_tensor *in, const fl_tensor *weigh
   if (!Fits(weights)) return FL_ERR_UNSUPPORTED;
   const int64_t N = in->shape[0], C = in->shape[1], F = out->shape[1];
   if (out->shape[0] != N || weights->shape[0] != F || weights->shape[1] != C) return FL_ERR_SHAPE;
+  int64_t extent[2];
   for (int d = 0; d < 2; ++d) {
     const int64_t before = pads ? pads[d] : 0, after = pads ? pads[d + 2] : 0;
     if (before < 0 || after < 0) return FL_ERR_ATTR;
     if (before > 0x3fffffff) return FL_ERR_TOO_LARGE;
     // (the whole output and nothing else: a smaller one would be a convolution with other strides or dilations, or a crop)
-    if (out->shape[2 + d] != in->shape[2 + d] + before + after - 2) return FL_ERR_SHAPE;
+    extent[d] = in->shape[2 + d] + before + after - 2;
+    if (out->shape[2 + d] != (pooled ? extent[d] / 2 : extent[d])) return FL_ERR_SHAPE;
   }
-  if (Numel(in) > 0x7fffffff || Numel(out) > 0x7fffffff) return FL_ERR_UNSUPPORTED;
+  if (Numel(in) > 0x7fffffff || N * F * extent[0] * extent[1] > 0x7fffffff) return FL_ERR_UNSUPPORTED;
   for (int d = 0; d < 4; ++d) {
     // (byte offsets inside an image are 32-bit)
     if (in->strides[d] < 0 || in->strides[d] * (in->shape[d] + kChunk) > 0x3fffffff || out->strides[d] > 0x7fffffff) return FL_ERR_UNSUPPORTED;
@@ -453,7 +491,8 @@ int fluidml_hip_conv3x3_packed_chain(const fl_tensor *in, const fl_tensor *weigh
   PartsArgs p;
   std::memset(&p, 0, sizeof(p));
   p.C = static_cast<int32_t>(C), p.H = static_cast<int32_t>(in->shape[2]), p.W = static_cast<int32_t>(in->shape[3]);
-  p.F = static_cast<int32_t>(F), p.OH = static_cast<int32_t>(out->shape[2]), p.OW = static_cast<int32_t>(out->shape[3]);
+  p.F = static_cast<int32_t>(F), p.OH = static_cast<int32_t>(extent[0]), p.OW = static_cast<int32_t>(extent[1]);
+  p.pooled = pooled ? 1 : 0;
   p.ph = pads ? static_cast<int32_t>(pads[0]) : 0, p.pw = pads ? static_cast<int32_t>(pads[1]) : 0;
   p.chunks = static_cast<int32_t>(Ceil(C, kChunk)), p.ftiles = static_cast<int32_t>(Ceil(F, 32));
   p.sXn = static_cast<int32_t>(in->strides[0]), p.sXc = static_cast<int32_t>(in->strides[1]);
@@ -505,6 +544,18 @@ int fluidml_hip_conv3x3_packed_chain(const fl_tensor *in, const fl_tensor *weigh
 #undef FL_PARTS
   NotePackedParts(parts);
   return LaunchStatus();
+}
+
+int fluidml_hip_conv3x3_packed_chain(const fl_tensor *in, const fl_tensor *weights, const void *packed, int32_t parts,
+                                     const fl_tensor *bias, const fl_tensor *out, const int64_t *pads,
+                                     const fl_ew_program *chain, uint32_t flags, void *stream) {
+  return PackedChain(in, weights, packed, parts, bias, out, pads, chain, flags, false, stream);
+}
+
+int fluidml_hip_conv3x3_packed_chain_pool(const fl_tensor *in, const fl_tensor *weights, const void *packed, int32_t parts,
+                                          const fl_tensor *bias, const fl_tensor *out, const int64_t *pads,
+                                          const fl_ew_program *chain, uint32_t flags, void *stream) {
+  return PackedChain(in, weights, packed, parts, bias, out, pads, chain, flags, true, stream);
 }
 
 }  // extern "C"

@@ -626,6 +626,13 @@ __device__ __forceinline__ T WaveReduce(T v, F f) {
   return GroupReduce<kWave>(v, f);
 }
 
+// arith.maximumf: a NaN stays one
+__device__ __forceinline__ float MaximumF(float a, float b) {
+  float r = fmaxf(a, b);
+  if (a != a) r = a;
+  if (b != b) r = b;
+  return r;
+}
 struct MaxOp {
   __device__ __forceinline__ float operator()(float a, float b) const { return fmaxf(a, b); }
 };

@@ -20,13 +20,6 @@ struct PoolArgs {
   uint32_t n_window;
 };
 
-__device__ __forceinline__ float MaximumF(float a, float b) {
-  float r = fmaxf(a, b);
-  if (a != a) r = a;
-  if (b != b) r = b;
-  return r;
-}
-
 template <bool IS_MAX>
 __global__ __launch_bounds__(kBlock) void PoolKernel(PoolArgs p, float *__restrict__ out,
                                                      const float *__restrict__ in) {

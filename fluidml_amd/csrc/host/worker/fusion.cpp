@@ -1265,6 +1265,7 @@ class Scheduler {
     if (l.kind == Launch::Kind::ConvChain) {
       if (auto wider = WithGateAndSkip(i, l)) return wider;
       if (auto wider = WithMean(i, l)) return wider;
+      if (auto wider = WithPool(i, l)) return wider;
     }
     // longest variant whose late reads are safe: with the chain, then without it
     for (int attempt = 0; attempt < 2; ++attempt) {
@@ -1384,6 +1385,47 @@ class Scheduler {
     if (!Safe(l.members, {{i, l.a}, {i, l.b}}) || (clash && !Movable(l.out)) || !OutputDisjoint(l.out2, {&l.a, &l.b, &l.out})) return std::nullopt;
     if (clash) pending_moves_.push_back(l.out.name);
     l.bytes = Bytes({&l.a, &l.b, &l.out}) + static_cast<double>(steps_[i].kernel->GetConstantBytes()) + static_cast<double>(l.out2.meta.GetSize());
+    l.flops = Flops(l.members);
+    return l;
+  }
+
+  // A dense 3x3 convolution of unit stride (with the chain already matched in `plain`) whose only reader is a MaxPool of 2 x 2
+  // windows: the kernel against packed weights holds whole windows in neighbouring lanes and writes their maxima.  Environment
+  // FLUIDML_CONV_POOL=0 (read at every compile) keeps the pools separate.
+  std::optional<Launch> WithPool(size_t i, const Launch &plain) {
+    if (const char *v = std::getenv("FLUIDML_CONV_POOL"); v != nullptr && std::string(v) == "0") return std::nullopt;
+    const flow::Attrs &at = Attrs(i);
+    const auto &w_shape = steps_[i].in1.meta.GetShape();
+    const std::vector<int64_t> ones{1, 1}, twos{2, 2};
+    // (the layers that the launch plan packs: with fewer than sixteen channels it does not)
+    if (plain.b.space != Operand::Space::Constant || plain.b.viewed || w_shape.size() != 4 || w_shape[0] < 32 || w_shape[1] < 16 ||
+        w_shape[2] != 3 || w_shape[3] != 3 || at.group != 1 || at.strides != ones || at.dilations != ones) {
+      return std::nullopt;
+    }
+    const size_t value = plain.members.back();
+    const auto pool = SoleReader(value);
+    if (!pool || Kind(*pool) != OpKind::MaxPoolWithoutPadding || Attrs(*pool).kernel_shape != twos || Attrs(*pool).strides != twos) {
+      return std::nullopt;
+    }
+    Launch l = plain;
+    l.members.push_back(*pool);
+    l.out = steps_[*pool].out;
+    l.whole = steps_[value].out;
+    l.pooled = true;
+    if (!IsFloat(l.out) || !IsFloat(l.whole) || l.a.viewed) return std::nullopt;
+    // (what the kernel against packed weights addresses: 31 bits of bytes inside an image and a channel block more, 31 of elements)
+    const std::vector<int64_t> &shape = l.a.meta.GetShape(), strides = utils::GenStrides(shape, l.a.layout);
+    for (size_t d = 0; d < shape.size(); ++d) {
+      if (strides[d] * (shape[d] + 16) > 0x3fffffff) return std::nullopt;
+    }
+    if (l.whole.meta.GetSize() / sizeof(float) > 0x7fffffff) return std::nullopt;
+    // (the plan may put the pooled tensor over the convolution's input, dead by then in the plan but read by this launch)
+    const bool clash = !OutputDisjoint(l.out, {&l.a, &l.b});
+    std::vector<std::string> moves;
+    if ((clash && !Movable(l.out)) || !SafeWithMoves(l.members, {{i, l.a}, {i, l.b}}, &moves)) return std::nullopt;
+    if (clash) moves.push_back(l.out.name);
+    pending_moves_.insert(pending_moves_.end(), moves.begin(), moves.end());
+    l.bytes = Bytes({&l.a, &l.b, &l.out}) + static_cast<double>(steps_[i].kernel->GetConstantBytes());
     l.flops = Flops(l.members);
     return l;
   }

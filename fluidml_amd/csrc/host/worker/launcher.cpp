@@ -178,6 +178,7 @@ void LaunchPlan::Materialize() {
   }
   for (Step &s : steps_) s.kernel->Prepare();
   PackConvWeights();
+  PreparePools();
   PackContractionWeights();
   std::vector<Transfer::Slot> in, out;
   for (const Argument &a : arguments_) {
@@ -347,6 +348,21 @@ void LaunchPlan::PackConvWeights() {
   }
 }
 
+namespace {
+std::string WholeName(const Launch &l) { return "whole:" + l.whole.name; }
+}  // namespace
+
+// A buffer for the result of each convolution that hands its pool a tensor after all.
+void LaunchPlan::PreparePools() {
+  for (const Launch &l : GetSchedule()) {
+    if (!l.pooled || packed_.count(l.b.name)) continue;
+    RawSlot &slot = privates_[WholeName(l)];
+    if (slot.device != nullptr) continue;
+    slot.bytes = l.whole.meta.GetSize();
+    Check(fluidml_hip_arena_create(slot.bytes, &slot.device), "allocating a device buffer");
+  }
+}
+
 // Environment FLUIDML_MATMUL_PACKED=0 (read at every compile) leaves all weights as they stand.
 void LaunchPlan::PackContractionWeights() {
   const char *env = std::getenv("FLUIDML_MATMUL_PACKED");
@@ -448,7 +464,7 @@ void LaunchPlan::SettleWeights() {
 }
 
 int LaunchPlan::IssuePackedConv(const Step &step, const Operand &weights, const fl_tensor &in, const fl_tensor &out,
-                                const fl_ew_program *chain, void *stream) const {
+                                const fl_ew_program *chain, bool pooled, void *stream) const {
   const auto it = IsPackableConv(step, weights) ? packed_.find(weights.name) : packed_.end();
   if (it == packed_.end()) return FL_ERR_UNSUPPORTED;
   const kernel::TensorView w = ViewOf(Resolve(weights), weights);
@@ -456,9 +472,10 @@ int LaunchPlan::IssuePackedConv(const Step &step, const Operand &weights, const 
   kernel::TensorView c;
   if (bias != nullptr) c = bias->View();
   const bool padded = step.node->GetKind() == flow::OpKind::ConvWithPadding;
-  const int rc = fluidml_hip_conv3x3_packed_chain(&in, &w.t, it->second.device, it->second.parts, bias ? &c.t : nullptr, &out,
-                                                  padded ? step.node->GetAttrs().pads.data() : nullptr, chain, 0, stream);
-  if (rc == FL_ERR_UNSUPPORTED && constants_.at(weights.name).packed_only) {
+  const auto run = pooled ? fluidml_hip_conv3x3_packed_chain_pool : fluidml_hip_conv3x3_packed_chain;
+  const int rc = run(&in, &w.t, it->second.device, it->second.parts, bias ? &c.t : nullptr, &out,
+                     padded ? step.node->GetAttrs().pads.data() : nullptr, chain, 0, stream);
+  if (rc == FL_ERR_UNSUPPORTED && !pooled && constants_.at(weights.name).packed_only) {
     throw std::logic_error("plan: weights " + weights.name + " are packed, their convolution is not");
   }
   return rc;
@@ -684,7 +701,7 @@ void LaunchPlan::IssueStep(kernel::LaunchContext &ctx, const Step &s, const Oper
   } else {
     const Operand &op1 = in1_view ? *in1_view : s.in1;
     const kernel::TensorView in1 = ViewOf(Resolve(op1), op1);
-    const int rc = IssuePackedConv(s, op1, in0.t, out.t, nullptr, ctx.stream);
+    const int rc = IssuePackedConv(s, op1, in0.t, out.t, nullptr, false, ctx.stream);
     if (rc != FL_ERR_UNSUPPORTED) ctx.Note(rc, "conv3x3_packed_chain");
     else if (s.has_buffer) dynamic_cast<kernel::DoubleInputsWithBufferKernel &>(*k).Run(ctx, in0, in1, out, buffer);
     else dynamic_cast<kernel::DoubleInputsWithoutBufferKernel &>(*k).Run(ctx, in0, in1, out);
@@ -858,6 +875,23 @@ void LaunchPlan::Issue(kernel::LaunchContext &ctx, const Launch &l, int *rc_out)
       kernel::TensorView c;
       if (bias != nullptr) c = bias->View();
       const bool padded = steps_[l.owner].node->GetKind() == flow::OpKind::ConvWithPadding;
+      if (l.pooled) {
+        rc = IssuePackedConv(steps_[l.owner], l.b, a.t, out.t, &l.chain, true, ctx.stream);
+        if (rc != FL_ERR_UNSUPPORTED) break;
+        // the convolution, then the pool
+        const kernel::TensorView whole = ViewOf(privates_.at(WholeName(l)).device, l.whole);
+        rc = IssuePackedConv(steps_[l.owner], l.b, a.t, whole.t, &l.chain, false, ctx.stream);
+        if (rc == FL_ERR_UNSUPPORTED) {
+          rc = fluidml_hip_conv_chain(&a.t, &b.t, bias ? &c.t : nullptr, &whole.t, padded ? at.pads.data() : nullptr,
+                                      at.strides.data(), at.dilations.data(), at.group, &l.chain, contract_flags, ctx.stream);
+        }
+        if (rc == FL_OK) {
+          const flow::Attrs &pool = steps_[l.members.back()].node->GetAttrs();
+          rc = fluidml_hip_max_pool_without_padding(&whole.t, &out.t, pool.kernel_shape.data(), pool.strides.data(),
+                                                    static_cast<int32_t>(pool.kernel_shape.size()), ctx.stream);
+        }
+        break;
+      }
       if (l.has_out2) {
         const kernel::TensorView mean = ViewOf(Resolve(l.out2), l.out2);
         rc = fluidml_hip_conv_chain_mean(&a.t, &b.t, bias ? &c.t : nullptr, &out.t, padded ? at.pads.data() : nullptr,
@@ -875,7 +909,7 @@ void LaunchPlan::Issue(kernel::LaunchContext &ctx, const Launch &l, int *rc_out)
                                               contract_flags | (l.skip_is_factor ? FL_CONTRACT_ADDEND_IS_FACTOR : 0u), ctx.stream);
         break;
       }
-      rc = IssuePackedConv(steps_[l.owner], l.b, a.t, out.t, &l.chain, ctx.stream);
+      rc = IssuePackedConv(steps_[l.owner], l.b, a.t, out.t, &l.chain, false, ctx.stream);
       if (rc != FL_ERR_UNSUPPORTED) break;
       rc = fluidml_hip_conv_chain(&a.t, &b.t, bias ? &c.t : nullptr, &out.t, padded ? at.pads.data() : nullptr,
                                   at.strides.data(), at.dilations.data(), at.group, &l.chain, contract_flags, ctx.stream);

@@ -114,6 +114,10 @@ struct Launch {
   // member, `out` the tensor it reads, which is written too)
   Operand out2;
   bool has_out2 = false;
+  // ConvChain whose result goes into a MaxPool of 2 x 2 windows (the last member) alone: `out` = the pooled tensor, `whole` = the
+  // convolution's result, which nothing holds unless the weights turn out not to be packed (PreparePools)
+  bool pooled = false;
+  Operand whole;
   double s0 = 0, s1 = 0, s2 = 0;
   int64_t axis = 0;
   std::vector<int64_t> perm;
@@ -301,6 +305,7 @@ class LaunchPlan {
   // Weights of 3x3 convolutions laid out for the matrix cores (fluidml_hip_conv3x3_pack), once per plan; issuing a
   // convolution whose weights are not among them takes them as they stand.
   void PackConvWeights();
+  void PreparePools();
   // The same for the weights of MatMul and Gemm (fluidml_hip_contract_pack); the library finds them by their address.
   void PackContractionWeights();
   // Once the schedule and its tile configurations are final: frees the packed weights that no launch takes, and the weights
@@ -308,7 +313,7 @@ class LaunchPlan {
   void SettleWeights();
   // (FL_ERR_UNSUPPORTED, nothing launched, where they are not, or the operands do not fit)
   int IssuePackedConv(const Step &step, const Operand &weights, const fl_tensor &in, const fl_tensor &out,
-                      const fl_ew_program *chain, void *stream) const;
+                      const fl_ew_program *chain, bool pooled, void *stream) const;
   void LaunchAll(kernel::LaunchContext &ctx) const;
   void Replay(kernel::LaunchContext &ctx);
   void PlanBranches() const;

@@ -522,6 +522,9 @@ int fluidml_hip_conv_chain(const fl_tensor *in, const fl_tensor *weights, const 
 int fluidml_hip_conv3x3_packed_bytes(const fl_tensor *weights, int32_t parts, size_t *bytes);
 int fluidml_hip_conv3x3_pack(const fl_tensor *weights, int32_t parts, void *packed, void *stream);
 int fluidml_hip_conv3x3_packed_chain(const fl_tensor *in, const fl_tensor *weights, const void *packed, int32_t parts, const fl_tensor *bias, const fl_tensor *out, const int64_t *pads, const fl_ew_program *chain, uint32_t flags, void *stream);
+/* The same with a MaxPoolWithoutPaddingKernel of 2 x 2 windows and strides behind the chain (reference maxpool.cpp:17-82) in the
+ * same launch: `out` is the pooled tensor, the convolution's own result is not written. */
+int fluidml_hip_conv3x3_packed_chain_pool(const fl_tensor *in, const fl_tensor *weights, const void *packed, int32_t parts, const fl_tensor *bias, const fl_tensor *out, const int64_t *pads, const fl_ew_program *chain, uint32_t flags, void *stream);
 /* [MulCommonKernel(x, scale per channel) ->] Conv{With,Without}PaddingKernel -> elementwise chain [-> AddCommonKernel
  * with a tensor of the output's shape] as ONE launch (reference mul.cpp, conv.cpp:27-280, add.cpp:75-137: the
  * projection of an inverted-residual block behind its squeeze-and-excitation gate, with the skip connection).
