@@ -159,6 +159,7 @@ struct PlaneArgs {
   FastDiv div_ow, div_pitch;
   fl_ew_program chain;
 };
+static_assert(sizeof(PlaneArgs) >= 5 * 32 && offsetof(PlaneArgs, chain) <= 5 * 32, "five times eight words");
 
 template <int K>
 __global__ __launch_bounds__(kBlock) void ConvDepthwisePlaneKernel(PlaneArgs p, float *__restrict__ out,
@@ -166,6 +167,9 @@ __global__ __launch_bounds__(kBlock) void ConvDepthwisePlaneKernel(PlaneArgs p, 
                                                                    const float *__restrict__ w) {
   extern __shared__ __align__(16) float plane[];
   __shared__ float partial[kBlock / kWave];
+  typedef int32_t Line __attribute__((ext_vector_type(8), aligned(4)));
+  const Line *lines = reinterpret_cast<const Line *>(&p);  // (all arguments in one fetch)
+  asm volatile("" ::"s"(lines[0]), "s"(lines[1]), "s"(lines[2]), "s"(lines[3]), "s"(lines[4]), "s"(in), "s"(w));
   const int32_t c = blockIdx.x, n = blockIdx.y;
   const int tid = threadIdx.x;
   float wv[K * K];
@@ -174,12 +178,26 @@ __global__ __launch_bounds__(kBlock) void ConvDepthwisePlaneKernel(PlaneArgs p, 
   const float bias = p.bias != nullptr ? p.bias[c * p.sB] : 0.0f;
   const float *src = in + static_cast<int64_t>(n) * p.sXn + static_cast<int64_t>(c) * p.sXc;
   const uint32_t n_stage = static_cast<uint32_t>(p.rows * p.pitch);
-  for (uint32_t i = tid; i < n_stage; i += kBlock) {
-    uint32_t r, cc;
-    p.div_pitch.DivMod(i, r, cc);
-    const int32_t ih = static_cast<int32_t>(r) - p.pad_h, iw = static_cast<int32_t>(cc) - p.pad_w;
-    const bool inside = static_cast<uint32_t>(ih) < static_cast<uint32_t>(p.H) && static_cast<uint32_t>(iw) < static_cast<uint32_t>(p.W);
-    plane[i] = inside ? src[ih * p.sXh + iw * p.sXw] : 0.0f;
+  // kAhead places per round trip, none behind a condition: outside the input its nearest place is read and a zero stored (planes
+  // of 14 x 14 to 30 x 30: one round trip instead of up to four, nine launches of EfficientNet-B0 5.2 -> 4.5 us each)
+  constexpr int kAhead = 4;
+  for (uint32_t i0 = tid; i0 < n_stage; i0 += kAhead * kBlock) {
+    float x[kAhead];
+    bool ok[kAhead];
+#pragma unroll
+    for (int a = 0; a < kAhead; ++a) {
+      uint32_t r, cc;
+      p.div_pitch.DivMod(min(i0 + a * kBlock, n_stage - 1), r, cc);
+      const int32_t ih = static_cast<int32_t>(r) - p.pad_h, iw = static_cast<int32_t>(cc) - p.pad_w;
+      const int32_t row = min(max(ih, 0), p.H - 1), col = min(max(iw, 0), p.W - 1);
+      ok[a] = row == ih && col == iw;
+      x[a] = src[row * p.sXh + col * p.sXw];
+    }
+#pragma unroll
+    for (int a = 0; a < kAhead; ++a) {
+      asm volatile("" : "+v"(x[a]));  // (the compiler puts the load behind the condition again)
+      if (i0 + a * kBlock < n_stage) plane[i0 + a * kBlock] = ok[a] ? x[a] : 0.0f;
+    }
   }
   __syncthreads();
   float *dst = out + static_cast<int64_t>(n) * p.sOn + static_cast<int64_t>(c) * p.sOc;
