@@ -123,8 +123,11 @@ __global__ __launch_bounds__(64 * WN *KS) void MatmulRowsKernel(float *C_, const
   const int gt = ks * 64 + lane;
   auto row_of = [&](int v) { return KS > 1 ? (gt + v * 64 * KS) / BN : v / (4 * W) * 16 + 4 * g + v % (4 * W) / W; };
   auto col_of = [&](int v) { return KS > 1 ? n0 + (gt + v * 64 * KS) % BN : n_first + v % W; };
+  // (KS == 1: a lane moved left to lie inside N repeats columns of its neighbours and stores only those that are its own: one
+  // thread per element, which may then be the addend's too)
   auto lives = [&](int v) {
-    return m0 + row_of(v) < p.M && col_of(v) < p.N && (KS == 1 || kValues % (64 * KS) == 0 || gt + v * 64 * KS < kValues);
+    if constexpr (KS == 1) return m0 + row_of(v) < p.M && col_of(v) >= n0 + W * c;
+    return m0 + row_of(v) < p.M && col_of(v) < p.N && (kValues % (64 * KS) == 0 || gt + v * 64 * KS < kValues);
   };
   auto place = [&](int r, int n) {
     int64_t col = static_cast<int64_t>(n) * sCn;

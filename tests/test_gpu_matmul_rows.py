@@ -103,9 +103,15 @@ def test_rows_infinities(device):
             close(out[fine], want[fine], "finite results")
 
 
-@pytest.mark.parametrize("C,F,H,W", [(4, 24, 9, 7), (144, 40, 28, 28), (1152, 320, 7, 7), (16, 96, 61, 67), (32, 16, 112, 112)])
-def test_rows_pointwise_conv(device, C, F, H, W):
-    """Pointwise convolution with a scale per channel and a skip tensor, both alone and together, odd numbers of pixels."""
+# 16x16, 32x48, 16x16, 16x128, 16x128, 16x256 (its last workgroup's last waves lie past the pixels), 16x256 (one lane's second column does)
+POINTWISE = [(4, 24, 9, 7), (144, 40, 28, 28), (1152, 320, 7, 7), (16, 96, 61, 67), (32, 16, 112, 112), (16, 96, 127, 99), (28, 130, 65, 63)]
+
+
+@pytest.mark.parametrize("C,F,H,W", POINTWISE)
+@pytest.mark.parametrize("in_place", [False, True], ids=["", "in_place"])
+def test_rows_pointwise_conv(device, C, F, H, W, in_place):
+    """Pointwise convolution with a scale per channel and a skip tensor, both alone and together, odd numbers of pixels; the skip
+    tensor may be the result's own memory: every element is read and written by one thread."""
     import torch
 
     from fluidml_amd import cabi
@@ -124,6 +130,9 @@ def test_rows_pointwise_conv(device, C, F, H, W):
         want = torch.einsum("fc,cp->fp", w.double()[:, :, 0, 0].cpu(), (x * s if s is not None else x).double().cpu().view(C, -1))
         want = (want + b.double().cpu()[:, None]).clamp_min(0).view(1, F, H, W) + (e.double().cpu() if e is not None else 0)
         out = torch.full((1, F, H, W), 9.0, device=device)
+        if in_place and e is not None:
+            out.copy_(e)
+            e = out
         if s is None and e is None:
             cabi.call("conv_chain", ref(x), ref(w), ref(b), ref(out), None, one, one, ctypes.c_int64(1), ctypes.byref(relu), ctypes.c_uint32(0), None)
         else:
