@@ -62,6 +62,10 @@ __device__ __forceinline__ T At(const void *base, O bytes) {
   return *reinterpret_cast<const T *>(static_cast<const char *>(base) + bytes);
 }
 
+// Two workgroups of eight waves fit a compute unit if they make do with 128 registers, and with V's columns one by one up to
+// 8 tiles of keys times tiles of columns do (128 heads x 257 x 257, 32 columns, V transposed: with 130 registers 75 us, with 128 60).
+constexpr int MinWaves(int waves, int tiles, bool vec) { return !vec && waves == 8 && tiles <= 8 ? 4 : 1; }
+
 // Consecutive floats, at any address.
 template <int N>
 struct __attribute__((packed, aligned(4))) Run {
@@ -76,9 +80,9 @@ struct __attribute__((packed, aligned(4))) Run {
 // MASK, COND: an additive mask, a condition may be there.
 // QT: tiles of 16 queries a workgroup takes with the keys and values it has loaded.
 template <int NW, int KT, int DT, int QT, bool FULL, bool VEC, bool MASK, bool COND>
-__global__ __launch_bounds__(64 * NW) void AttentionKernel(AttentionArgs a, float *__restrict__ out, const float *__restrict__ q,
-                                                           const float *__restrict__ kt, const float *__restrict__ v,
-                                                           const float *__restrict__ mask, const uint8_t *__restrict__ cond) {
+__global__ __launch_bounds__(64 * NW, MinWaves(NW, KT * DT, VEC)) void AttentionKernel(
+    AttentionArgs a, float *__restrict__ out, const float *__restrict__ q, const float *__restrict__ kt, const float *__restrict__ v,
+    const float *__restrict__ mask, const uint8_t *__restrict__ cond) {
   constexpr int kLd = 16 * DT + 4;  // floats per query in LDS: lanes of consecutive queries in different banks
   __shared__ __attribute__((aligned(16))) float ctx[QT * NW * kQ * kLd];
   __shared__ float stat[2][QT][NW][kQ];  // the waves' maxima and sums
@@ -174,21 +178,35 @@ __global__ __launch_bounds__(64 * NW) void AttentionKernel(AttentionArgs a, floa
   }
   float vreg[KT][4][DT];
   const float *vb = v + off[3];
+  auto load_v = [&] {
 #pragma unroll
-  for (int t = 0; t < KT; ++t)
+    for (int t = 0; t < KT; ++t)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int n = min(key(t, 4 * grp + i), last_key);
-      if constexpr (VEC) {
-        const Run<DT> x = At<Run<DT>>(vb, bytes(n * a.sVn + column(0, l16)));
+      for (int i = 0; i < 4; ++i) {
+        const int n = min(key(t, 4 * grp + i), last_key);
+        if constexpr (VEC) {
+          const Run<DT> x = At<Run<DT>>(vb, bytes(n * a.sVn + column(0, l16)));
 #pragma unroll
-        for (int j = 0; j < DT; ++j) vreg[t][i][j] = x.v[j];
-      } else {
-        const float *at = vb + n * a.sVn;
+          for (int j = 0; j < DT; ++j) vreg[t][i][j] = x.v[j];
+        } else {
+          const float *at = vb + n * a.sVn;
 #pragma unroll
-        for (int j = 0; j < DT; ++j) vreg[t][i][j] = at[(FULL ? column(j, l16) : min(column(j, l16), a.D - 1)) * a.sVd];
+          for (int j = 0; j < DT; ++j) vreg[t][i][j] = at[(FULL ? column(j, l16) : min(column(j, l16), a.D - 1)) * a.sVd];
+        }
       }
-    }
+  };
+  // V's columns one by one: these loads keep the other waves' loads of K waiting, so they leave once this wave's K is there, and
+  // with many of them (or with some and a mask) behind the scores, where K's registers are free again.  Measured (us; before the loads were put ahead
+  // of the scores, with all of them there, now): 128 heads x 200 x 200, 40 columns, a condition
+  // 39.0, 47.5, 33.8; V transposed: 128 x 256 x 256, 48, a condition 72.0, 90.3, 67.5; 128 x 300 x 300, 48 134, 155, 136;
+  // 128 x 300 x 300, 64 157, 174, 167.
+  constexpr bool kBehindScores = !VEC && KT == 4 && (DT == 4 || (DT == 2 && (MASK || COND)));
+  if constexpr (!VEC && !kBehindScores) {
+#pragma unroll
+    for (int t = 0; t < KT; ++t) asm volatile("" ::"v"(kreg[t][DT - 1][3]));
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if constexpr (!kBehindScores) load_v();
 
   // ---- scores ------------------------------------------------------------------------------------------------------
   if constexpr (!FULL) {
@@ -216,6 +234,12 @@ __global__ __launch_bounds__(64 * NW) void AttentionKernel(AttentionArgs a, floa
         for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(kreg[t][j][e], qreg[u][j][e], acc, 0, 0, 0);
       s[u][t][0] = acc.x, s[u][t][1] = acc.y, s[u][t][2] = acc.z, s[u][t][3] = acc.w;
     }
+
+  if constexpr (kBehindScores) {
+    __builtin_amdgcn_sched_barrier(0);
+    load_v();
+    __builtin_amdgcn_sched_barrier(0);
+  }
 
   // ---- scale, mask, condition; exponentials about the maximum of the wave's keys ---------------------------------
   const bool ragged = n0 + 16 * KT > a.Skv;  // some of the wave's keys do not exist
@@ -424,16 +448,21 @@ int fluidml_hip_attention(const fl_tensor *q, const fl_tensor *kt, const fl_tens
   a.vec_q = vec ? 1 : 0;
 #define FL_ATTENTION_AS(...) \
   FL_LAUNCH((AttentionKernel<__VA_ARGS__>), grid, block, 0, AsStream(stream), a, o, qp, kp, vp, mp, cp)
+#define FL_ATTENTION_SCATTERED(NW_, KT_, DT_, FULL_)                                                                 \
+  do {                                                                                                               \
+    if (mp == nullptr && cp == nullptr) FL_ATTENTION_AS(NW_, KT_, DT_, 1, FULL_, false, false, false);               \
+    else if (cp == nullptr) FL_ATTENTION_AS(NW_, KT_, DT_, 1, FULL_, false, true, false);                            \
+    else if (mp == nullptr) FL_ATTENTION_AS(NW_, KT_, DT_, 1, FULL_, false, false, true);                            \
+    else FL_ATTENTION_AS(NW_, KT_, DT_, 1, FULL_, false, true, true);                                                \
+  } while (0)
 #define FL_ATTENTION_D(NW_, KT_, DT_, QT_)                                                                           \
   do {                                                                                                               \
     const dim3 block(64 * NW_);                                                                                      \
     if (a.D == 16 * DT_ && runs && cp == nullptr) FL_ATTENTION_AS(NW_, KT_, DT_, QT_, true, true, true, false);      \
     else if (a.D == 16 * DT_ && runs && mp == nullptr) FL_ATTENTION_AS(NW_, KT_, DT_, QT_, true, true, false, true); \
     else if (a.D == 16 * DT_ && runs) FL_ATTENTION_AS(NW_, KT_, DT_, QT_, true, true, true, true);                   \
-    else if (a.D == 16 * DT_ && cp == nullptr) FL_ATTENTION_AS(NW_, KT_, DT_, 1, true, false, true, false);          \
-    else if (a.D == 16 * DT_) FL_ATTENTION_AS(NW_, KT_, DT_, 1, true, false, true, true);                            \
-    else if (cp == nullptr) FL_ATTENTION_AS(NW_, KT_, DT_, 1, false, false, true, false);                            \
-    else FL_ATTENTION_AS(NW_, KT_, DT_, 1, false, false, true, true);                                                \
+    else if (a.D == 16 * DT_) FL_ATTENTION_SCATTERED(NW_, KT_, DT_, true);                                           \
+    else FL_ATTENTION_SCATTERED(NW_, KT_, DT_, false);                                                               \
   } while (0)
 #define FL_ATTENTION(NW_, KT_, QT_)                       \
   do {                                                    \
@@ -450,6 +479,7 @@ int fluidml_hip_attention(const fl_tensor *q, const fl_tensor *kt, const fl_tens
   else FL_ATTENTION(8, 4, 1);
 #undef FL_ATTENTION
 #undef FL_ATTENTION_D
+#undef FL_ATTENTION_SCATTERED
 #undef FL_ATTENTION_AS
   return LaunchStatus();
 }

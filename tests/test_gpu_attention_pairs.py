@@ -61,6 +61,10 @@ def run(device, batch, sq, skv, d, masked, where, turned, divisor, spoil=False):
     ((2, 3, 3), 250, 300, 64, True, 8.0),    # three batch dims that do not merge; no unit strides: one tile of queries
     ((3, 6), 250, 300, 40, False, 8.0),      # head columns in no sixteens: one tile
     ((2, 3), 50, 120, 64, True, 4.0),
+    ((5,), 70, 200, 48, False, 8.0),         # V's columns one by one, in all its forms
+    ((2, 3), 33, 200, 40, True, 8.0),
+    ((5,), 70, 333, 32, True, 8.0),
+    ((3,), 20, 270, 16, True, 8.0),
 ])
 @pytest.mark.parametrize("masked,where", [(False, False), (True, False), (False, True), (True, True)], ids=["plain", "mask", "cond", "both"])
 def test_attention_pairs(device, batch, sq, skv, d, turned, divisor, masked, where):
@@ -77,3 +81,28 @@ def test_attention_pairs_not_finite(device):
     assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
     fine = want.isfinite()
     assert (got - want)[fine].abs().max() <= 2.0 ** -24 * (2 * 64 * 64 / 8 / 4 + 512 / 16 + 16)
+
+
+@pytest.mark.parametrize("d,skv", [(40, 200), (64, 256), (32, 300)])
+@pytest.mark.parametrize("masked,where", [(False, False), (True, False), (False, True), (True, True)], ids=["plain", "mask", "cond", "both"])
+def test_attention_scattered_fits(device, d, skv, masked, where):
+    """V in columns one by one: up to 256 keys, beyond with up to 32 head columns, two workgroups fit a compute unit."""
+    import torch
+
+    from util import launches
+
+    t = torch.rand(2, d, skv, device=device)
+    q, kt, v = torch.rand(2, 64, d, device=device), t, t.transpose(1, 2)
+    mask = torch.rand(1, 1, skv, device=device) if masked else None
+    cond = torch.ones(1, 64, skv, dtype=torch.bool, device=device) if where else None
+    out = torch.empty(2, 64, d, device=device)
+
+    def call(stream):
+        from fluidml_amd import cabi
+
+        cabi.call("attention", ref(q), ref(kt), ref(v), ref(out), ctypes.c_double(8.0), 1, ref(mask) if masked else None,
+                  ref(cond) if where else None, ctypes.c_double(-1e9), stream)
+
+    call(None)
+    (name, fit), = launches(call)
+    assert "AttentionKernel" in name and fit >= 2

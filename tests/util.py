@@ -129,3 +129,40 @@ def assert_close_or_exact(got, ref, exact_fn, reduction_length, what="", report=
     assert np.count_nonzero(bad) <= 0.01 * bad.size, (
         f"{what}: {np.count_nonzero(bad)} of {bad.size} elements pass only through the float64 evaluation (more than 1 %)"
     )
+
+
+class _KernelNode(ctypes.Structure):  # hipKernelNodeParams
+    _fields_ = [("block", ctypes.c_uint32 * 3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", ctypes.c_uint32 * 3),
+                ("params", ctypes.c_void_p), ("shared", ctypes.c_uint32)]
+
+
+def launches(call):
+    """The kernels that `call(stream)` launches, in the order of its graph: (mangled name, workgroups a compute unit holds).
+
+    The call is recorded, not run; it must have run once before (a first call may allocate)."""
+    import torch
+
+    from fluidml_amd import cabi
+
+    hip = cabi.lib  # (its runtime's entry points are found through it)
+    hip.hipKernelNameRefByPtr.restype = ctypes.c_char_p
+    stream, graph, count = ctypes.c_void_p(torch.cuda.Stream().cuda_stream), ctypes.c_void_p(), ctypes.c_size_t()
+    assert hip.hipStreamBeginCapture(stream, 2) == 0
+    try:
+        call(stream)
+    finally:
+        assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+    assert hip.hipGraphGetNodes(graph, None, ctypes.byref(count)) == 0
+    nodes = (ctypes.c_void_p * count.value)()
+    assert hip.hipGraphGetNodes(graph, nodes, ctypes.byref(count)) == 0
+    found = []
+    for node in nodes:
+        p, fit = _KernelNode(), ctypes.c_int()
+        assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(p)) == 0
+        threads = p.block[0] * p.block[1] * p.block[2]
+        name = hip.hipKernelNameRefByPtr(ctypes.c_void_p(p.func), stream)
+        assert hip.hipOccupancyMaxActiveBlocksPerMultiprocessor(ctypes.byref(fit), ctypes.c_void_p(p.func), threads,
+                                                                ctypes.c_size_t(p.shared)) == 0
+        found.append((name.decode(), fit.value))
+    assert hip.hipGraphDestroy(graph) == 0
+    return found
