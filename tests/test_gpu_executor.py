@@ -92,7 +92,11 @@ def test_dp_measured_layouts_match_oracle(device, tiny_bert, monkeypatch, tmp_pa
     doc = json.load(open(json_path))
     assert {"dp_table", "plan", "whole_graph_ns"} <= set(doc)
     timing = doc["whole_graph_ns"]
-    assert timing["kept"] == ("dp" if timing["dp"] <= timing["default_layouts"] else "default_layouts")
+    # (the proposal has to win by 1.5 %; both times stand there without their fraction of a nanosecond)
+    if timing["kept"] == "dp":
+        assert timing["dp"] < 0.985 * (timing["default_layouts"] + 1)
+    else:
+        assert timing["kept"] == "default_layouts" and timing["dp"] + 1 > 0.985 * timing["default_layouts"]
     assert ("dp_plan" in doc) == (timing["kept"] == "default_layouts")
     for name, layout in first.items():
         if name in doc["plan"] and name not in {v.name for v in net.outputs}:
