@@ -457,20 +457,34 @@ int LaunchShape(const MatmulArgs &p, uint32_t n_batch, float *C, const float *A,
 // 16x16 their waves stand side by side:
 //   144 x 3136 x 24        6.5     8.2    7.7    12     6.1    10     16x128 5.5, 16x256 5.9
 //   96 x 12544 x 16       10.8     19     17     26     14     20     16x128 10.5, 16x256 8.7
+// Where the tiled kernel's rule is the faster one (us, this rule without the exceptions behind it; sixteen sets of operands in turn, the
+// pointwise convolutions one):
+//   * tiles larger than 16x32: eight slices share 4, 12 or 20 stages unevenly, and the chunks of 128 terms of the tiled kernel divide
+//     those sums: 192 x 1024 x 384 5.5, 6.4, x 512 6.1, 6.4, x 640 6.8, 8.2, x 704 9.6, 8.1, x 1152 12.2, 11.1; 192 x 768 x 384
+//     5.5, 6.2, x 640 6.8, 7.6; 512 x 768 x 128 4.9, 5.5 (with 16x48 and 32x32 as fast), x 192 6.4, 6.4, x 384 7.9, 8.4
+//   * waves side by side, more than three workgroups to a compute unit: tiles of 64 rows read B a quarter as often, and are
+//     faster where they pad less than a third: 240 x 6400 x 64 (750) 9.1, 8.6, 128 x 12544 x 64 (784) 9.4, 10.2,
+//     1024 x 50176 x 48 119, 167; 72 x 50176 x 64 19.9, 17.1, 144 x 50176 x 64 28.3, 27.8
+//   * the same with a scale per row of B, which every row tile multiplies by again, in the tile of 16x256 past one workgroup to a
+//     compute unit: 256 x 3136 x 32 (208) 6.7, 5.2, 192 x 12544 x 32 (588) 9.0, 10.6, 1024 x 50176 x 32 107, 127;
+//     112 x 50176 x 32, which 64 rows pad by a seventh, 19.4, 18.7
+// The limits of K, this kernel over the tiled one's time on the other side too: 16x16, x 1536 0.83 to 0.88, x 2048 0.90 to 0.97 (32 x
+// 2048 1.11), x 2432 0.98 to 1.05, x 3072 1.00 to 1.08; the larger tiles, x 1088 and 1152 0.80 to 0.98 (192 x 768 and 96 x 1536 1.02 to
+// 1.09), x 1408 0.83 to 1.12, x 1664 0.88 to 1.14, x 2048 0.79 to 1.05.
 Shape Choose(const MatmulArgs &p, uint32_t n_batch, bool extra) {
-  auto fits = [&](int bm, int bn) {
-    return static_cast<int64_t>((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn) * n_batch <= 256;
-  };
+  auto tiles = [&](int bm, int bn) { return static_cast<int64_t>((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn) * n_batch; };
+  auto fits = [&](int bm, int bn) { return tiles(bm, bn) <= 256; };
   const bool stats = extra && p.ln_stats_out != nullptr;  // runs of 32 columns
   if (p.K <= 2048 && !stats && fits(16, 16)) return k16x16;
   if (p.K <= 1152) {
-    if (fits(16, 32)) return k16x32;
-    if (!stats && fits(16, 48)) return k16x48;
-    if (fits(32, 32)) return k32x32;
-    if (!stats && fits(32, 48)) return k32x48;
+    const Shape shape = fits(16, 32) ? k16x32 : !stats && fits(16, 48) ? k16x48 : fits(32, 32) ? k32x32 : !stats && fits(32, 48) ? k32x48 : kNone;
+    const bool uneven = p.K % 256 == 128 && p.K <= 640 && (p.K > 128 || shape == k32x48);
+    if (shape != kNone) return shape != k16x32 && uneven ? kNone : shape;
   }
-  if (p.K <= 64 && !extra) return p.K <= 32 && !fits(16, 128) ? k16x256_K1 : k16x128_K2;
-  return kNone;
+  if (p.K > 64 || extra) return kNone;
+  const int64_t padded = (p.M + 63) / 64 * 64;  // the rows that the tiled kernel multiplies
+  if (p.K <= 32 && !fits(16, 128)) return p.k_scale == nullptr || fits(16, 256) || 7 * padded >= int64_t{8} * p.M ? k16x256_K1 : kNone;
+  return tiles(16, 128) <= 3 * 256 || 3 * padded >= int64_t{4} * p.M ? k16x128_K2 : kNone;
 }
 
 }  // namespace

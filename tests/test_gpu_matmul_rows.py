@@ -5,6 +5,7 @@ import ctypes
 import pytest
 
 from test_gpu_matmul_parts import Problem, close
+from util import launches
 
 pytestmark = pytest.mark.gpu
 STAGED = 1 << 4 | 1 << 8  # FL_TILE_32x32_STAGED, K not split
@@ -139,3 +140,61 @@ def test_rows_pointwise_conv(device, C, F, H, W, in_place):
             cabi.call("conv_chain_scale_add", ref(x), ref(w), ref(b), ref(out), None, one, one, ctypes.c_int64(1), ctypes.byref(relu),
                       ref(s) if s is not None else None, ref(e) if e is not None else None, ctypes.c_uint32(0), None)
         close(out, want, f"scale {s is not None} skip {e is not None}")
+
+
+# template arguments: matrix tiles of rows, columns per lane, waves side by side, slices of K
+TILES = {"16x16": (1, 1, 1, 8), "16x32": (1, 2, 1, 8), "16x48": (1, 3, 1, 8), "32x32": (2, 2, 1, 8), "32x48": (2, 3, 1, 8),
+         "16x128": (1, 2, 4, 2), "16x256": (1, 2, 8, 1)}
+
+
+def tile_of(call):
+    """The tile of the one launch of `call`, None if it is another kernel's."""
+    call(None)
+    (name, _), = launches(call)
+    if "MatmulRowsKernel" not in name:
+        return None
+    return next(t for t, a in TILES.items() if "MatmulRowsKernelI" + "".join(f"Li{n}E" for n in a) in name)
+
+
+# both sides of each line the rule draws
+@pytest.mark.parametrize("M,K,N,tile", [
+    (256, 2048, 256, "16x16"), (256, 2052, 256, None), (257, 1152, 256, "16x32"), (257, 1156, 256, None),
+    (192, 320, 768, "16x48"), (192, 384, 768, None), (192, 512, 768, "16x48"), (192, 640, 768, None), (192, 704, 768, "16x48"),
+    (192, 128, 768, "16x48"), (192, 896, 768, "16x48"),
+    (192, 128, 1024, "32x32"), (192, 384, 1024, None), (192, 640, 1024, None), (192, 896, 1024, "32x32"),
+    (512, 128, 768, None), (512, 192, 768, "32x48"), (512, 384, 768, None), (512, 512, 768, "32x48"),
+    (128, 384, 768, "16x32"), (128, 640, 768, "16x32"),
+    (513, 68, 768, None),
+])
+def test_rows_rule(device, M, K, N, tile):
+    with Problem(device, M, K, N) as p:
+        out, none = p.out(), ctypes.byref(p.cabi.make_chain([]))
+        assert tile_of(lambda s: p.cabi.call("matmul_chain", p.ref(p.x), p.ref(p.w[0]), p.ref(p.b[0]), p.ref(out), none, 0, s)) == tile
+
+
+@pytest.mark.parametrize("C,F,pixels,tile,scaled", [
+    (64, 256, 6144, "16x128", "16x128"),   # 768 workgroups
+    (64, 256, 6272, None, None),           # 784
+    (48, 128, 12544, None, None),
+    (64, 96, 12544, "16x128", "16x128"),   # 64 rows pad a third
+    (64, 112, 25600, None, None),          # and less
+    (40, 1024, 6400, None, None),
+    (24, 256, 4096, "16x256", "16x256"),   # 256 workgroups
+    (24, 256, 4224, "16x256", None),
+    (32, 1024, 6400, "16x256", None),
+    (16, 112, 25600, "16x256", "16x256"),  # 64 rows pad a seventh
+    (16, 120, 25600, "16x256", None),
+])
+def test_rows_rule_pointwise(device, C, F, pixels, tile, scaled):
+    import torch
+
+    from fluidml_amd import cabi
+
+    x, w, b = (torch.zeros(*s, device=device) for s in ((1, C, pixels, 1), (F, C, 1, 1), (F,)))
+    scale, out = torch.zeros(1, C, 1, 1, device=device), torch.zeros(1, F, pixels, 1, device=device)
+    ref = lambda t: ctypes.byref(cabi.make_tensor(t.data_ptr(), cabi.FL_FLOAT32, t.shape, t.stride()))
+    one, none = cabi.i64_array([1, 1]), ctypes.byref(cabi.make_chain([]))
+    assert tile_of(lambda s: cabi.call("conv_chain", ref(x), ref(w), ref(b), ref(out), None, one, one, ctypes.c_int64(1), none,
+                                       ctypes.c_uint32(0), s)) == tile
+    assert tile_of(lambda s: cabi.call("conv_chain_scale_add", ref(x), ref(w), ref(b), ref(out), None, one, one, ctypes.c_int64(1), none,
+                                       ref(scale), None, ctypes.c_uint32(0), s)) == scaled
