@@ -138,10 +138,9 @@ __global__ __launch_bounds__(64 * WN *KS) void MatmulRowsKernel(float *C_, const
     }
     return static_cast<int64_t>(m0 + r) * sCm + col;
   };
-  constexpr bool PRE = EV <= 8;  // (more: asked for behind the K loop, the registers are taken)
-  constexpr int PV = PRE ? EV : 1;
-  float pre_bias[PV], pre_add[EXTRA != 0 ? PV : 1], pre_add2[EXTRA != 0 ? PV : 1], ln_col[NORM ? PV : 1], ln_col2[NORM ? PV : 1];
-  if constexpr (PRE) {
+  static_assert(EV <= 8, "more values would take the registers of the tiles in flight");
+  float pre_bias[EV], pre_add[EXTRA != 0 ? EV : 1], pre_add2[EXTRA != 0 ? EV : 1], ln_col[NORM ? EV : 1], ln_col2[NORM ? EV : 1];
+  {
     auto ask = [&](const float *from, int64_t at) { return (from != nullptr ? from : A)[from != nullptr ? at : 0]; };
     const float *c1 = NORM && p.ln_mode == 1 ? (blockIdx.y > 0 && p.n_groups > 1 ? p.g_ln_c1[blockIdx.y - 1] : p.ln_c1) : nullptr;
 #pragma unroll
@@ -205,7 +204,6 @@ __global__ __launch_bounds__(64 * WN *KS) void MatmulRowsKernel(float *C_, const
   auto merge_rows = [&](auto behind_c) {  // behind_c: stages requested since
     if constexpr (NORM) {
       WaitLoads<decltype(behind_c)::value * kLoads>();
-      static_assert(PRE, "the LayerNormalization's vectors are asked for ahead");
       // the mean of the row is the weighted mean of the partial means, its squared deviations the partials' own plus
       // count * (partial mean - mean)^2 each (as in matmul.hip)
       if (p.ln_mode != 0 && (kThreads == BM * kNormLanes || ln_row < BM)) {
@@ -343,38 +341,25 @@ __global__ __launch_bounds__(64 * WN *KS) void MatmulRowsKernel(float *C_, const
   // ---- epilogue -------------------------------------------------------------------------------------------------------
 #pragma unroll
   for (int v = 0; v < EV; ++v) {
-    const int r = row_of(v), m = m0 + r, n = col_of(v);
     if constexpr (NORM) {
+      const int r = row_of(v);
       if (p.ln_mode == 1) vals[v] = ln_rows[BM + min(r, BM - 1)] * (vals[v] - ln_rows[min(r, BM - 1)] * ln_col[v]);
     }
-    if (bias != nullptr) {
-      float d;
-      if constexpr (PRE) d = pre_bias[v];
-      else d = lives(v) ? bias[m * p.sDm + n * p.sDn] : 0.0f;
-      vals[v] = p.ca * vals[v] + p.cb * d;
-    }
+    if (bias != nullptr) vals[v] = p.ca * vals[v] + p.cb * pre_bias[v];
   }
   if (p.chain_n != 0) RunChainBlock<EV>(p.chain, vals);
   if constexpr (EXTRA != 0) {
     if (p.addend != nullptr) {
 #pragma unroll
       for (int v = 0; v < EV; ++v) {
-        float add, add2;
-        if constexpr (PRE) {
-          add = pre_add[v];
-          add2 = pre_add2[v];
-        } else {
-          const int64_t at = place(row_of(v), col_of(v));
-          add = lives(v) ? p.addend[at] : 0.0f;
-          add2 = p.addend2 != nullptr && lives(v) ? p.addend2[at] : 0.0f;
-        }
+        float add = pre_add[v];
         if constexpr (NORM) {
           // the addend is the un-normalised tensor of a LayerNormalization: normalise it on the way in
           const int r = min(row_of(v), BM - 1);
           if (p.ln_mode == 2) add = (add - ln_rows[r]) * ln_rows[BM + r] * ln_col[v] + ln_col2[v];
         }
         vals[v] = p.addend_is_factor != 0 ? vals[v] * add : vals[v] + add;
-        if (p.addend2 != nullptr) vals[v] += add2;
+        if (p.addend2 != nullptr) vals[v] += pre_add2[v];
       }
     }
   }
