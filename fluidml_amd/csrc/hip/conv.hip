@@ -391,10 +391,11 @@ int Conv(const fl_tensor *in, const fl_tensor *weights, const fl_tensor *bias, c
     return ConvImplicitGemm(in, weights, bias, out, pads, strides, dilations, chain, bf16, stream, extras);
   }
   if (!depthwise && flags == 0 && ns == 2) {
-    // sums of at most 32 terms (with the opt-in bf16 precision only the kind that the next kernel leaves in fp32)
-    const bool unit_3x3 = p.k_shape[0] == 3 && p.k_shape[1] == 3 && p.stride[0] == 1 && p.stride[1] == 1 && p.dilation[0] == 1 &&
-                          p.dilation[1] == 1;
-    if (ConvHaloEnabled() && (!bf16 || (unit_3x3 && F >= 32))) {
+    // sums of at most 32 terms (with the opt-in bf16 precision only the kind that the next kernel leaves in fp32; the switch of the
+    // next kernel sends every 3 x 3 kernel to the implicit GEMM, and no other)
+    const bool is_3x3 = p.k_shape[0] == 3 && p.k_shape[1] == 3;
+    const bool unit_3x3 = is_3x3 && p.stride[0] == 1 && p.stride[1] == 1 && p.dilation[0] == 1 && p.dilation[1] == 1;
+    if ((!is_3x3 || ConvHaloEnabled()) && (!bf16 || (unit_3x3 && F >= 32))) {
       const int rc = ConvShort(in, weights, bias, out, pads, strides, dilations, chain, stream);
       if (rc != FL_ERR_UNSUPPORTED) return rc;
     }

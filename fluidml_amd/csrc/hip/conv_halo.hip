@@ -500,7 +500,7 @@ __global__ __launch_bounds__(kThreads) void ConvHalo3x3Bf16Kernel(float *__restr
 
 }  // namespace
 
-// Environment FLUIDML_CONV_HALO=0 keeps every convolution on the implicit-GEMM path.
+// Environment FLUIDML_CONV_HALO=0 keeps every 3 x 3 convolution on the implicit-GEMM path.
 bool ConvHaloEnabled() {
   const char *v = std::getenv("FLUIDML_CONV_HALO");  // (read at every call)
   return v == nullptr || std::strtol(v, nullptr, 10) != 0;

@@ -124,6 +124,13 @@ def test_conv_short_rule(device, N, F, H, W, kernel, short):
     assert ("ConvShortKernel" in name) == short
 
 
+def test_conv_short_switch(device, monkeypatch):
+    """FLUIDML_CONV_HALO=0 is about kernels of 3 x 3."""
+    monkeypatch.setenv("FLUIDML_CONV_HALO", "0")
+    assert "ConvShortKernel" not in check(device, SHORT[0], "planes")
+    assert "ConvShortKernel" in check(device, SHORT[4], "planes")
+
+
 def test_conv_short_edges_hold_no_infinity(device):
     """What a run reads beside the image's edge belongs to another row or term and reaches no result."""
     import torch
