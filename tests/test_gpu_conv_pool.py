@@ -53,6 +53,25 @@ def test_conv_pool(device, N, C, H, W, F, pads, tile, splits, last):
         assert torch.equal(pooled.cpu().nan_to_num(7.0), want.nan_to_num(7.0))
 
 
+def test_conv_without_pool_fits(device):
+    """The pooled epilogue costs the launch without one no workgroup per compute unit."""
+    import torch
+
+    from fluidml_amd import cabi
+    from util import launches
+
+    x, w, b, out = (torch.zeros(*s, device=device) for s in ((1, 64, 16, 16), (128, 64, 3, 3), (128,), (1, 128, 16, 16)))
+    size = ctypes.c_size_t()
+    cabi.call("conv3x3_packed_bytes", ref(w), 1, ctypes.byref(size))
+    packed = torch.zeros(size.value, dtype=torch.uint8, device=device)
+    for tile in (1, 2):
+        call = lambda s: cabi.call("conv3x3_packed_chain", ref(x), ref(w), packed.data_ptr(), 1, ref(b), ref(out), cabi.i64_array([1] * 4),
+                                   ctypes.byref(cabi.make_chain([])), tile << 4 | 1 << 8, s)
+        call(None)
+        (name, fit), = launches(call)
+        assert "ConvPartsKernel" in name and fit >= 3
+
+
 @pytest.mark.parametrize("packed", ["1", "0"])
 def test_graph_conv_pool(device, tmp_path, monkeypatch, packed):
     """The launch takes the pool with it, also where the weights are not packed (two kernels then), and gives the same."""
