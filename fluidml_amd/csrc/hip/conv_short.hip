@@ -169,8 +169,10 @@ int ConvShort(const fl_tensor *in, const fl_tensor *weights, const fl_tensor *bi
   // (us, implicit GEMM and here, one image, kernels of 2 x 2 over eight channels): 16 filters of 56^2 5.7, 5.9, 96^2 6.4, 5.9; 32 of
   // 56^2 5.8, 6.6, 88^2 6.0, 6.6, 96^2 6.6, 6.7, 112^2 7.9, 6.8; 64 of 64^2 6.0, 6.7, 80^2 6.7, 6.8, 96^2 10.9, 6.9; 128 of 28^2 5.9,
   // 6.6, 56^2 6.7, 6.8: the line lies where there are 144 waves, whatever the kernel, the channels and the images.  The 3 x 3 kernels
-  // of unit stride that conv_halo.hip takes otherwise cost more there: few waves 5.9, 5.9 to 6.1, 9216 pixels 6.9, 6.1.
-  const bool halo = KH == 3 && KW == 3 && (!strides || strides[0] == 1) && (!dilations || (dilations[0] == 1 && dilations[1] == 1));
+  // of unit stride that conv_halo.hip takes otherwise cost more there: few waves 5.9, 5.9 to 6.1, 9216 pixels 6.9, 6.1; with
+  // weights that it does not take, channels last, they do not: 64 filters of 14^2 4.9, 6.3.
+  const bool halo = KH == 3 && KW == 3 && (!strides || strides[0] == 1) && (!dilations || (dilations[0] == 1 && dilations[1] == 1)) &&
+                    weights->strides[3] == 1 && weights->strides[2] == 3 && weights->strides[1] == 9;
   if (!halo && out->shape[0] * OH * OW * ((F + 16 * FT - 1) / (16 * FT)) < 144 * 64) return FL_ERR_UNSUPPORTED;
   const int64_t fours = out->shape[0] * OH * ((OW + 3) / 4);
   if (fours > INT32_MAX - 64) return FL_ERR_UNSUPPORTED;

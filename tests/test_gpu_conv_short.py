@@ -118,10 +118,13 @@ def test_conv_short_rule(device, N, F, H, W, kernel, short):
 
     case = (N, 2, F, H, W, kernel, (1, 1), (1, 1), (0, 0, 0, 0))
     x, w, b = (torch.zeros(*s, device=device) for s in ((N, 2, H, W), (F, 2) + kernel, (F,)))
-    call = conv(x, w, b, torch.zeros(N, F, H - kernel[0] + 1, W - kernel[1] + 1, device=device), case)
-    call(None)
-    (name, _), = launches(call)
-    assert ("ConvShortKernel" in name) == short
+    out = torch.zeros(N, F, H - kernel[0] + 1, W - kernel[1] + 1, device=device)
+    # (that kernel does not take weights whose channels come last)
+    for weights, expected in ((w, short), (w.to(memory_format=torch.channels_last), short and kernel != (3, 3))):
+        call = conv(x, weights, b, out, case)
+        call(None)
+        (name, _), = launches(call)
+        assert ("ConvShortKernel" in name) == expected
 
 
 def test_conv_short_switch(device, monkeypatch):
