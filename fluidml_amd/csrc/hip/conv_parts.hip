@@ -56,6 +56,7 @@ struct PartsArgs {
   uint32_t n_splits;
   int32_t chunks_per_split;
   int32_t weight_major;  // consecutive workgroups share weights (else: the patch)
+  int32_t pooled;        // the result is the maximum of each 2 x 2 pixels (the strides are the pooled tensor's)
   const float *bias;
   int32_t sB;
   float *partials;
@@ -65,10 +66,8 @@ struct PartsArgs {
 
 // WF waves along the filters (32 each), 4 / WF along the rows; a wave owns TN tiles of 2 rows x 16 columns.
 // RAGGED: the channels do not come in sixteens; the missing ones read as zero (and are zero in the packed weights).
-// POOLED: the result is the maximum of each 2 x 2 pixels (the strides are the pooled tensor's).  A kernel of its own: its epilogue
-// behind a condition took the other launches more registers and a wave per SIMD (bf16, 8 x 256 x 56^2 -> 512 without a pool 87 -> 104 us,
-// 1 x 512 x 224^2 -> 512 300 -> 343).
-template <int PARTS, int WF, int TN, bool RAGGED, bool POOLED>
+// POOLS: the launch may be a pooled one; see Launch.
+template <int PARTS, int WF, int TN, bool RAGGED, bool POOLS>
 __global__ __launch_bounds__(kThreads, 2) void ConvPartsKernel(float *out, const float *in, const u32x4 *packed, PartsArgs p) {
   // (no __restrict__: loads of memory known to be constant move freely, and the compiler sinks the ones that are
   // requested ahead of time down to their first use; these keep their place between the scheduling barriers below)
@@ -308,7 +307,7 @@ __global__ __launch_bounds__(kThreads, 2) void ConvPartsKernel(float *out, const
 #pragma unroll
     for (int e = 0; e < 16; ++e) vals[e] = acc[j][e] + bias_v[e];
     if (p.chain.n != 0) RunChainBlock<16>(p.chain, vals);
-    if constexpr (POOLED) {
+    if (POOLS && p.pooled != 0) {
       // The four pixels of a window are a lane's neighbour and the two in the next row of sixteen.  Each exchange halves the
       // filters a lane goes on with instead of computing every maximum twice, and all lanes store in the end: lane r of
       // the upper (0) and the lower row (1), column parity c, has the filters e = 4 k + 2 r + c.
@@ -406,17 +405,23 @@ Cut ChooseCut(const PartsArgs &p, int64_t images, int parts) {
   return best;
 }
 
+// The pooled epilogue behind a condition costs launches without a pool registers, and bf16 ones of more than two workgroups per
+// compute unit up to a fifth of their time (8 x 256 x 56^2 -> 512: 86 us without the condition, 104 with it, 896 workgroups; 8 x 256 x
+// 56^2 -> 256, 448, 44.6 and 44.9): those have a kernel without it.  The others share one, because a kernel that has not run just
+// before starts with its instructions missing (VGG-16 of one image with two kernels throughout 438 us, with one 436; bf16 401, 398).
 template <int PARTS, int WF, int TN>
-void Launch(const PartsArgs &p, uint32_t grid, bool pooled, float *out, const float *in, const u32x4 *packed, hipStream_t s) {
-#define FL_PARTS_AS(RAGGED_, POOLED_) \
-  FL_LAUNCH((ConvPartsKernel<PARTS, WF, TN, RAGGED_, POOLED_>), dim3(grid), dim3(kThreads), 0, s, out, in, packed, p)
-  if (p.C % kChunk != 0) {
-    if (pooled) FL_PARTS_AS(true, true);
-    else FL_PARTS_AS(true, false);
-  } else {
-    if (pooled) FL_PARTS_AS(false, true);
-    else FL_PARTS_AS(false, false);
+void Launch(const PartsArgs &p, uint32_t grid, float *out, const float *in, const u32x4 *packed, hipStream_t s) {
+#define FL_PARTS_AS(RAGGED_, POOLS_) \
+  FL_LAUNCH((ConvPartsKernel<PARTS, WF, TN, RAGGED_, POOLS_>), dim3(grid), dim3(kThreads), 0, s, out, in, packed, p)
+  if constexpr (PARTS == 1) {
+    if (!p.pooled && grid > 2 * 256) {
+      if (p.C % kChunk != 0) FL_PARTS_AS(true, false);
+      else FL_PARTS_AS(false, false);
+      return;
+    }
   }
+  if (p.C % kChunk != 0) FL_PARTS_AS(true, true);
+  else FL_PARTS_AS(false, true);
 #undef FL_PARTS_AS
 }
 
@@ -499,6 +504,7 @@ static int PackedChain(const fl_tensor *in, const fl_tensor *weights, const void
   std::memset(&p, 0, sizeof(p));
   p.C = static_cast<int32_t>(C), p.H = static_cast<int32_t>(in->shape[2]), p.W = static_cast<int32_t>(in->shape[3]);
   p.F = static_cast<int32_t>(F), p.OH = static_cast<int32_t>(extent[0]), p.OW = static_cast<int32_t>(extent[1]);
+  p.pooled = pooled ? 1 : 0;
   p.ph = pads ? static_cast<int32_t>(pads[0]) : 0, p.pw = pads ? static_cast<int32_t>(pads[1]) : 0;
   p.chunks = static_cast<int32_t>(Ceil(C, kChunk)), p.ftiles = static_cast<int32_t>(Ceil(F, 32));
   p.sXn = static_cast<int32_t>(in->strides[0]), p.sXc = static_cast<int32_t>(in->strides[1]);
@@ -540,10 +546,10 @@ static int PackedChain(const fl_tensor *in, const fl_tensor *weights, const void
   hipStream_t s = AsStream(stream);
 #define FL_PARTS(PARTS_)                                            \
   do {                                                              \
-    if (cut.wf == 4 && cut.tn == 4) Launch<PARTS_, 4, 4>(p, grid, pooled, o, x, w, s); \
-    else if (cut.wf == 4) Launch<PARTS_, 4, 2>(p, grid, pooled, o, x, w, s);           \
-    else if (cut.tn == 4) Launch<PARTS_, 2, 4>(p, grid, pooled, o, x, w, s);           \
-    else Launch<PARTS_, 2, 2>(p, grid, pooled, o, x, w, s);                            \
+    if (cut.wf == 4 && cut.tn == 4) Launch<PARTS_, 4, 4>(p, grid, o, x, w, s); \
+    else if (cut.wf == 4) Launch<PARTS_, 4, 2>(p, grid, o, x, w, s);           \
+    else if (cut.tn == 4) Launch<PARTS_, 2, 4>(p, grid, o, x, w, s);           \
+    else Launch<PARTS_, 2, 2>(p, grid, o, x, w, s);                            \
   } while (0)
   if (parts == 3) FL_PARTS(3);
   else FL_PARTS(1);

@@ -22,6 +22,8 @@ def ref(t):
     (1, 5, 4, 4, 33, [0, 0, 0, 0]),      # one window
     (3, 31, 5, 33, 96, [2, 0, 1, 2]),
     (1, 160, 6, 6, 160, [1, 1, 1, 1]),   # split by the library's rule
+    (5, 16, 67, 70, 130, [1, 1, 1, 1]),  # more than two workgroups to a compute unit (with two tiles per wave): another kernel without the pool
+    (7, 9, 66, 129, 64, [1, 1, 1, 1]),
 ])
 @pytest.mark.parametrize("tile,splits", [(0, 0), (1, 3), (2, 2)])
 @pytest.mark.parametrize("last", [False, True], ids=["planes", "channels_last"])
@@ -54,22 +56,21 @@ def test_conv_pool(device, N, C, H, W, F, pads, tile, splits, last):
 
 
 def test_conv_without_pool_fits(device):
-    """The pooled epilogue costs the launch without one no workgroup per compute unit."""
+    """The pooled epilogue takes bf16 launches of many workgroups without a pool none of their registers."""
     import torch
 
     from fluidml_amd import cabi
     from util import launches
 
-    x, w, b, out = (torch.zeros(*s, device=device) for s in ((1, 64, 16, 16), (128, 64, 3, 3), (128,), (1, 128, 16, 16)))
+    x, w, b, out = (torch.zeros(*s, device=device) for s in ((4, 64, 112, 112), (128, 64, 3, 3), (128,), (4, 128, 112, 112)))
     size = ctypes.c_size_t()
     cabi.call("conv3x3_packed_bytes", ref(w), 1, ctypes.byref(size))
     packed = torch.zeros(size.value, dtype=torch.uint8, device=device)
-    for tile in (1, 2):
-        call = lambda s: cabi.call("conv3x3_packed_chain", ref(x), ref(w), packed.data_ptr(), 1, ref(b), ref(out), cabi.i64_array([1] * 4),
-                                   ctypes.byref(cabi.make_chain([])), tile << 4 | 1 << 8, s)
-        call(None)
-        (name, fit), = launches(call)
-        assert "ConvPartsKernel" in name and fit >= 3
+    call = lambda s: cabi.call("conv3x3_packed_chain", ref(x), ref(w), packed.data_ptr(), 1, ref(b), ref(out), cabi.i64_array([1] * 4),
+                               ctypes.byref(cabi.make_chain([])), 1 << 4 | 1 << 8, s)  # (two tiles per wave: 784 workgroups)
+    call(None)
+    (name, fit), = launches(call)
+    assert "ConvPartsKernel" in name and fit >= 3
 
 
 @pytest.mark.parametrize("packed", ["1", "0"])
