@@ -16,18 +16,24 @@
 //     taps (3.8 conflict cycles per LDS instruction, reads and writes of 16 bytes per lane together);
 //   * per chunk of 16 channels one barrier, TN x 54 products per wave; LDS is double buffered and the next chunk's
 //     loads are in flight across the products;
-//   * the loads that run ahead are held in their place by scheduling barriers (the compiler moves them down to their use);
+//   * the loads that run ahead are held in their place by scheduling barriers (the compiler moves them down to their use), those of
+//     the patch one by one between the products: sixteen in a row hold up the wave at the address unit, and its products behind
+//     them (one part, 8 x 512 x 28^2 -> 512: 51.5 -> 43.7 us, of 30 that the products alone take; three parts 160 -> 156);
+//   * one part, where a chunk's products take 0.5 us and one or two workgroups share a compute unit: two chunks of activations and
+//     17 taps of weights in flight, the conversion of the next chunk between the products (8 x 512 x 14^2 -> 512: 27 -> 22 us
+//     before the loads were spread).  With more workgroups per compute unit those fill the waits, and the registers and
+//     the longer start cost more (8 x 64 x 224^2 -> 64: 54 us with one chunk ahead, 60 with two);
 //   * few tiles: the channels of a tile go to several workgroups, whose partial tiles meet in the stream's workspace and
 //     are added in split order by the wave that arrives last.
 // Measured against conv_halo.hip, bias and ReLU included (us; TFLOP/s of the convolution's own operations):
 //   images x channels x size -> filters        fp32 before -> now            bf16 before -> now
 //   8 x  64 x 224^2 ->  64                     289 -> 161 (184)               95 -> 62 (480)
-//   8 x 128 x 112^2 -> 128                     286 -> 154 (192)               87 -> 52 (573)
-//   8 x 256 x  56^2 -> 256                     290 -> 152 (194)              105 -> 46 (642)
-//   8 x 512 x  28^2 -> 512                     324 -> 159 (187)              108 -> 55 (542)
-//   8 x 512 x  14^2 -> 512                      92 ->  50 (147)               35 -> 27 (276)
-//   1 x 256 x  56^2 -> 256                      52 ->  31 (118)               23 -> 16 (230)
-//   4 x 256 x  37^2 -> 256                     156 ->  46 (142)              106 -> 20 (327)
+//   8 x 128 x 112^2 -> 128                     286 -> 154 (192)               87 -> 50 (595)
+//   8 x 256 x  56^2 -> 256                     290 -> 150 (197)              105 -> 43 (688)
+//   8 x 512 x  28^2 -> 512                     324 -> 156 (190)              108 -> 43 (688)
+//   8 x 512 x  14^2 -> 512                      92 ->  50 (147)               35 -> 21 (352)
+//   1 x 256 x  56^2 -> 256                      52 ->  30 (123)               23 -> 15 (247)
+//   4 x 256 x  37^2 -> 256                     156 ->  46 (142)              106 -> 17 (384)
 // A 2 x 2 pool behind the chain is taken in the epilogue, where neighbouring lanes hold whole windows: a quarter of the result
 // is written and nothing read back (us, convolution and pool): 8 x 64 x 224^2 fp32 166 + 18 -> 162, bf16 70 + 18 -> 64;
 // 8 x 256 x 56^2 fp32 158 + 6 -> 153; the five pools of VGG-16 at batch 8 43 -> 0 altogether.
@@ -43,8 +49,10 @@ constexpr int kThreads = 256;
 constexpr int kChunk = 16;   // input channels per chunk
 constexpr int kCols = 16;    // output columns of a workgroup's tile
 constexpr int kPatchCols = kCols + 2;
-constexpr int kAhead = 2;    // taps whose weights are in flight
-constexpr int kSlots = kAhead + 1;
+// Taps whose weights are in flight while DEPTH chunks of activations are: one fewer than there are places for them, and the places
+// divide the taps of DEPTH chunks.
+constexpr int Ahead(int depth) { return depth == 2 ? 17 : 2; }
+constexpr int kMostAhead = Ahead(2);
 
 struct PartsArgs {
   int32_t C, H, W, F, OH, OW;
@@ -67,14 +75,19 @@ struct PartsArgs {
 // WF waves along the filters (32 each), 4 / WF along the rows; a wave owns TN tiles of 2 rows x 16 columns.
 // RAGGED: the channels do not come in sixteens; the missing ones read as zero (and are zero in the packed weights).
 // POOLS: the launch may be a pooled one; see Launch.
-template <int PARTS, int WF, int TN, bool RAGGED, bool POOLS>
-__global__ __launch_bounds__(kThreads, 2) void ConvPartsKernel(float *out, const float *in, const u32x4 *packed, PartsArgs p) {
+// DEPTH: chunks of activations in flight; 2 with one part and up to two workgroups per compute unit (see above).
+// (Three workgroups per compute unit where one part meets 64 filters, 8 x 64 x 224^2 -> 64: 54 us, with two 57; with 128 filters
+// they are slower, 8 x 128 x 112^2 -> 128: 46 against 44.5.)
+template <int PARTS, int WF, int TN, bool RAGGED, bool POOLS, int DEPTH>
+__global__ __launch_bounds__(kThreads, PARTS == 1 && DEPTH == 1 && WF == 2 ? 3 : 2) void ConvPartsKernel(
+    float *out, const float *in, const u32x4 *packed, PartsArgs p) {
   // (no __restrict__: loads of memory known to be constant move freely, and the compiler sinks the ones that are
   // requested ahead of time down to their first use; these keep their place between the scheduling barriers below)
   constexpr int kRows = 2 * TN * (4 / WF);
   constexpr int kPix = (kRows + 2) * kPatchCols;
   constexpr int kItems = 2 * kPix;  // (channel half, pixel): eight channels each
   constexpr int kPer = (kItems + kThreads - 1) / kThreads;
+  constexpr int kAhead = Ahead(DEPTH), kSlots = kAhead + 1;
   __shared__ u32x4 lds[2 * PARTS * kItems];
   __shared__ uint32_t tiny_inputs;  // (BadSum)
   const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
@@ -113,45 +126,36 @@ __global__ __launch_bounds__(kThreads, 2) void ConvPartsKernel(float *out, const
               static_cast<uint32_t>(iw) < static_cast<uint32_t>(p.W);
     x_at[t] = x_ok[t] ? 4u * (ih * p.sXh + iw * p.sXw + (RAGGED ? 0 : 8 * h * p.sXc)) : 0u;
   }
-  float xr[kPer][8];
+  float xr[DEPTH][kPer][8];
   uint32_t tiny_key = 0xffffffffu;
   if (PARTS == 3 && tid == 0) tiny_inputs = 0;
-  auto load_patch = [&](int c) {
-#pragma unroll
-    for (int t = 0; t < kPer; ++t) {
-      if constexpr (RAGGED) {
-        const int c8 = c * kChunk + 8 * ((tid + t * kThreads) / kPix);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          xr[t][e] = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(image) +
-                                                      (4u * min(c8 + e, p.C - 1) * p.sXc + x_at[t]));
-        }
-      } else {
-        const char *plane = reinterpret_cast<const char *>(image + static_cast<int64_t>(c) * kChunk * p.sXc);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          xr[t][e] = *reinterpret_cast<const float *>(plane + static_cast<int64_t>(e) * p.sXc * 4 + x_at[t]);
-        }
-      }
+  // value v of this thread's of chunk c: channel v % 8 of item v / 8
+  auto load_value = [&](int c, auto set_c, auto value_c) {
+    constexpr int S = decltype(set_c)::value, t = decltype(value_c)::value / 8, e = decltype(value_c)::value % 8;
+    if constexpr (RAGGED) {
+      const int c8 = c * kChunk + 8 * ((tid + t * kThreads) / kPix);
+      xr[S][t][e] = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(image) +
+                                                     (4u * min(c8 + e, p.C - 1) * p.sXc + x_at[t]));
+    } else {
+      const char *plane = reinterpret_cast<const char *>(image + (static_cast<int64_t>(c) * kChunk + e) * p.sXc);
+      xr[S][t][e] = *reinterpret_cast<const float *>(plane + x_at[t]);
     }
   };
-  auto store_patch = [&](int c, int buf) {
+  auto store_item = [&](int c, int buf, auto set_c, int t) {
+    constexpr int S = decltype(set_c)::value;
+    const int i = tid + t * kThreads;
+    if (i < kItems) {
+      float x[8];
 #pragma unroll
-    for (int t = 0; t < kPer; ++t) {
-      const int i = tid + t * kThreads;
-      if (i < kItems) {
-        float x[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const bool ok = x_ok[t] && (!RAGGED || c * kChunk + 8 * (i / kPix) + e < p.C);
-          x[e] = ok ? xr[t][e] : 0.0f;
-        }
-        if constexpr (PARTS == 3) tiny_key = TinyKey(tiny_key, x);
-        u32x4 parts[PARTS];
-        SplitParts<PARTS>(x, parts);
-#pragma unroll
-        for (int s = 0; s < PARTS; ++s) lds[(buf * PARTS + s) * kItems + i] = parts[s];
+      for (int e = 0; e < 8; ++e) {
+        const bool ok = x_ok[t] && (!RAGGED || c * kChunk + 8 * (i / kPix) + e < p.C);
+        x[e] = ok ? xr[S][t][e] : 0.0f;
       }
+      if constexpr (PARTS == 3) tiny_key = TinyKey(tiny_key, x);
+      u32x4 parts[PARTS];
+      SplitParts<PARTS>(x, parts);
+#pragma unroll
+      for (int s = 0; s < PARTS; ++s) lds[(buf * PARTS + s) * kItems + i] = parts[s];
     }
   };
 
@@ -172,12 +176,18 @@ __global__ __launch_bounds__(kThreads, 2) void ConvPartsKernel(float *out, const
   const int py = wp * 2 * TN + lrow / 16, px = lrow % 16;
   const int b_base = half * kPix + py * kPatchCols + px;
 
-  load_patch(c_first);
+  // (without a condition, so that the compiler can count the loads in flight: past the end the last chunk again)
+  StaticFor<DEPTH>([&](auto d) {
+    StaticFor<8 * kPer>([&](auto v) { load_value(min(c_first + decltype(d)::value, c_end - 1), d, v); });
+  });
   StaticFor<kAhead>([&](auto t) { load_a(decltype(t)::value, t); });
-  store_patch(c_first, 0);
+#pragma unroll
+  for (int t = 0; t < kPer; ++t) store_item(c_first, 0, std::integral_constant<int, 0>{}, t);
   __syncthreads();
-  for (int c = c_first; c < c_end; ++c) {
-    const int buf = (c - c_first) & 1;
+  // Chunk c: its patch lies in LDS buffer (c - c_first) % 2, the next one's is in the registers of set (c + 1 - c_first) % DEPTH.
+  auto chunk = [&](int c, auto idx_c) __attribute__((always_inline)) {
+    constexpr int I = decltype(idx_c)::value;
+    const int buf = DEPTH == 1 ? (c - c_first) & 1 : I;
     const u32x4 *xs = lds + buf * PARTS * kItems + b_base;
     u32x4 b[2][PARTS];  // operand of the current tile and tap, and of the next
     auto load_b = [&](auto step_c) {
@@ -186,22 +196,42 @@ __global__ __launch_bounds__(kThreads, 2) void ConvPartsKernel(float *out, const
       for (int s = 0; s < PARTS; ++s) b[step % 2][s] = xs[s * kItems + (2 * j + tap / 3) * kPatchCols + tap % 3];
     };
     load_b(std::integral_constant<int, 0>{});
-    // (without a condition, so that the compiler can count the loads in flight: the last chunk requests itself again)
-    load_patch(min(c + 1, c_end - 1));
+    const int c_load = min(c + DEPTH, c_end - 1);
     StaticFor<9 * TN>([&](auto step_c) {
-      constexpr int step = decltype(step_c)::value, tap = step / TN, j = step % TN;
+      constexpr int step = decltype(step_c)::value, tap = step / TN, j = step % TN, place = I * 9 + tap;
       // (runs kAhead taps past this wave's chunks at the end: other weights, or the padding behind the last ones)
-      if constexpr (j == 0) load_a(tap + kAhead, std::integral_constant<int, (tap + kAhead) % kSlots>{});
+      if constexpr (j == 0) load_a(tap + kAhead, std::integral_constant<int, (place + kAhead) % kSlots>{});
       if constexpr (step + 1 < 9 * TN) load_b(std::integral_constant<int, step + 1>{});
-      // nothing moves across: the compiler otherwise sinks both kinds of loads down to their first use
+      // the loads of the patch one by one: a wave that issues them in a row waits for the address unit, and its products behind it
+      constexpr int kLoadSteps = DEPTH == 1 ? 4 * TN : 9 * TN;
+      StaticFor<8 * kPer>([&](auto v) {
+        if constexpr (step == v * kLoadSteps / (8 * kPer)) load_value(c_load, std::integral_constant<int, I % DEPTH>{}, v);
+      });
+      // nothing moves across: the compiler otherwise sinks all kinds of loads down to their first use
       __builtin_amdgcn_sched_barrier(0);
-      MfmaParts<PARTS>(a[tap % kSlots], b[step % 2], acc[j], low[PARTS == 3 ? j : 0]);
+      MfmaParts<PARTS>(a[place % kSlots], b[step % 2], acc[j], low[PARTS == 3 ? j : 0]);
+      // the next chunk on its way into LDS between the products of the last third of the taps, where nobody else fills the pipe
+      if constexpr (DEPTH == 2) {
+        StaticFor<kPer>([&](auto t) {
+          if constexpr (step == 6 * TN + t * 3 * TN / kPer) store_item(min(c + 1, c_end - 1), buf ^ 1, std::integral_constant<int, 1 - I>{}, t);
+        });
+      }
     });
+    if constexpr (DEPTH == 1) {
+      if (c + 1 < c_end) StaticFor<kPer>([&](auto t) { store_item(c + 1, buf ^ 1, std::integral_constant<int, 0>{}, t); });
+    }
     a_src += 9 * PARTS * 64;
-    if (c + 1 < c_end) store_patch(c + 1, buf ^ 1);
     // one barrier per chunk: the buffer written here was last read in the previous chunk, and every wave passed the
     // previous barrier only after finishing that read
     __syncthreads();
+  };
+  for (int c = c_first;;) {  // (every workgroup has a chunk)
+    chunk(c, std::integral_constant<int, 0>{});
+    if (++c >= c_end) break;
+    if constexpr (DEPTH == 2) {
+      chunk(c, std::integral_constant<int, 1>{});
+      if (++c >= c_end) break;
+    }
   }
 
   if constexpr (PARTS == 3) {
@@ -267,7 +297,7 @@ __global__ __launch_bounds__(kThreads, 2) void ConvPartsKernel(float *out, const
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[j][e] = 0.0f;
-    constexpr uint32_t kTogether = TN == 2 ? 4 : 1;  // splits whose loads are in flight together
+    constexpr uint32_t kTogether = TN == 2 ? 4 : 2;  // splits whose loads are in flight together
     for (uint32_t z0 = 0; z0 < n_splits; z0 += kTogether) {
       float part[kTogether][TN][16];
 #pragma unroll
@@ -411,17 +441,22 @@ Cut ChooseCut(const PartsArgs &p, int64_t images, int parts) {
 // before starts with its instructions missing (VGG-16 of one image with two kernels throughout 438 us, with one 436; bf16 401, 398).
 template <int PARTS, int WF, int TN>
 void Launch(const PartsArgs &p, uint32_t grid, float *out, const float *in, const u32x4 *packed, hipStream_t s) {
-#define FL_PARTS_AS(RAGGED_, POOLS_) \
-  FL_LAUNCH((ConvPartsKernel<PARTS, WF, TN, RAGGED_, POOLS_>), dim3(grid), dim3(kThreads), 0, s, out, in, packed, p)
+#define FL_PARTS_AS(RAGGED_, POOLS_, DEPTH_) \
+  FL_LAUNCH((ConvPartsKernel<PARTS, WF, TN, RAGGED_, POOLS_, DEPTH_>), dim3(grid), dim3(kThreads), 0, s, out, in, packed, p)
   if constexpr (PARTS == 1) {
-    if (!p.pooled && grid > 2 * 256) {
-      if (p.C % kChunk != 0) FL_PARTS_AS(true, false);
-      else FL_PARTS_AS(false, false);
+    if (grid <= 2 * 256) {
+      if (p.C % kChunk != 0) FL_PARTS_AS(true, true, 2);
+      else FL_PARTS_AS(false, true, 2);
+      return;
+    }
+    if (!p.pooled) {
+      if (p.C % kChunk != 0) FL_PARTS_AS(true, false, 1);
+      else FL_PARTS_AS(false, false, 1);
       return;
     }
   }
-  if (p.C % kChunk != 0) FL_PARTS_AS(true, true);
-  else FL_PARTS_AS(false, true);
+  if (p.C % kChunk != 0) FL_PARTS_AS(true, true, 1);
+  else FL_PARTS_AS(false, true, 1);
 #undef FL_PARTS_AS
 }
 
@@ -442,7 +477,7 @@ int fluidml_hip_conv3x3_packed_bytes(const fl_tensor *weights, int32_t parts, si
   FL_CHECK(CheckView(weights));
   if (parts != 1 && parts != 3) return FL_ERR_ATTR;
   if (!Fits(weights)) return FL_ERR_UNSUPPORTED;
-  const int64_t taps = Ceil(weights->shape[0], 32) * Ceil(weights->shape[1], kChunk) * 9 + kAhead;
+  const int64_t taps = Ceil(weights->shape[0], 32) * Ceil(weights->shape[1], kChunk) * 9 + (parts == 1 ? kMostAhead : Ahead(1));
   *bytes = static_cast<size_t>(taps) * parts * 1024;
   return FL_OK;
 }

@@ -72,6 +72,25 @@ def test_packed_conv(device, N, C, H, W, F, pads, tile, splits):
     assert_close(got, _oracle(rounded(x), rounded(w), None, pads, relu=False), what="bf16")
 
 
+@pytest.mark.parametrize("N,C,H,W,F,tile", [
+    (1, 16, 10, 18, 64, 1),      # a single chunk
+    (1, 17, 10, 18, 128, 2),     # two, the second of one channel
+    (2, 48, 9, 20, 160, 1),      # three: the second set of registers stays behind
+    (1, 80, 12, 7, 96, 2),       # five
+    (8, 40, 140, 60, 64, 1),     # more than two workgroups per compute unit: 576 of 64 filters, the last chunk half full
+    (3, 16, 171, 62, 130, 1),    # 1032 of 128 filters, half of them nearly empty
+])
+def test_packed_conv_bf16_chunks(device, N, C, H, W, F, tile):
+    """Exact: operands of a few bits, so that every product and every sum of them is a float32."""
+    print("[case]", N, C, H, W, F, tile, flush=True)
+    rng = np.random.default_rng(5)
+    x = rng.integers(-8, 9, (N, C, H, W)).astype(np.float32)
+    w = rng.integers(-4, 5, (F, C, 3, 3)).astype(np.float32)
+    bias = rng.integers(-16, 17, F).astype(np.float32)
+    got = _run(device, x, w, bias, [1, 1, 1, 1], 1, tile, 1)
+    np.testing.assert_array_equal(got, _oracle(x, w, bias, [1, 1, 1, 1]))
+
+
 def test_packed_conv_layouts(device):
     x, w, bias = _operands(8, 2, 24, 11, 18, 40)
     want = _oracle(x, w, bias, [1, 1, 1, 1])
