@@ -10,6 +10,9 @@
 //   * The rows of A are split into their parts once per workgroup, on their way from registers into LDS, where they lie
 //     as [part][k / 8][row][8]: a lane's A operand is one 128-bit read, 32 consecutive places per half wave.  The places
 //     of one k / 8 are padded, so that the writes (consecutive lanes: consecutive k of a row) spread over the banks.
+//   * The loads of a chunk leave between the products of an earlier one, a few per product (three parts): in a row behind the
+//     barrier, sixteen cycles of the address unit each, they held up all waves and the products behind them (512 x 3072 x 768
+//     22.4 -> 19.9 us, 256 x 3072 x 768 16.6 -> 14.6, 512 x 768 x 3072 25.0 -> 23.0, 256 x 50304 x 512 100 -> 93).
 //   * WN waves side by side times KS = 4 / WN slices of K; two steps of 16 k per wave and chunk, one barrier per chunk, LDS
 //     double buffered, DEPTH chunks of both operands in flight in registers: a launch of a small transformer has a few
 //     chunks per workgroup and is a chain of trips to memory otherwise.
@@ -103,23 +106,20 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
   floatx4 ar[kSets][kPer][2];
   u32x4 br[kSets][kSteps][PARTS];
   const int last = c_end - 1;
-  auto load_chunk = [&](int c, auto set_c) {
-    constexpr int S = decltype(set_c)::value;
+  constexpr int kLoads = 2 * kPer + kSteps * PARTS;  // of a wave per chunk, 16 bytes per lane each
+  // load i of chunk c: the items of A, then the weights
+  auto load = [&](int c, auto set_c, auto load_c) __attribute__((always_inline)) {
+    constexpr int S = decltype(set_c)::value, i = decltype(load_c)::value;
     const int cc = min(c, last);  // (past the end: the last chunk again, so that the number of loads in flight is known)
-    const uint32_t at = 4u * static_cast<uint32_t>(cc) * BK;
-#pragma unroll
-    for (int t = 0; t < kPer; ++t) {
+    if constexpr (i < 2 * kPer) {
       // (k past K: the first eight of the row, replaced by zero when they are stored)
-      const uint32_t off = a_at[t] + (cc * BK + a_k[t] < p.K ? at : 0u - 4u * a_k[t]);
-      ar[S][t][0] = *reinterpret_cast<const floatx4 *>(a_base + off);
-      ar[S][t][1] = *reinterpret_cast<const floatx4 *>(a_base + off + 16);
-    }
-    const int step0 = cc * kChunkSteps + ks * kSteps;
-#pragma unroll
-    for (int u = 0; u < kSteps; ++u) {
-      const char *from = b_base + static_cast<int64_t>(min(step0 + u, all_steps - 1)) * (PARTS * 1024);  // (uniform)
-#pragma unroll
-      for (int s = 0; s < PARTS; ++s) br[S][u][s] = *reinterpret_cast<const u32x4 *>(from + s * 1024 + lane * 16u);
+      constexpr int t = i / 2;
+      const uint32_t off = a_at[t] + (cc * BK + a_k[t] < p.K ? 4u * static_cast<uint32_t>(cc) * BK : 0u - 4u * a_k[t]);
+      ar[S][t][i % 2] = *reinterpret_cast<const floatx4 *>(a_base + off + 16 * (i % 2));
+    } else {
+      constexpr int u = (i - 2 * kPer) / PARTS, s = (i - 2 * kPer) % PARTS;
+      const char *from = b_base + static_cast<int64_t>(min(cc * kChunkSteps + ks * kSteps + u, all_steps - 1)) * (PARTS * 1024);  // (uniform)
+      br[S][u][s] = *reinterpret_cast<const u32x4 *>(from + s * 1024 + lane * 16u);
     }
   };
   // item t of chunk c: its parts, into LDS
@@ -141,7 +141,9 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[i][e] = low[PARTS == 3 ? i : 0][e] = 0.0f;
 
-  StaticFor<DEPTH>([&](auto d) { load_chunk(c_begin + decltype(d)::value, d); });
+  StaticFor<DEPTH>([&](auto d) {
+    StaticFor<kLoads>([&](auto i) { load(c_begin + decltype(d)::value, d, i); });
+  });
 
   // ---- what the epilogue needs, requested behind the first tiles ------------------------------------------------
   const int n = n0 + wn * 32 + lrow;
@@ -158,18 +160,26 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
     p.div_inner.DivMod(static_cast<uint32_t>(n < p.N ? n : 0), hi, lo);
     col = static_cast<int64_t>(hi) * sCn_outer + static_cast<int64_t>(lo) * sCn;
   }
-  constexpr bool PRE_ADD = EXTRA != 0 && kShare <= 8;
-  float pre_add[PRE_ADD ? kShare : 1], pre_add2[PRE_ADD ? kShare : 1];
-  if constexpr (PRE_ADD) {
+  // the addends: with a few values per lane here, else behind the K loop, where the registers of the tiles are free; either way the
+  // exchange of the slices and splits lies between them and their use (asked for behind it, 512 x 768 x 3072 with an addend and
+  // row statistics took 29.3 us, now 28.1)
+  constexpr bool EARLY_ADD = EXTRA != 0 && kShare <= 8;
+  float pre_add[EXTRA != 0 ? kShare : 1], pre_add2[EXTRA != 0 ? kShare : 1];
+  auto load_addends = [&] {
+    if (p.addend == nullptr) return;
 #pragma unroll
     for (int v = 0; v < kShare; ++v) {
       const int m = m0 + share_row(v);
-      const bool inside = m < p.M && n < p.N;
-      const int64_t at = static_cast<int64_t>(m) * sCm + col;
-      pre_add[v] = p.addend != nullptr && inside ? p.addend[at] : 0.0f;
-      pre_add2[v] = p.addend2 != nullptr && inside ? p.addend2[at] : 0.0f;
+      pre_add[v] = m < p.M && n < p.N ? p.addend[static_cast<int64_t>(m) * sCm + col] : 0.0f;
     }
-  }
+    if (p.addend2 == nullptr) return;
+#pragma unroll
+    for (int v = 0; v < kShare; ++v) {
+      const int m = m0 + share_row(v);
+      pre_add2[v] = m < p.M && n < p.N ? p.addend2[static_cast<int64_t>(m) * sCm + col] : 0.0f;
+    }
+  };
+  if constexpr (EARLY_ADD) load_addends();
   constexpr int kNormLanes = NORM ? (kThreads / BM > 16 ? 16 : kThreads / BM) : 1;  // lanes that merge a row's statistics
   constexpr int kNormPer = 32 / kNormLanes;                                         // partials each: rows of up to 1024 elements
   float ln_col = 0.0f, ln_col2 = 0.0f;
@@ -229,10 +239,12 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
   // a compute unit nobody else fills the matrix pipe while a wave converts, so the conversion of the next chunk runs
   // between the products of this one: a product keeps the pipe busy for 32 cycles, in which eight other instructions issue.
   constexpr int kGroups = kSteps * TM;
-  auto chunk = [&](int c, auto idx_c) {
+  auto chunk = [&](int c, auto idx_c) __attribute__((always_inline)) {
     constexpr int I = decltype(idx_c)::value;
-    load_chunk(c + DEPTH, std::integral_constant<int, (I + DEPTH) % kSets>{});
-    __builtin_amdgcn_sched_barrier(0);  // (the loads keep their place: they are DEPTH chunks early)
+    if constexpr (PARTS == 1) {
+      StaticFor<kLoads>([&](auto i) { load(c + DEPTH, std::integral_constant<int, (I + DEPTH) % kSets>{}, i); });
+      __builtin_amdgcn_sched_barrier(0);  // (the loads keep their place: they are DEPTH chunks early)
+    }
     const u32x4 *as = lds + (I % 2) * kStage + (ks * kSteps * 2 + half) * kPitch + lrow;
     u32x4 a[2][PARTS];
     auto load_a = [&](int g) {
@@ -240,9 +252,15 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
       for (int s = 0; s < PARTS; ++s) a[g % 2][s] = as[s * (kK8 * kPitch) + 2 * (g / TM) * kPitch + 32 * (g % TM)];
     };
     load_a(0);
-#pragma unroll
-    for (int g = 0; g < kGroups; ++g) {
-      if (g + 1 < kGroups) load_a(g + 1);
+    StaticFor<kGroups>([&](auto group_c) {
+      constexpr int g = decltype(group_c)::value;
+      if constexpr (g + 1 < kGroups) load_a(g + 1);
+      if constexpr (PARTS == 3) {
+        StaticFor<kLoads>([&](auto i) {
+          if constexpr (i * kGroups / kLoads == g) load(c + DEPTH, std::integral_constant<int, (I + DEPTH) % kSets>{}, i);
+        });
+        __builtin_amdgcn_sched_barrier(0);
+      }
       MfmaParts<PARTS>(a[g % 2], br[I % kSets][g / TM], acc[g % TM], low[PARTS == 3 ? g % TM : 0]);
       // (also behind the last chunk, which is then converted again: a condition would end the block that is scheduled)
 #pragma unroll
@@ -254,7 +272,7 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // a product
         __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);  // vector instructions
       }
-    }
+    });
     // one barrier per chunk: the buffer written here was last read in the previous chunk
     __syncthreads();
   };
@@ -319,6 +337,8 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
       }
     }
   }
+
+  if constexpr (EXTRA != 0 && !EARLY_ADD) load_addends();
 
   // ---- the K slices of the workgroup meet in LDS; every wave takes its share on --------------------------------
   float vals[kShare];
@@ -402,15 +422,8 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
         float add[EV], add2[EV];
 #pragma unroll
         for (int e = 0; e < EV; ++e) {
-          if constexpr (PRE_ADD) {
-            add[e] = pre_add[v0 + e];
-            add2[e] = pre_add2[v0 + e];
-          } else {
-            const int m = m0 + share_row(v0 + e);
-            const bool inside = m < p.M && n < p.N;
-            add[e] = inside ? p.addend[static_cast<int64_t>(m) * sCm + col] : 0.0f;
-            add2[e] = p.addend2 != nullptr && inside ? p.addend2[static_cast<int64_t>(m) * sCm + col] : 0.0f;
-          }
+          add[e] = pre_add[v0 + e];
+          add2[e] = pre_add2[v0 + e];
         }
         if (p.ln_mode == 2) {
           // the addend is the un-normalised tensor of a LayerNormalization: normalise it on the way in
