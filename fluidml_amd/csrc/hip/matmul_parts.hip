@@ -31,6 +31,11 @@ namespace {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
+// four floats next to each other, at any float's address, one access
+struct __attribute__((packed, aligned(4))) FourFloats {
+  float v[4];
+};
+
 constexpr int kPackThreads = 256;
 constexpr int kSteps = 2;  // steps of 16 k per wave and chunk
 
@@ -441,10 +446,28 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
         }
       }
     }
+    if (sCm == 1) {
+      // a result whose rows lie next to each other (K of an attention block, a third of its launch): a lane's four rows in one
+      // store.  One by one each takes a line per lane, four times over (512 rows, 3 x 768 columns, K = 768: 22.9 us, now 20.4; the
+      // few-rows kernel and the tiled one at 37 and 128 rows gained nothing by the same)
 #pragma unroll
-    for (int e = 0; e < EV; ++e) {
-      const int m = m0 + share_row(v0 + e);
-      if (m < p.M && n < p.N) C[static_cast<int64_t>(m) * sCm + col] = out[e];
+      for (int e = 0; e < EV; e += 4) {
+        const int m = m0 + share_row(v0 + e);
+        if (m + 3 < p.M && n < p.N) {
+          *reinterpret_cast<FourFloats *>(C + (m + col)) = {{out[e], out[e + 1], out[e + 2], out[e + 3]}};
+        } else {
+#pragma unroll
+          for (int u = 0; u < 3; ++u) {
+            if (m + u < p.M && n < p.N) C[m + u + col] = out[e + u];
+          }
+        }
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < EV; ++e) {
+        const int m = m0 + share_row(v0 + e);
+        if (m < p.M && n < p.N) C[static_cast<int64_t>(m) * sCm + col] = out[e];
+      }
     }
     if constexpr (NORM) {
       if (p.ln_stats_out != nullptr) {

@@ -99,6 +99,26 @@ def test_packed_tiles(device, tile, M, K, N):
 
 
 @pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("M,N,pad", [(64, 64, 0), (66, 72, 1), (97, 130, 3), (131, 33, 0)])
+def test_packed_results_with_rows_side_by_side(device, tile, M, N, pad):
+    """The result's rows at unit stride, runs of four of them whole and cut off, at addresses that are no multiple of 16 bytes."""
+    with Problem(device, M, 256, N) as p:
+        p.pack()
+        out = p.torch.full((N * (M + pad) + 4,), 9.0, device=device)
+        for first in (0, 1):
+            view = out[first:]
+            ref = p.ref(view, (M, N), (1, M + pad))
+            rc = p.cabi.lib.fluidml_hip_matmul_chain(p.ref(p.x), p.ref(p.w[0]), p.ref(p.b[0]), ref, ctypes.byref(p.cabi.make_chain([])),
+                                                     flags_of(tile), None)
+            assert rc == 0
+            got = p.torch.as_strided(view, (M, N), (1, M + pad))
+            close(got, p.x.double() @ p.w[0].double() + p.b[0].double(), "transposed")
+            if pad:
+                assert (p.torch.as_strided(view, (N - 1, pad), (M + pad, 1), view.storage_offset() + M) == 9.0).all()
+            out.fill_(9.0)
+
+
+@pytest.mark.parametrize("tile", TILES)
 def test_packed_bf16(device, tile):
     for M, K, N in [(33, 264, 65), (128, 768, 96)]:
         with Problem(device, M, K, N) as p:
