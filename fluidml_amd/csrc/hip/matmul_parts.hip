@@ -50,8 +50,8 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
   // 16-byte places per k / 8: sixteen lanes write kK8 values of k / 8 in 16 / kK8 rows, to sixteen different places
   constexpr int kPitch = BM + (kK8 >= 16 ? 1 : 16 / kK8);
   constexpr int kItems = BM * kK8;                  // eight k of a row
-  constexpr int kPer = kItems / kThreads;
-  static_assert(kItems % kThreads == 0, "every thread stages the same number of items");
+  constexpr int kPer = (kItems + kThreads - 1) / kThreads;
+  constexpr bool kWhole = kItems % kThreads == 0;   // else the last item of some threads lies past the tile's rows
   constexpr int kStage = PARTS * kK8 * kPitch;      // 16-byte places per LDS buffer
   constexpr int kShare = TM * 16 / KS;              // values per lane a wave finishes
   constexpr int kRed = KS > 1 ? TM * kWaves * 256 : 0;   // 16-byte places of the K slices' partial tiles
@@ -137,7 +137,9 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
     u32x4 parts[PARTS];
     SplitParts<PARTS>(x, parts);
 #pragma unroll
-    for (int s = 0; s < PARTS; ++s) lds[buf * kStage + s * (kK8 * kPitch) + a_to[t]] = parts[s];
+    for (int s = 0; s < PARTS; ++s) {
+      if (kWhole || t + 1 < kPer || tid + t * kThreads < kItems) lds[buf * kStage + s * (kK8 * kPitch) + a_to[t]] = parts[s];
+    }
   };
 
   floatx16 acc[TM], low[PARTS == 3 ? TM : 1];
@@ -601,6 +603,12 @@ int LaunchTile(MatmulArgs q, uint32_t n_batch, float *C, const float *A, hipStre
   return FL_OK;
 }
 
+// 96 rows by 128 columns, the rule's alone: 65 to 96 rows against so many columns that tiles of 96 rows still fill the chip.  Two
+// tiles of 64 rows multiply up to twice as many rows and take the weights in twice (us, 64x128 and this: 77 x 50304 x 512 57,
+// 50; 65 rows 56, 50; 96 rows 58, 51; 80 x 33024 x 256 27.1, 25.6; 90 x 40000 x 1024 77, 76).  With more rows nothing is gained
+// (280 x 33000 x 768 109, 111), with one part neither (90 x 40000 x 1024 32.4, 34.7).
+constexpr int kPacked96x128 = 1 << 8;
+
 template <int PARTS, int EXTRA>
 int LaunchTiles(const MatmulArgs &p, uint32_t n_batch, float *C, const float *A, hipStream_t s, int tile, int splits) {
   switch (tile) {
@@ -608,8 +616,12 @@ int LaunchTiles(const MatmulArgs &p, uint32_t n_batch, float *C, const float *A,
     case FL_TILE_PACKED_64x64: return LaunchTile<PARTS, 2, 2, 2, 2, EXTRA>(p, n_batch, C, A, s, splits);
     case FL_TILE_PACKED_64x128: return LaunchTile<PARTS, 2, 4, 1, 3, EXTRA>(p, n_batch, C, A, s, splits);
     case FL_TILE_PACKED_64x128_K2: return LaunchTile<PARTS, 2, 4, 2, 2, EXTRA>(p, n_batch, C, A, s, splits);
-    default: return FL_ERR_UNSUPPORTED;
+    default: break;
   }
+  if constexpr (PARTS == 3) {
+    if (tile == kPacked96x128) return LaunchTile<PARTS, 3, 4, 1, 1, EXTRA>(p, n_batch, C, A, s, splits);
+  }
+  return FL_ERR_UNSUPPORTED;
 }
 
 }  // namespace
@@ -663,7 +675,8 @@ int LaunchPacked(const MatmulArgs &args, uint32_t n_batch, bool extra, int parts
   int tile = choice.tile, splits = choice.splits > 0 ? choice.splits : 1;
   if (tile == FL_TILE_RULE) {
     if (choice.splits != 0 || !WorthPacking(p.M, static_cast<int64_t>(p.N) * std::max(1, p.n_groups), p.K, parts)) return FL_ERR_UNSUPPORTED;
-    // One workgroup per compute unit is the aim.  More 64x128 tiles than compute units: four waves each, two of them fit one.
+    // One workgroup per compute unit is the aim.  More 64x128 tiles than compute units: four waves each, two of them fit one
+    // (96x128 where one row of such tiles takes all rows, see above).
     // Half as many and more: eight waves each (a second K slice).  Fewer: K split over workgroups until they fill the chip,
     // from a length on at which the exchange of the partial tiles pays; below it smaller tiles.  Measured (us):
     //   three parts  512x3072, K = 768: 64x128_K2 21.8, 64x128 23.6, 64x64 24.9; 256x50304, K = 512: 64x128 94, 64x64 106, K2 124;
@@ -677,7 +690,7 @@ int LaunchPacked(const MatmulArgs &args, uint32_t n_batch, bool extra, int parts
     auto tiles = [&](int bm, int bn) { return static_cast<int64_t>((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn) * n_batch; };
     const int64_t t128 = tiles(64, 128), t64 = tiles(64, 64), t32 = tiles(32, 64);
     if (t128 > 256) {
-      tile = FL_TILE_PACKED_64x128;
+      tile = parts == 3 && p.M > 64 && p.M <= 96 && tiles(96, 128) > 256 ? kPacked96x128 : FL_TILE_PACKED_64x128;
     } else if (t128 > 128) {
       tile = FL_TILE_PACKED_64x128_K2;
     } else if (parts == 3 ? p.K >= 1280 && t128 >= 32 : p.K >= 2048 && t32 > 256) {

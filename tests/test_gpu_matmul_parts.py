@@ -294,6 +294,17 @@ def test_packed_tiles_of_the_rule(device, M, K, N):
             assert got.value == (parts if parts == 1 or (M * N >= 280000 and float(M) * K * N >= 5.8e8) else 0)
 
 
+@pytest.mark.parametrize("M", [65, 77, 95, 96, 97])  # tiles of 96 rows, their last rows missing or all there, and one row more
+@pytest.mark.parametrize("K,N", [(712, 32800), (1160, 32769)])  # 257 of 128 columns, the last chunk of K a quarter full
+def test_packed_tiles_of_96_rows(device, M, K, N):
+    with Problem(device, M, K, N) as p:
+        p.pack()
+        out = p.out()
+        print("[case]", M, K, N, flush=True)
+        assert p.chain(out, 0, [(p.cabi.EW_RELU, 0.0)]) == 0
+        close(out, (p.x.double() @ p.w[0].double() + p.b[0].double()).clamp(min=0), "rows")
+
+
 def test_a_plan_frees_the_packed_weights_no_launch_takes(device, tmp_path, monkeypatch):
     """The tile configuration of a contraction is picked after its weights have been packed."""
     import json
