@@ -414,8 +414,11 @@ int64_t TilesPix(const PartsArgs &p, int64_t images, const Cut &c) {
 }
 Cut ChooseCut(const PartsArgs &p, int64_t images, int parts) {
   // A workgroup's time goes with its chunks and TN (the matrix pipe is what it waits for), a launch's with the number
-  // of workgroups a compute unit gets; a split adds the exchange of the partial tiles.  In microseconds.
-  const double chunk_us = parts == 3 ? 0.9 : 0.3, fixed_us = 3.0;
+  // of workgroups a compute unit gets; a split adds the exchange of the partial tiles, which the wave that arrives last takes in,
+  // four tiles at a time.  In microseconds.  (1 x 512 x 14^2 -> 512, three parts, TN = 2: in 16 splits 25.1 us, in 11 21.8, in 8 22.3, in
+  // 4 25.9; at 1 us per eight partial tiles it took 16.  One part keeps its cuts, though some small launches would take up to a sixth
+  // less with others, 1 x 256 x 28^2 -> 512 13.8 us for 16.4: another order of sums is another rounding of the next layer's operands.)
+  const double chunk_us = parts == 3 ? 0.9 : 0.3, fixed_us = 3.0, exchange_us = parts == 3 ? 2.0 : 1.0;
   Cut best;
   best.cost = 1e30;
   for (int tn : {4, 2}) {
@@ -428,7 +431,7 @@ Cut ChooseCut(const PartsArgs &p, int64_t images, int parts) {
       const int64_t per = Ceil(p.chunks, s);
       c.splits = Ceil(p.chunks, per);
       if (c.splits != s) continue;
-      c.cost = Ceil(tiles * s, 256) * (fixed_us + per * tn * chunk_us) + (s > 1 ? 2.0 + Ceil(s * tn, 8) * 1.0 : 0.0);
+      c.cost = Ceil(tiles * s, 256) * (fixed_us + per * tn * chunk_us) + (s > 1 ? 2.0 + Ceil(s * tn, 8) * exchange_us : 0.0);
       if (c.cost < best.cost) best = c;
     }
   }
