@@ -76,11 +76,12 @@ struct PartsArgs {
 // RAGGED: the channels do not come in sixteens; the missing ones read as zero (and are zero in the packed weights).
 // POOLS: the launch may be a pooled one; see Launch.
 // DEPTH: chunks of activations in flight; 2 with one part and up to two workgroups per compute unit (see above).
-// (Three workgroups per compute unit where one part meets 64 filters, 8 x 64 x 224^2 -> 64: 54 us, with two 57; with 128 filters
-// they are slower, 8 x 128 x 112^2 -> 128: 46 against 44.5.)
-template <int PARTS, int WF, int TN, bool RAGGED, bool POOLS, int DEPTH>
-__global__ __launch_bounds__(kThreads, PARTS == 1 && DEPTH == 1 && WF == 2 ? 3 : 2) void ConvPartsKernel(
-    float *out, const float *in, const u32x4 *packed, PartsArgs p) {
+// SPLITS: the launch may have its channels split.  With one part and more than two workgroups per compute unit none has, and the
+// exchange's registers would leave two of those a compute unit for three and spill (bf16, us, with the exchange and without it:
+// 8 x 64 x 224^2 -> 64 57 and 55, pooled 52 and 50, 2 x 96 x 150^2 -> 256 34 and 31, 3 x 64 x 112^2 -> 256 27 and 23, 16 x 64 x 112^2 -> 128
+// 57 and 51; 784 workgroups, of which three on each compute unit leave sixteen over, run 1 to 3 % longer, 8 x 128 x 112^2 -> 128 44.6 and 46).
+template <int PARTS, int WF, int TN, bool RAGGED, bool POOLS, int DEPTH, bool SPLITS>
+__global__ __launch_bounds__(kThreads, 2) void ConvPartsKernel(float *out, const float *in, const u32x4 *packed, PartsArgs p) {
   // (no __restrict__: loads of memory known to be constant move freely, and the compiler sinks the ones that are
   // requested ahead of time down to their first use; these keep their place between the scheduling barriers below)
   constexpr int kRows = 2 * TN * (4 / WF);
@@ -276,7 +277,7 @@ __global__ __launch_bounds__(kThreads, PARTS == 1 && DEPTH == 1 && WF == 2 ? 3 :
   // ---- channels split over workgroups: combine the partial tiles ----------------------------------------------
   // The hand-off of conv_halo.hip: device-coherent stores, the explicit wait, one arrival per wave, loads behind the
   // branch on the returned count.  Sums in split order, so the result does not depend on who arrives last.
-  if (p.n_splits > 1) {
+  if (SPLITS && p.n_splits > 1) {
     const uint32_t n_splits = p.n_splits, slot = tile_id * 4 + wave;
     float *all = p.partials + static_cast<size_t>(slot) * n_splits * (TN * 1024);
     float *mine = all + split * (TN * 1024);
@@ -444,22 +445,28 @@ Cut ChooseCut(const PartsArgs &p, int64_t images, int parts) {
 // before starts with its instructions missing (VGG-16 of one image with two kernels throughout 438 us, with one 436; bf16 401, 398).
 template <int PARTS, int WF, int TN>
 void Launch(const PartsArgs &p, uint32_t grid, float *out, const float *in, const u32x4 *packed, hipStream_t s) {
-#define FL_PARTS_AS(RAGGED_, POOLS_, DEPTH_) \
-  FL_LAUNCH((ConvPartsKernel<PARTS, WF, TN, RAGGED_, POOLS_, DEPTH_>), dim3(grid), dim3(kThreads), 0, s, out, in, packed, p)
+#define FL_PARTS_AS(RAGGED_, POOLS_, DEPTH_, SPLITS_) \
+  FL_LAUNCH((ConvPartsKernel<PARTS, WF, TN, RAGGED_, POOLS_, DEPTH_, SPLITS_>), dim3(grid), dim3(kThreads), 0, s, out, in, packed, p)
   if constexpr (PARTS == 1) {
-    if (grid <= 2 * 256) {
-      if (p.C % kChunk != 0) FL_PARTS_AS(true, true, 2);
-      else FL_PARTS_AS(false, true, 2);
+    // (every launch that is split: its partial tiles fit the workspace)
+    constexpr uint32_t kTwoPerUnit = 2 * 256;
+    static_assert(kWorkspaceTiles <= kTwoPerUnit * 4 * TN, "a launch of more workgroups has no splits");
+    if (grid <= kTwoPerUnit) {
+      if (p.C % kChunk != 0) FL_PARTS_AS(true, true, 2, true);
+      else FL_PARTS_AS(false, true, 2, true);
       return;
     }
-    if (!p.pooled) {
-      if (p.C % kChunk != 0) FL_PARTS_AS(true, false, 1);
-      else FL_PARTS_AS(false, false, 1);
-      return;
+    if (p.C % kChunk != 0) {
+      if (p.pooled) FL_PARTS_AS(true, true, 1, false);
+      else FL_PARTS_AS(true, false, 1, false);
+    } else {
+      if (p.pooled) FL_PARTS_AS(false, true, 1, false);
+      else FL_PARTS_AS(false, false, 1, false);
     }
+  } else {
+    if (p.C % kChunk != 0) FL_PARTS_AS(true, true, 1, true);
+    else FL_PARTS_AS(false, true, 1, true);
   }
-  if (p.C % kChunk != 0) FL_PARTS_AS(true, true, 1);
-  else FL_PARTS_AS(false, true, 1);
 #undef FL_PARTS_AS
 }
 

@@ -91,6 +91,37 @@ def test_packed_conv_bf16_chunks(device, N, C, H, W, F, tile):
     np.testing.assert_array_equal(got, _oracle(x, w, bias, [1, 1, 1, 1]))
 
 
+def _recorded(device, N, C, H, W, F, parts, tile=0, splits=0, pool=False):
+    """What a convolution launches: (kernel's name, workgroups a compute unit holds, grid, bytes of scratch)."""
+    import torch
+
+    from fluidml_amd import cabi
+    from util import launched
+
+    shape = (N, F, H // 2, W // 2) if pool else (N, F, H, W)
+    x, w, b, out = (torch.zeros(*s, device=device) for s in ((N, C, H, W), (F, C, 3, 3), (F,), shape))
+    ref = lambda t: ctypes.byref(cabi.make_tensor(t.data_ptr(), cabi.FL_FLOAT32, t.shape, t.stride()))
+    size = ctypes.c_size_t()
+    cabi.call("conv3x3_packed_bytes", ref(w), parts, ctypes.byref(size))
+    packed = torch.zeros(size.value, dtype=torch.uint8, device=device)
+    name = "conv3x3_packed_chain_pool" if pool else "conv3x3_packed_chain"
+    call = lambda s: cabi.call(name, ref(x), ref(w), packed.data_ptr(), parts, ref(b), ref(out), cabi.i64_array([1] * 4),
+                               ctypes.byref(cabi.make_chain([])), tile << 4 | splits << 8, s)
+    call(None)
+    found, = launched(call)
+    assert "ConvPartsKernel" in found[0]
+    return found
+
+
+@pytest.mark.parametrize("C", [64, 40])
+@pytest.mark.parametrize("F,tile", [(128, 1), (128, 2), (64, 1), (64, 2)])
+@pytest.mark.parametrize("pool", [False, True])
+def test_packed_conv_bf16_of_many_workgroups_fits(device, C, F, tile, pool):
+    """No launch of more than two workgroups per compute unit has splits, and none holds registers for their exchange."""
+    name, fit, grid, scratch = _recorded(device, 8, C, 160, 112, F, 1, tile, 1, pool)
+    assert grid[0] > 512 and fit >= 3 and scratch == 0, (name, fit, grid, scratch)
+
+
 def test_packed_conv_layouts(device):
     x, w, bias = _operands(8, 2, 24, 11, 18, 40)
     want = _oracle(x, w, bias, [1, 1, 1, 1])

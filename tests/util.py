@@ -136,10 +136,21 @@ class _KernelNode(ctypes.Structure):  # hipKernelNodeParams
                 ("params", ctypes.c_void_p), ("shared", ctypes.c_uint32)]
 
 
+class _FuncAttributes(ctypes.Structure):  # hipFuncAttributes
+    _fields_ = [("version", ctypes.c_int), ("cache", ctypes.c_int), ("constants", ctypes.c_size_t), ("scratch", ctypes.c_size_t),
+                ("most_shared", ctypes.c_int), ("most_threads", ctypes.c_int), ("registers", ctypes.c_int), ("carveout", ctypes.c_int),
+                ("ptx", ctypes.c_int), ("shared", ctypes.c_size_t)]
+
+
 def launches(call):
     """The kernels that `call(stream)` launches, in the order of its graph: (mangled name, workgroups a compute unit holds).
 
     The call is recorded, not run; it must have run once before (a first call may allocate)."""
+    return [(name, fit) for name, fit, _, _ in launched(call)]
+
+
+def launched(call):
+    """The same with the grid and the bytes of scratch memory per lane: (name, workgroups a compute unit holds, grid, scratch)."""
     import torch
 
     from fluidml_amd import cabi
@@ -163,6 +174,8 @@ def launches(call):
         name = hip.hipKernelNameRefByPtr(ctypes.c_void_p(p.func), stream)
         assert hip.hipOccupancyMaxActiveBlocksPerMultiprocessor(ctypes.byref(fit), ctypes.c_void_p(p.func), threads,
                                                                 ctypes.c_size_t(p.shared)) == 0
-        found.append((name.decode(), fit.value))
+        attributes = _FuncAttributes()
+        assert hip.hipFuncGetAttributes(ctypes.byref(attributes), ctypes.c_void_p(p.func)) == 0
+        found.append((name.decode(), fit.value, tuple(p.grid), attributes.scratch))
     assert hip.hipGraphDestroy(graph) == 0
     return found
