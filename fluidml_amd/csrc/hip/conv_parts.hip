@@ -19,10 +19,10 @@
 //   * the loads that run ahead are held in their place by scheduling barriers (the compiler moves them down to their use), those of
 //     the patch one by one between the products: sixteen in a row hold up the wave at the address unit, and its products behind
 //     them (one part, 8 x 512 x 28^2 -> 512: 51.5 -> 43.7 us, of 30 that the products alone take; three parts 160 -> 156);
-//   * one part, where a chunk's products take 0.5 us and one or two workgroups share a compute unit: two chunks of activations and
-//     17 taps of weights in flight, the conversion of the next chunk between the products (8 x 512 x 14^2 -> 512: 27 -> 22 us
-//     before the loads were spread).  With more workgroups per compute unit those fill the waits, and the registers and
-//     the longer start cost more (8 x 64 x 224^2 -> 64: 54 us with one chunk ahead, 60 with two);
+//   * one part, where a chunk's products take 0.5 us and one or two workgroups of a few chunks share a compute unit: two chunks
+//     of activations and 17 taps of weights in flight, the conversion of the next chunk between the products (8 x 512 x 14^2 ->
+//     512: 27 -> 22 us before the loads were spread).  With more workgroups per compute unit those fill the waits, and the
+//     registers and the longer start cost more (8 x 64 x 224^2 -> 64: 54 us with one chunk ahead, 60 with two);
 //   * few tiles: the channels of a tile go to several workgroups, whose partial tiles meet in the stream's workspace and
 //     are added in split order by the wave that arrives last.
 // Measured against conv_halo.hip, bias and ReLU included (us; TFLOP/s of the convolution's own operations):
@@ -75,7 +75,7 @@ struct PartsArgs {
 // WF waves along the filters (32 each), 4 / WF along the rows; a wave owns TN tiles of 2 rows x 16 columns.
 // RAGGED: the channels do not come in sixteens; the missing ones read as zero (and are zero in the packed weights).
 // POOLS: the launch may be a pooled one; see Launch.
-// DEPTH: chunks of activations in flight; 2 with one part and up to two workgroups per compute unit (see above).
+// DEPTH: chunks of activations in flight; 2 with one part, up to two workgroups per compute unit (see above) and a few chunks each (see Launch).
 // SPLITS: the launch may have its channels split.  With one part and more than two workgroups per compute unit none has, and the
 // exchange's registers would leave two of those a compute unit for three and spill (bf16, us, with the exchange and without it:
 // 8 x 64 x 224^2 -> 64 57 and 55, pooled 52 and 50, 2 x 96 x 150^2 -> 256 34 and 31, 3 x 64 x 112^2 -> 256 27 and 23, 16 x 64 x 112^2 -> 128
@@ -452,8 +452,19 @@ void Launch(const PartsArgs &p, uint32_t grid, float *out, const float *in, cons
     constexpr uint32_t kTwoPerUnit = 2 * 256;
     static_assert(kWorkspaceTiles <= kTwoPerUnit * 4 * TN, "a launch of more workgroups has no splits");
     if (grid <= kTwoPerUnit) {
-      if (p.C % kChunk != 0) FL_PARTS_AS(true, true, 2, true);
-      else FL_PARTS_AS(false, true, 2, true);
+      // Two chunks in flight from five chunks per workgroup on, from four where the channels are split and the weights take longer
+      // to come: with fewer, the requests ahead are mostly for chunks that a workgroup does not have (bf16, us, one chunk ahead and two:
+      // 1 chunk 3 x 16 x 79^2 -> 160 11.2, 13.1; 2 4 x 32 x 56^2 -> 128 7.6, 8.0; 4 8.7, 8.9; 5 9.4, 9.4; 6 10.1, 9.9; 8 11.4, 11.0; 16
+      // 17.0, 15.5.  Split: 2 1 x 128 x 28^2 -> 512 13.9, 15.0; 3 3 x 192 x 14^2 -> 512 13.5, 14.3; 4 2 x 512 x 14^2 -> 512 19.3, 18.4, 1 x
+      // 512 x 28^2 -> 256 19.0, 18.0, but 1 x 256 x 56^2 -> 128 12.0, 12.4; 6 1 x 384 x 28^2 -> 512 17.9, 16.6).
+      const bool two = p.chunks_per_split >= (p.n_splits > 1 ? 4 : 5);
+      if (p.C % kChunk != 0) {
+        if (two) FL_PARTS_AS(true, true, 2, true);
+        else FL_PARTS_AS(true, true, 1, true);
+      } else {
+        if (two) FL_PARTS_AS(false, true, 2, true);
+        else FL_PARTS_AS(false, true, 1, true);
+      }
       return;
     }
     if (p.C % kChunk != 0) {

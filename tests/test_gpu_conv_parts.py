@@ -107,8 +107,7 @@ def _recorded(device, N, C, H, W, F, parts, tile=0, splits=0, pool=False):
     name = "conv3x3_packed_chain_pool" if pool else "conv3x3_packed_chain"
     call = lambda s: cabi.call(name, ref(x), ref(w), packed.data_ptr(), parts, ref(b), ref(out), cabi.i64_array([1] * 4),
                                ctypes.byref(cabi.make_chain([])), tile << 4 | splits << 8, s)
-    call(None)
-    found, = launched(call)
+    found, = launched(call, first_on_its_stream=True)
     assert "ConvPartsKernel" in found[0]
     return found
 
@@ -120,6 +119,27 @@ def test_packed_conv_bf16_of_many_workgroups_fits(device, C, F, tile, pool):
     """No launch of more than two workgroups per compute unit has splits, and none holds registers for their exchange."""
     name, fit, grid, scratch = _recorded(device, 8, C, 160, 112, F, 1, tile, 1, pool)
     assert grid[0] > 512 and fit >= 3 and scratch == 0, (name, fit, grid, scratch)
+
+
+@pytest.mark.parametrize("C", [16, 64, 65, 80, 256, 320])
+@pytest.mark.parametrize("F,tile,splits", [(128, 1, 1), (64, 2, 1), (96, 1, 4), (48, 2, 4), (96, 2, 8)])
+@pytest.mark.parametrize("pool", [False, True])
+def test_packed_conv_bf16_chunks_ahead(device, C, F, tile, splits, pool):
+    """Two chunks of activations are in flight where a workgroup has five and more, four of split channels; the sums are the same either way.  Exact:
+    operands of a few bits, so that every product and every sum of them is a float32."""
+    print("[case]", C, F, tile, splits, pool, flush=True)
+    chunks = -(-C // 16)
+    per = -(-chunks // splits)
+    name, _, grid, _ = _recorded(device, 2, C, 20, 35, F, 1, tile, splits, pool)
+    assert f"ELi{2 if per >= (4 if per < chunks else 5) else 1}ELb1EE" in name, (name, grid, per)
+    if pool:
+        return
+    rng = np.random.default_rng(C + F)
+    x = rng.integers(-8, 9, (2, C, 20, 35)).astype(np.float32)
+    w = rng.integers(-4, 5, (F, C, 3, 3)).astype(np.float32)
+    bias = rng.integers(-16, 17, F).astype(np.float32)
+    got = _run(device, x, w, bias, [1, 1, 1, 1], 1, tile, splits, times=2)
+    np.testing.assert_array_equal(got, _oracle(x, w, bias, [1, 1, 1, 1]))
 
 
 def test_packed_conv_layouts(device):

@@ -149,15 +149,21 @@ def launches(call):
     return [(name, fit) for name, fit, _, _ in launched(call)]
 
 
-def launched(call):
-    """The same with the grid and the bytes of scratch memory per lane: (name, workgroups a compute unit holds, grid, scratch)."""
+def launched(call, first_on_its_stream=False):
+    """The same with the grid and the bytes of scratch memory per lane: (name, workgroups a compute unit holds, grid, scratch).
+    `first_on_its_stream`: run it there once, so that the stream has the workspace that a split launch needs."""
     import torch
 
     from fluidml_amd import cabi
 
     hip = cabi.lib  # (its runtime's entry points are found through it)
     hip.hipKernelNameRefByPtr.restype = ctypes.c_char_p
-    stream, graph, count = ctypes.c_void_p(torch.cuda.Stream().cuda_stream), ctypes.c_void_p(), ctypes.c_size_t()
+    own = torch.cuda.Stream()
+    stream, graph, count = ctypes.c_void_p(own.cuda_stream), ctypes.c_void_p(), ctypes.c_size_t()
+    if first_on_its_stream:
+        torch.cuda.synchronize()
+        call(stream)
+        own.synchronize()
     assert hip.hipStreamBeginCapture(stream, 2) == 0
     try:
         call(stream)
