@@ -416,10 +416,19 @@ int64_t TilesPix(const PartsArgs &p, int64_t images, const Cut &c) {
 Cut ChooseCut(const PartsArgs &p, int64_t images, int parts) {
   // A workgroup's time goes with its chunks and TN (the matrix pipe is what it waits for), a launch's with the number
   // of workgroups a compute unit gets; a split adds the exchange of the partial tiles, which the wave that arrives last takes in,
-  // four tiles at a time.  In microseconds.  (1 x 512 x 14^2 -> 512, three parts, TN = 2: in 16 splits 25.1 us, in 11 21.8, in 8 22.3, in
-  // 4 25.9; at 1 us per eight partial tiles it took 16.  One part keeps its cuts, though some small launches would take up to a sixth
-  // less with others, 1 x 256 x 28^2 -> 512 13.8 us for 16.4: another order of sums is another rounding of the next layer's operands.)
-  const double chunk_us = parts == 3 ? 0.9 : 0.3, fixed_us = 3.0, exchange_us = parts == 3 ? 2.0 : 1.0;
+  // eight tiles of 2 x 16 pixels at a time.  In microseconds.
+  const double chunk_us = parts == 3 ? 0.9 : 0.3, fixed_us = 3.0;
+  // Eight partial tiles cost 1 us where few workgroups exchange theirs, and with three parts 2 us from about 64 workgroups on (us,
+  // TN = 2: 1 x 512 x 14^2 -> 512 in 16 splits, 256 workgroups, 24.7, in 11 21.4, in 8 21.2, in 4 25.9; 1 x 128 x 28^2 -> 256 in 8 18.6, in 4
+  // 15.0; but 1 x 512 x 16^2 -> 64 in 16 splits, 32 workgroups, 17.9, in 8 19.4; 1 x 192 x 16^2 -> 64 in 12 14.2, in 4 15.7).  Ten are
+  // taken for eight (8 x 384 x 10^2 -> 256 in five 24.0, in four 25.2).  The first eight cost 1 us with up to 64 filters, where a chunk's
+  // patch has twice the rows and not splitting is dearer (1 x 48 x 56^2 -> 64 in three 12.3, in one 13.2; 4 x 48 x 14^2 -> 512 13.4, 11.9).
+  // One part keeps 1 us throughout (1 x 256 x 28^2 -> 512 would take a sixth less with other cuts).
+  auto exchange_us = [&](const Cut &c, int64_t workgroups) {
+    const int64_t partials = c.splits * c.tn, rounds = partials <= 10 ? 1 : Ceil(partials, 8);
+    if (parts == 1 || workgroups <= 64) return 2.0 + Ceil(partials, 8);
+    return 2.0 + (rounds == 1 && c.wf == 2 ? 1.0 : 2.0 * rounds);
+  };
   Cut best;
   best.cost = 1e30;
   for (int tn : {4, 2}) {
@@ -432,7 +441,7 @@ Cut ChooseCut(const PartsArgs &p, int64_t images, int parts) {
       const int64_t per = Ceil(p.chunks, s);
       c.splits = Ceil(p.chunks, per);
       if (c.splits != s) continue;
-      c.cost = Ceil(tiles * s, 256) * (fixed_us + per * tn * chunk_us) + (s > 1 ? 2.0 + Ceil(s * tn, 8) * exchange_us : 0.0);
+      c.cost = Ceil(tiles * s, 256) * (fixed_us + per * tn * chunk_us) + (s > 1 ? exchange_us(c, tiles * s) : 0.0);
       if (c.cost < best.cost) best = c;
     }
   }

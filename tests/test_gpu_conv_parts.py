@@ -142,6 +142,20 @@ def test_packed_conv_bf16_chunks_ahead(device, C, F, tile, splits, pool):
     np.testing.assert_array_equal(got, _oracle(x, w, bias, [1, 1, 1, 1]))
 
 
+@pytest.mark.parametrize("N,C,hw,F,workgroups", [
+    # three parts, two tiles per wave; the partial tiles of few workgroups are cheap to bring together
+    (1, 512, 16, 64, 2 * 16), (3, 512, 7, 64, 3 * 16), (1, 192, 16, 64, 2 * 12), (3, 192, 7, 64, 3 * 12), (1, 48, 11, 96, 3 * 3), (2, 48, 20, 64, 12 * 3),
+    # those of many are not, all 64 filters of a small launch in one workgroup apart
+    (1, 512, 14, 512, 16 * 8), (1, 128, 28, 256, 28 * 4), (1, 192, 14, 512, 16 * 4), (4, 48, 14, 512, 64), (1, 48, 56, 64, 28 * 3), (1, 96, 56, 64, 28 * 3),
+    (8, 384, 10, 256, 48 * 5), (3, 512, 14, 512, 48 * 5),
+])
+def test_packed_conv_splits_of_the_rule(device, N, C, hw, F, workgroups):
+    _, _, grid, _ = _recorded(device, N, C, hw, hw, F, 3)
+    assert grid[0] == workgroups
+    x, w, bias = _operands(7, N, C, hw, hw, F)
+    assert_close(_run(device, x, w, bias, [1, 1, 1, 1], 3, times=2), _oracle(x, w, bias, [1, 1, 1, 1]), what="three parts")
+
+
 def test_packed_conv_layouts(device):
     x, w, bias = _operands(8, 2, 24, 11, 18, 40)
     want = _oracle(x, w, bias, [1, 1, 1, 1])
