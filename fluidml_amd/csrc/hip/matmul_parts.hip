@@ -167,23 +167,25 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
     p.div_inner.DivMod(static_cast<uint32_t>(n < p.N ? n : 0), hi, lo);
     col = static_cast<int64_t>(hi) * sCn_outer + static_cast<int64_t>(lo) * sCn;
   }
-  // the addends: with a few values per lane here, else behind the K loop, where the registers of the tiles are free; either way the
-  // exchange of the slices and splits lies between them and their use (asked for behind it, 512 x 768 x 3072 with an addend and
-  // row statistics took 29.3 us, now 28.1)
-  constexpr bool EARLY_ADD = EXTRA != 0 && kShare <= 8;
-  float pre_add[EXTRA != 0 ? kShare : 1], pre_add2[EXTRA != 0 ? kShare : 1];
+  // The addends: with a few values per lane here, else behind the K loop, where the registers of the tiles are free; all of a lane's
+  // together, and with K slices or splits before their exchange (us, asked for sixteen by sixteen where they are used and so: 512 x 768 x
+  // 3072 with row statistics 29.3, 28.1; without an exchange 300 x 33000 x 512 86.3, 80.2, one part 1024 x 3072 x 1024 21.7, 19.7).  The
+  // second one is rare: with more than sixteen values per lane it is asked for where it is used.  Held beside the first it costs
+  // 64x128 tiles of one part a wave per SIMD (128 x 50304 x 512 27.3, now 25.5) and those of 96 rows scalar registers (53.0, 48.0).
+  constexpr bool EARLY_ADD = EXTRA != 0 && kShare <= 8, BOTH_ADD = EXTRA != 0 && kShare <= 16;
+  float pre_add[EXTRA != 0 ? kShare : 1], pre_add2[BOTH_ADD ? kShare : 1];
+  auto load_addend = [&](const float *from, float *to, int v) {
+    const int m = m0 + share_row(v);
+    *to = m < p.M && n < p.N ? from[static_cast<int64_t>(m) * sCm + col] : 0.0f;
+  };
   auto load_addends = [&] {
     if (p.addend == nullptr) return;
 #pragma unroll
-    for (int v = 0; v < kShare; ++v) {
-      const int m = m0 + share_row(v);
-      pre_add[v] = m < p.M && n < p.N ? p.addend[static_cast<int64_t>(m) * sCm + col] : 0.0f;
-    }
-    if (p.addend2 == nullptr) return;
+    for (int v = 0; v < kShare; ++v) load_addend(p.addend, pre_add + v, v);
+    if constexpr (BOTH_ADD) {
+      if (p.addend2 == nullptr) return;
 #pragma unroll
-    for (int v = 0; v < kShare; ++v) {
-      const int m = m0 + share_row(v);
-      pre_add2[v] = m < p.M && n < p.N ? p.addend2[static_cast<int64_t>(m) * sCm + col] : 0.0f;
+      for (int v = 0; v < kShare; ++v) load_addend(p.addend2, pre_add2 + v, v);
     }
   };
   if constexpr (EARLY_ADD) load_addends();
@@ -426,12 +428,9 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
     if (p.chain_n != 0) RunChainBlock<EV>(p.chain, out);
     if constexpr (EXTRA != 0) {
       if (p.addend != nullptr) {
-        float add[EV], add2[EV];
+        float add[EV];
 #pragma unroll
-        for (int e = 0; e < EV; ++e) {
-          add[e] = pre_add[v0 + e];
-          add2[e] = pre_add2[v0 + e];
-        }
+        for (int e = 0; e < EV; ++e) add[e] = pre_add[v0 + e];
         if (p.ln_mode == 2) {
           // the addend is the un-normalised tensor of a LayerNormalization: normalise it on the way in
 #pragma unroll
@@ -443,6 +442,12 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
 #pragma unroll
         for (int e = 0; e < EV; ++e) out[e] = p.addend_is_factor != 0 ? out[e] * add[e] : out[e] + add[e];
         if (p.addend2 != nullptr) {
+          float add2[EV];
+#pragma unroll
+          for (int e = 0; e < EV; ++e) {
+            if constexpr (BOTH_ADD) add2[e] = pre_add2[v0 + e];
+            else load_addend(p.addend2, add2 + e, v0 + e);
+          }
 #pragma unroll
           for (int e = 0; e < EV; ++e) out[e] += add2[e];
         }

@@ -193,6 +193,22 @@ def test_packed_epilogues(device, tile, splits):
             close(got, ref, f"result {i}")
 
 
+def test_packed_addend_keeps_four_to_a_unit(device):
+    """bf16 launches of 64x128 tiles with an addend hold no registers for the second one that none of them has."""
+    from util import launched
+
+    with Problem(device, 128, 256, 33000) as p:
+        e = p.rand(128, 33000)
+        p.pack(1)
+        out = p.out()
+        none = ctypes.byref(p.cabi.make_chain([]))
+        call = lambda s: p.cabi.call("matmul_chain_add", p.ref(p.x), p.ref(p.w[0]), p.ref(p.b[0]), p.ref(out), none, p.ref(e), None,
+                                     p.cabi.FL_CONTRACT_BF16, s)
+        (name, fit, _, scratch), = launched(call, first_on_its_stream=True)
+        assert "MatmulPartsKernelILi1ELi2ELi4ELi1E" in name and fit >= 4 and scratch == 0, (name, fit, scratch)
+        close(out, p.x.bfloat16().double() @ p.w[0].bfloat16().double() + p.b[0].double() + e.double(), "addend")
+
+
 def test_packed_gemm(device):
     with Problem(device, 48, 200, 72, trans_b=True) as p:
         def call(flags):
