@@ -321,6 +321,101 @@ def test_packed_tiles_of_96_rows(device, M, K, N):
         close(out, (p.x.double() @ p.w[0].double() + p.b[0].double()).clamp(min=0), "rows")
 
 
+def _ran_on_96_rows(call, extra):
+    from util import launched
+
+    (name, fit, _, scratch), = launched(call, first_on_its_stream=True)
+    assert "MatmulPartsKernelILi3ELi3ELi4ELi1E" in name and f"ELi{extra}EEE" in name and fit >= 2 and scratch == 0, (name, fit, scratch)
+
+
+@pytest.mark.parametrize("M", [65, 77, 96])
+def test_packed_epilogues_of_96_rows(device, M):
+    """Each epilogue that a launch of the rule's tile of 96 rows can have, before packing (any tile) and after."""
+    K = 296  # the last chunk a quarter full
+
+    def norm(cabi, stats=None, out=None):
+        n = cabi.FlNormFusion()
+        n.deferred, n.width, n.epsilon = (cabi.FL_NORM_LHS, K, 1e-5) if stats is not None else (cabi.FL_NORM_NONE, 0, 0.0)
+        n.stats = stats.data_ptr() if stats is not None else None
+        n.stats_out = out.data_ptr() if out is not None else None
+        return n
+
+    def row_stats(torch, t):
+        runs = t.split(32, -1)
+        return torch.stack([torch.stack([r.mean(-1), ((r - r.mean(-1, keepdim=True)) ** 2).sum(-1)], -1) for r in runs], 1).contiguous()
+
+    # 257 tiles of one contraction; 86 of each of three members
+    for N, count in ((32800, 1), (11008, 3)):
+        print("[case]", M, K, N, count, flush=True)
+        with Problem(device, M, K, N, count=count) as p:
+            cabi, torch = p.cabi, p.torch
+            none = ctypes.byref(cabi.make_chain([]))
+            relu = ctypes.byref(cabi.make_chain([(cabi.EW_RELU, 0.0)]))
+            stats, c1 = row_stats(torch, p.x), [w.sum(0) for w in p.w]
+            e1, e2 = p.rand(M, N), p.rand(M, N)
+
+            def cases():
+                if count == 1:
+                    out = p.out()
+                    yield 1, [out], lambda s: cabi.call("matmul_chain_add", p.ref(p.x), p.ref(p.w[0]), p.ref(p.b[0]), p.ref(out), relu, p.ref(e1), None, 0, s)
+                    out2 = p.out()
+                    yield 1, [out2], lambda s: cabi.call("matmul_chain_add", p.ref(p.x), p.ref(p.w[0]), p.ref(p.b[0]), p.ref(out2), none, p.ref(e1), p.ref(e2), 0, s)
+                    out3, stats_n = p.out(), torch.full((M, 1025, 2), 9.0, device=device)
+                    n3 = norm(cabi, out=stats_n)
+                    yield 1, [out3, stats_n], lambda s: cabi.call("matmul_chain_group_norm", 1, p.ref(p.x), p.list(p.w), p.list(p.b), None, p.list([out3]), 0, None,
+                                                                  none, p.ref(e1), ctypes.byref(n3), 0, s)
+                    out4 = torch.full((N, M + 1), 9.0, device=device)
+                    yield 0, [out4], lambda s: cabi.call("matmul_chain", p.ref(p.x), p.ref(p.w[0]), p.ref(p.b[0]), p.ref(out4, (M, N), (1, M + 1)), none, 0, s)
+                outs = [p.out() for _ in range(count)]
+                n5 = norm(cabi, stats=stats)
+                yield 1, outs, lambda s: cabi.call("matmul_chain_group_norm", count, p.ref(p.x), p.list(p.w), p.list(p.b), p.list(c1), p.list(outs), 0, None,
+                                                   none, None, ctypes.byref(n5), 0, s)
+                if count > 1:  # columns as heads of 32 that a transpose moved apart
+                    heads = [torch.full((N // 32, M, 32), 9.0, device=device) for _ in range(count)]
+                    views = [p.tensor(o, (M, N), (32, 1)) for o in heads]
+                    outer = cabi.i64_array([32 * M] * count)
+                    yield 0, heads, lambda s: cabi.call("matmul_chain_group", count, p.ref(p.x), p.list(p.w), p.list(p.b), p.list(views), 32, outer, none, 0, s)
+
+            want = []
+            for _, outs, call in cases():
+                call(None)
+                want.append([o.clone() for o in outs])
+            p.pack()
+            for i, (extra, outs, call) in enumerate(cases()):
+                _ran_on_96_rows(call, extra)
+                for got, ref in zip(outs, want[i]):
+                    close(got, ref, f"case {i}")
+
+
+@pytest.mark.parametrize("M", [65, 96])
+def test_packed_96_rows_outside_the_parts(device, M):
+    K, N = 296, 32800
+    with Problem(device, M, K, N) as p:
+        p.x[3, 7], p.x[M - 1, K - 1], p.w[0][11, N - 1] = float("inf"), float("nan"), float("-inf")
+        want = p.x.double() @ p.w[0].double() + p.b[0].double()
+        p.pack()
+        out = p.out()
+        _ran_on_96_rows(lambda s: p.cabi.call("matmul_chain", p.ref(p.x), p.ref(p.w[0]), p.ref(p.b[0]), p.ref(out), ctypes.byref(p.cabi.make_chain([])), 0, s), 0)
+        assert p.torch.equal(out.isnan(), want.isnan()) and p.torch.equal(out.isinf(), want.isinf())
+        fine = want.isfinite()
+        close(out[fine], want[fine], "finite results beside infinities")
+    for x_scale, w_scale in ((1e-41, 1e-3), (1e-21, 2e-18)):  # products that vanish (weights from 2^-60 on)
+        with Problem(device, M, K, N) as p:
+            p.x.copy_((p.x.abs() + 0.5).double() * x_scale)
+            p.w[0].copy_((p.w[0].abs() + 0.5) * w_scale)
+            p.x[3] = 0
+            p.x[5, :7] = 0
+            p.x[7, 1:] = 0
+            p.b[0].zero_()
+            want = p.x.double() @ p.w[0].double()
+            p.pack()
+            out = p.out()
+            _ran_on_96_rows(lambda s: p.cabi.call("matmul_chain", p.ref(p.x), p.ref(p.w[0]), p.ref(p.b[0]), p.ref(out), ctypes.byref(p.cabi.make_chain([])), 0, s), 0)
+            err = (out.double() - want).abs()
+            assert (err <= K * 2.0 ** -150 + 1e-6 * want.abs()).all(), err.max().item()
+            assert (out[3] == 0).all() and (out[7] != 0).any()
+
+
 def test_a_plan_frees_the_packed_weights_no_launch_takes(device, tmp_path, monkeypatch):
     """The tile configuration of a contraction is picked after its weights have been packed."""
     import json
