@@ -10,8 +10,8 @@
 //   * The rows of A are split into their parts once per workgroup, on their way from registers into LDS, where they lie
 //     as [part][k / 8][row][8]: a lane's A operand is one 128-bit read, 32 consecutive places per half wave.  The places
 //     of one k / 8 are padded, so that the writes (consecutive lanes: consecutive k of a row) spread over the banks.
-//   * The loads of a chunk leave between the products of an earlier one, a few per product (three parts): in a row behind the
-//     barrier, sixteen cycles of the address unit each, they held up all waves and the products behind them (512 x 3072 x 768
+//   * The loads of a chunk leave between the products of the chunk DEPTH before it, a few per product (three parts): in a row behind
+//     the barrier, sixteen cycles of the address unit each, they held up all waves and the products behind them (512 x 3072 x 768
 //     22.4 -> 19.9 us, 256 x 3072 x 768 16.6 -> 14.6, 512 x 768 x 3072 25.0 -> 23.0, 256 x 50304 x 512 100 -> 93).
 //   * WN waves side by side times KS = 4 / WN slices of K; two steps of 16 k per wave and chunk, one barrier per chunk, LDS
 //     double buffered, DEPTH chunks of both operands in flight in registers: a launch of a small transformer has a few
@@ -248,6 +248,14 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
   // a compute unit nobody else fills the matrix pipe while a wave converts, so the conversion of the next chunk runs
   // between the products of this one: a product keeps the pipe busy for 32 cycles, in which eight other instructions issue.
   constexpr int kGroups = kSteps * TM;
+  // With one chunk ahead its rows are asked for and converted between the products of the same chunk: the loads leave with the first
+  // groups of products, the rows' before the weights', and the last groups convert.  (In the order of the deeper tiles the first
+  // conversion waited for loads that it was one product behind, in every chunk: us, 96 x 50304 x 512 47, now 44, 70 x 33000 x 2048 131
+  // and 119, 90 x 40000 x 1024 with an addend 73 and 67.)
+  constexpr int kLoadGroups = DEPTH == 1 ? kGroups - kPer : kGroups;
+  constexpr auto load_group = [](int i) { return i * kLoadGroups / kLoads; };
+  constexpr auto store_group = [](int t) { return DEPTH == 1 ? kLoadGroups + t : t * kGroups / kPer; };
+  static_assert(DEPTH > 1 || store_group(0) >= load_group(2 * kPer - 1) + 2, "products between a chunk's rows and their conversion");
   auto chunk = [&](int c, auto idx_c) __attribute__((always_inline)) {
     constexpr int I = decltype(idx_c)::value;
     if constexpr (PARTS == 1) {
@@ -266,7 +274,7 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
       if constexpr (g + 1 < kGroups) load_a(g + 1);
       if constexpr (PARTS == 3) {
         StaticFor<kLoads>([&](auto i) {
-          if constexpr (i * kGroups / kLoads == g) load(c + DEPTH, std::integral_constant<int, (I + DEPTH) % kSets>{}, i);
+          if constexpr (load_group(i) == g) load(c + DEPTH, std::integral_constant<int, (I + DEPTH) % kSets>{}, i);
         });
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -274,7 +282,7 @@ __global__ __launch_bounds__(64 * WN *KS, 2) void MatmulPartsKernel(float *C_, c
       // (also behind the last chunk, which is then converted again: a condition would end the block that is scheduled)
 #pragma unroll
       for (int t = 0; t < kPer; ++t) {
-        if (t * kGroups / kPer == g) store_item(c + 1, (I + 1) % 2, std::integral_constant<int, (I + 1) % kSets>{}, t);
+        if (store_group(t) == g) store_item(c + 1, (I + 1) % 2, std::integral_constant<int, (I + 1) % kSets>{}, t);
       }
 #pragma unroll
       for (int k = 0; k < (PARTS == 3 ? 6 : 1); ++k) {
