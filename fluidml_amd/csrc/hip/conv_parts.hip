@@ -27,17 +27,18 @@
 //     are added in split order by the wave that arrives last.
 // Measured against conv_halo.hip, bias and ReLU included (us; TFLOP/s of the convolution's own operations):
 //   images x channels x size -> filters        fp32 before -> now            bf16 before -> now
-//   8 x  64 x 224^2 ->  64                     289 -> 161 (184)               95 -> 62 (480)
-//   8 x 128 x 112^2 -> 128                     286 -> 154 (192)               87 -> 50 (595)
+//   8 x  64 x 224^2 ->  64                     289 -> 161 (184)               95 -> 59 (502)
+//   8 x 128 x 112^2 -> 128                     286 -> 154 (192)               87 -> 49 (603)
 //   8 x 256 x  56^2 -> 256                     290 -> 150 (197)              105 -> 43 (688)
 //   8 x 512 x  28^2 -> 512                     324 -> 156 (190)              108 -> 43 (688)
 //   8 x 512 x  14^2 -> 512                      92 ->  50 (147)               35 -> 21 (352)
 //   1 x 256 x  56^2 -> 256                      52 ->  30 (123)               23 -> 15 (247)
 //   4 x 256 x  37^2 -> 256                     156 ->  46 (142)              106 -> 17 (384)
 // A 2 x 2 pool behind the chain is taken in the epilogue, where neighbouring lanes hold whole windows: a quarter of the result
-// is written and nothing read back (us, convolution and pool): 8 x 64 x 224^2 fp32 166 + 18 -> 162, bf16 70 + 18 -> 64;
+// is written and nothing read back (us, convolution and pool): 8 x 64 x 224^2 fp32 166 + 18 -> 162, bf16 70 + 18 -> 53;
 // 8 x 256 x 56^2 fp32 158 + 6 -> 153; the five pools of VGG-16 at batch 8 43 -> 0 altogether.
-// (the tiles of 28^2 and 56^2 images are seven eighths full: 220 TFLOP/s of the 287 the instructions reach alone)
+// (the tiles of 56^2 images are seven eighths full, those of 28^2 and 14^2 ones 77 %: at 56^2 and 28^2 the pipes do 225 and 248 of the 287
+// TFLOP/s that the instructions reach alone)
 #include <algorithm>
 
 #include "fl_common.h"
@@ -77,9 +78,10 @@ struct PartsArgs {
 // POOLS: the launch may be a pooled one; see Launch.
 // DEPTH: chunks of activations in flight; 2 with one part, up to two workgroups per compute unit (see above) and a few chunks each (see Launch).
 // SPLITS: the launch may have its channels split.  With one part and more than two workgroups per compute unit none has, and the
-// exchange's registers would leave two of those a compute unit for three and spill (bf16, us, with the exchange and without it:
-// 8 x 64 x 224^2 -> 64 57 and 55, pooled 52 and 50, 2 x 96 x 150^2 -> 256 34 and 31, 3 x 64 x 112^2 -> 256 27 and 23, 16 x 64 x 112^2 -> 128
-// 57 and 51; 784 workgroups, of which three on each compute unit leave sixteen over, run 1 to 3 % longer, 8 x 128 x 112^2 -> 128 44.6 and 46).
+// exchange's registers would leave two of those a compute unit for three, or spill (bf16, bias and ReLU, us, with the exchange and
+// without it: 8 x 64 x 224^2 -> 64 61 and 59, pooled 56.5 and 53, 8 x 128 x 112^2 -> 128 50.2 and 49.4; without a chain 2 x 96 x 150^2 -> 256 34
+// and 31, 3 x 64 x 112^2 -> 256 27 and 23, but 784 workgroups, of which three on each compute unit leave sixteen over, 1 to 3 % longer,
+// 8 x 128 x 112^2 -> 128 44.6 and 46).
 template <int PARTS, int WF, int TN, bool RAGGED, bool POOLS, int DEPTH, bool SPLITS>
 __global__ __launch_bounds__(kThreads, 2) void ConvPartsKernel(float *out, const float *in, const u32x4 *packed, PartsArgs p) {
   // (no __restrict__: loads of memory known to be constant move freely, and the compiler sinks the ones that are
@@ -448,10 +450,10 @@ Cut ChooseCut(const PartsArgs &p, int64_t images, int parts) {
   return best;
 }
 
-// The pooled epilogue behind a condition costs launches without a pool registers, and bf16 ones of more than two workgroups per
-// compute unit up to a fifth of their time (8 x 256 x 56^2 -> 512: 86 us without the condition, 104 with it, 896 workgroups; 8 x 256 x
-// 56^2 -> 256, 448, 44.6 and 44.9): those have a kernel without it.  The others share one, because a kernel that has not run just
-// before starts with its instructions missing (VGG-16 of one image with two kernels throughout 438 us, with one 436; bf16 401, 398).
+// bf16 launches of more than two workgroups per compute unit have a kernel without the pooled epilogue, whose condition costs those
+// without a pool up to 1 % (8 x 64 x 224^2 -> 64 58.9 us without it, 59.4 with it; 8 x 256 x 56^2 -> 512 84.3, 84.6).  The others share one,
+// because a kernel that has not run just before starts with its instructions missing (VGG-16 of one image with two kernels throughout
+// 438 us, with one 436; bf16 401, 398).
 template <int PARTS, int WF, int TN>
 void Launch(const PartsArgs &p, uint32_t grid, float *out, const float *in, const u32x4 *packed, hipStream_t s) {
 #define FL_PARTS_AS(RAGGED_, POOLS_, DEPTH_, SPLITS_) \

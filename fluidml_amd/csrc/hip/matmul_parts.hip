@@ -617,9 +617,9 @@ int LaunchTile(MatmulArgs q, uint32_t n_batch, float *C, const float *A, hipStre
 }
 
 // 96 rows by 128 columns, the rule's alone: 65 to 96 rows against so many columns that tiles of 96 rows still fill the chip.  Two
-// tiles of 64 rows multiply up to twice as many rows and take the weights in twice (us, 64x128 and this: 77 x 50304 x 512 57,
-// 50; 65 rows 56, 50; 96 rows 58, 51; 80 x 33024 x 256 27.1, 25.6; 90 x 40000 x 1024 77, 76).  With more rows nothing is gained
-// (280 x 33000 x 768 109, 111), with one part neither (90 x 40000 x 1024 32.4, 34.7).
+// tiles of 64 rows multiply up to twice as many rows and take the weights in twice (us, 64x128 and this: 77 x 50304 x 512 58, 46; 65 rows
+// 58, 46; 96 rows 57, 47; 80 x 33024 x 256 28.0, 24.8; 90 x 40000 x 1024 69, 64; 70 x 33000 x 2048 132, 121).  Before the conversions went
+// behind the loads nothing was gained with more rows (280 x 33000 x 768 109, 111) or with one part (90 x 40000 x 1024 32.4, 34.7).
 constexpr int kPacked96x128 = 1 << 8;
 
 template <int PARTS, int EXTRA>
